@@ -1088,6 +1088,7 @@ int cpx_autotune(cpx_ctx *c, const cpx_u128 *xs, size_t n, uint32_t *threads, ui
   };
   double best_ms = 1e300, ms = 0;
   SegShape best = c->shape;
+  c->shape_tuned = true;                 // every trial runs the shape it names
   for (const SegShape &s : cands) {
     if (!seg_shape_supported(s) || seg_blocks_per_cu(s) < 1) continue;
     c->shape = s;

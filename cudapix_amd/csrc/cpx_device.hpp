@@ -145,6 +145,36 @@ __device__ __forceinline__ void st_out(i128 *p, i128 v)
   st_out(q + 1, (uint64_t)((u128)v >> 64));
 }
 
+// The integers of a period of 30030 coprime to it, as pi-table-like entries:
+// odd bits and count below per 64 integers (3.8 KB).
+struct Cop30030 {
+  PiEntry e[470];
+};
+constexpr Cop30030 make_cop30030()
+{
+  Cop30030 t{};
+  uint32_t n = 0;
+  for (uint32_t w = 0; w < 470; w++) {
+    t.e[w].count = n;
+    uint32_t b = 0;
+    for (uint32_t i = 0; i < 32; i++) {
+      const uint32_t m = 64 * w + 2 * i + 1;
+      if (m < 30030 && m % 3 && m % 5 && m % 7 && m % 11 && m % 13) { b |= 1u << i; n++; }
+    }
+    t.e[w].bits = b;
+  }
+  return t;
+}
+static __device__ const Cop30030 cop30030_table = make_cop30030();
+
+// Integers 1 <= m <= M coprime to 30030.
+__device__ __forceinline__ uint32_t cop30030_upto(uint32_t M)
+{
+  const uint32_t b = M / 30030u, k = (M - b * 30030u + 1) >> 1;
+  const PiEntry e = cop30030_table.e[k >> 5];
+  return b * COP30030_TOT + e.count + cpx_popc32(e.bits & cpx_lowmask32(k & 31u));
+}
+
 // Padded-linear LDS layout of a segment bitmap: segment word g lives at
 // lds[g + g / K].  Thread t owns the contiguous words [t*K, (t+1)*K); its
 // j-th word sits at lds[t*(K+1) + j], so lanes walking their own words in
@@ -169,17 +199,6 @@ __device__ __forceinline__ uint64_t first_odd_multiple_bit(uint64_t lo, uint32_t
   uint64_t r = cpx_mod64_32(start, p);
   uint64_t m = start + (r ? p - r : 0);               // first multiple >= start
   if (!(m & 1)) m += p;                               // odd multiple
-  return (m - lo - 1) >> 1;
-}
-
-// first_odd_multiple_bit for max(lo + 1, from) / p < 2^50, with the
-// reciprocal divide in place of the 64-bit remainder.
-__device__ __forceinline__ uint64_t first_odd_multiple_bit_r(uint64_t lo, uint32_t p, uint64_t from)
-{
-  const uint64_t start = lo + 1 > from ? lo + 1 : from;
-  const uint64_t r = start - cpx_div_leaf(start, (double)start, p) * p;
-  uint64_t m = start + (r ? p - r : 0);
-  if (!(m & 1)) m += p;
   return (m - lo - 1) >> 1;
 }
 
@@ -216,24 +235,5 @@ __device__ __forceinline__ void seg_cross_primes(uint32_t *lds, uint32_t K, uint
       uint32_t g = (uint32_t)(j >> 5);
       atomicAnd(&lds[seg_addr(g, K, T)], ~(1u << (j & 31)));
     }
-  }
-}
-
-// Fill an interleaved segment bitmap from a wheel pattern: segment word g is
-// pattern word (w0 + g) mod P, w0 = lo / 64.  Coalesced global reads.
-__device__ __forceinline__ void seg_fill_wheel(uint32_t *lds, uint32_t K, uint32_t T, uint64_t lo,
-                                               const PiEntry *__restrict__ pat, uint32_t P)
-{
-  const uint32_t t = threadIdx.x;
-  const uint32_t W = K * T;
-  // the pattern index steps by T mod P instead of a division per word, so
-  // the loads of the unrolled loop go out together
-  const uint32_t step = T % P;
-  uint32_t idx = (uint32_t)(((lo >> 6) + t) % P);
-#pragma unroll 8
-  for (uint32_t g = t; g < W; g += T) {
-    lds[seg_addr(g, K, T)] = pat[idx].bits;
-    idx += step;
-    if (idx >= P) idx -= P;
   }
 }

@@ -37,7 +37,21 @@ struct WheelInfo {
   uint32_t W;          // primorial W_c = 2 * 3 * ... * p_c
   uint32_t totient;    // Euler totient of W_c
   uint32_t pc;         // p_c
+  uint64_t pat_off;    // the segment pattern (entries; u32 words): word w holds the integers of
+  uint32_t pat_period; // [120 w, 120 w + 120) coprime to 30, multiples of 7 .. p_c cleared
+  uint32_t pad;
 };
+
+// The hard leaves' dense candidates: every sieved stage has p >= 13, so a leaf's
+// m (lpf(m) > p) is coprime to 30030.  The leaf table lists those m in order
+// (5760 per 30030 integers, 0.38 of the odd ones) as {m, mu(m) lpf(m)}; it
+// follows the mu*lpf table in one allocation.
+#define COP30030_TOT 5760u
+__host__ __device__ constexpr uint64_t cpx_leaf_entries(uint64_t nodd)
+{
+  return (2 * nodd / 30030 + 1) * COP30030_TOT;
+}
+__host__ __device__ constexpr uint64_t cpx_mlpf_words(uint64_t nodd) { return nodd + 2 * cpx_leaf_entries(nodd); }
 
 // Per-query record (device resident; host fills the static part).
 struct QueryDev {
@@ -48,7 +62,7 @@ struct QueryDev {
   uint64_t p2_e;          // even start of the P2 count range (sqrtx & ~1)
   uint64_t tm_off;        // first element of this query in hard_T
   uint32_t c, B;          // hard stages b = c+1 .. B (1-based prime indices)
-  uint32_t nstage;        // B - c
+  uint32_t nstage;        // B - cs: the sieved ones
   uint32_t a;             // pi(y)
   uint32_t pi_cbrt, pi_qrt, pi_sqrtz, small;   // small: answered by one pi-table lookup
   uint64_t hard_nseg, hard_row0;      // hard segments and first output row (T, bact, rowinfo)
@@ -62,7 +76,7 @@ struct QueryDev {
   uint32_t n_p2_parts;                // P2 by table lookups: partial sums of pi(x/p) (after the hard ones)
   uint32_t p2tab;                     // P2 from table lookups instead of P2 segment rows
   uint32_t omega;                     // the hard leaves with x/(pq) < p^2 go to lookups (below)
-  uint32_t pad_o;
+  uint32_t cs;                        // wheel of the segment sieve; stages c < b <= cs: dir_desc
   uint64_t pi_e;                      // written by setup: pi(p2_e)
   uint64_t pi_sqrtx;                  // written by setup: pi(sqrt x)
 };
@@ -125,7 +139,7 @@ __host__ __device__ __forceinline__ uint32_t cpx_fastmod32(uint32_t a, uint32_t 
 // segment once for up to CPX_GROUP queries of similar x (same wheel), and
 // evaluates every member's leaves, counters and P2 counts against it.
 #ifndef CPX_GROUP
-#define CPX_GROUP 8
+#define CPX_GROUP 32
 #endif
 struct GroupDev {
   uint32_t n;                   // members, sorted by x
@@ -190,6 +204,7 @@ struct BatchDev {
   const uint32_t *primes; uint64_t nprimes;
   const double *prinv;                        // 1/p (nearest) of primes[i]
   const int32_t *mlpf;   uint64_t mlpf_n;     // mu(m)*lpf(m) for odd m, index m>>1
+  const int2 *mleaf;                          // the leaf table
   const PiEntry *wheel;  const WheelInfo *winfo;
   // plan
   QueryDev *queries;     uint32_t *nqueries;
@@ -201,6 +216,7 @@ struct BatchDev {
   BlockDesc *easy_desc;  uint32_t *n_easy;
   BlockDesc *fin_desc;   uint32_t *n_fin;     // hard carry blocks (begin = the stage)
   BlockDesc *p2_desc;    uint32_t *n_p2;      // P2 lookups (prime index ranges)
+  BlockDesc *dir_desc;   uint32_t *n_dir;     // hard leaves of the wheel stages (odd m)
   HardRowInfo *rowinfo;                       // [row]
   // outputs
   uint32_t *hard_T;                           // per row, active stages: survivors before stage
@@ -223,11 +239,12 @@ struct BatchDev {
 };
 
 // Segment-kernel shape: T threads, K words (32 bits) per thread, so a segment
-// holds 32*K*T odd numbers.
+// holds 32*K*T numbers coprime to 30.
 struct SegShape {
   int threads;
   int kwords;
   uint64_t seg_bits() const { return 32ull * kwords * threads; }
+  uint64_t seg_ints() const { return seg_bits() / 8 * 30; }
 };
 
 // ------------------------------------------------------------- launchers

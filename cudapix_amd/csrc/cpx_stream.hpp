@@ -116,6 +116,7 @@ struct StreamArgs {
 #define CPX_TILE_ORD 0xfffffffdu
 #define CPX_TILE_TRIV 0xfffffffcu
 #define CPX_TILE_NOP 0xfffffffbu     // no work (a cohort whose queries are all table lookups)
+#define CPX_TILE_DIR 0xfffffffau     // hard leaves of the wheel stages
 
 // A block that finds no work for this long leaves even if the host never
 // closes; a main tile waits at most this long for its cohort's copy units

@@ -37,6 +37,43 @@ __device__ __forceinline__ i128 ordinary_part(const BatchDev &bd, const BlockDes
   return sum;
 }
 
+// ------------------------------------------- hard leaves of wheel stages
+// The segment sieve starts from the wheel of the first q.cs primes; the hard
+// leaves of the stages c < b <= cs, p = p_b, need no sieve: with b - 1 <= 7
+// primes below p, phi(x/(p m), b - 1) is the wheel's closed form, as in the
+// ordinary leaves.  This thread's share of
+//   sum over odd m of d, m > y/p, lpf(m) > p of mu(m) phi(x/(p m), b - 1).
+// Bound by the integer divides (a 128/64 one per m, two per leaf).
+template <uint32_t NT>
+__device__ __forceinline__ i128 direct_part(const BatchDev &bd, const BlockDesc &d, uint32_t t)
+{
+  const QueryDev &q = bd.queries[d.query];
+  const u128 x = ((u128)q.x_hi << 64) | q.x_lo;
+  const uint32_t p0 = bd.primes[q.c];
+  i128 sum = 0;
+  for (uint64_t i = d.begin + t; i < d.end; i += NT) {
+    const int32_t v = bd.mlpf[i];
+    const uint32_t av = (uint32_t)(v < 0 ? -v : v);
+    if (av <= p0) continue;
+    const uint64_t m = 2 * i + 1;
+    uint64_t r;
+    const u128 u = cpx_div128_64(x, m, &r);
+    i128 s = 0;
+    for (uint32_t b = q.c; b < q.cs; b++) {
+      const uint32_t p = bd.primes[b];
+      if (av <= p) break;
+      if (m * p <= q.y) continue;
+      const WheelInfo wi = bd.winfo[b];
+      const u128 k = cpx_div128_64(cpx_div128_64(u, p, &r), wi.W, &r);
+      const uint32_t kk = (uint32_t)((r + 1) >> 1);
+      const PiEntry e = bd.wheel[wi.off + (kk >> 5)];
+      s += (i128)(k * wi.totient) + (i128)(e.count + cpx_popc32(e.bits & cpx_lowmask32(kk & 31u)));
+    }
+    sum += v > 0 ? s : -s;
+  }
+  return sum;
+}
+
 // ------------------------------------------------------------ trivial U
 // U = sum over primes sqrt(z) < p <= cbrt(x) of [pi(y) - pi(x / p^2)]
 // (src/trivial.cu:31-62).  Items: prime index i (p = primes[i]).

@@ -189,7 +189,7 @@ int make_host_query(cpx_ctx *c, u128 x, uint64_t y, uint32_t cc, HostQuery *hq)
   if (cc < 1 || cc > 8) return ctx_fail(c, CPX_EINVAL, "c must be in 1..8");
   if (x < CPX_SMALL_X) {
     h.small = true;
-    h.y = 1; h.c = 1;
+    h.y = 1; h.c = h.cs = 1;
     *hq = h;
     return CPX_OK;
   }
@@ -212,6 +212,7 @@ int make_host_query(cpx_ctx *c, u128 x, uint64_t y, uint32_t cc, HostQuery *hq)
   uint32_t k = 0;
   while (k < 8 && sp[k] <= h.qrtx) k++;
   h.c = cc < k ? cc : k;
+  h.cs = k;                                       // (k >= 5 for x >= 2^14)
   // the easy leaves divide x / p for p > x^(1/4) as 64-bit values (x < ~2^85);
   // the hard segment tiles hold x / p in 80 bits
   if ((x / h.qrtx) >> 64) return ctx_fail(c, CPX_ERANGE, "x / x^(1/4) must fit 64 bits");
@@ -240,35 +241,42 @@ static int build_bootstrap(cpx_ctx *c)
 
 int build_wheels(cpx_ctx *c, uint32_t want)
 {
-  uint32_t cmax = std::max(c->opts.c, want);
+  // phi tables of the wheels to c, and to 7 for the hard leaves of the wheel
+  // stages; the segment sieve takes the pattern of up to 8 primes whatever c is
+  uint32_t cmax = std::max({c->opts.c, want, 7u});
   if (cmax > 8) cmax = 8;
   if (c->wheel_c >= cmax && c->wheel.p) return CPX_OK;
   static const uint32_t sp[8] = {2, 3, 5, 7, 11, 13, 17, 19};
   std::vector<WheelInfo> wi(9);
-  uint64_t off = 0, W = 1, tot = 1, period = 1;
-  for (uint32_t k = 1; k <= cmax; k++) {
+  uint64_t off = 0, W = 1, tot = 1, period = 1, pat = 1, period_max = 1;
+  for (uint32_t k = 1; k <= 8; k++) {
     W *= sp[k - 1];
     tot *= sp[k - 1] - 1;
     if (k >= 2) period *= sp[k - 1];
+    if (k >= 4) pat *= sp[k - 1];
     wi[k].off = off;
-    wi[k].period = (uint32_t)period;
+    wi[k].period = k <= cmax ? (uint32_t)period : 0u;
     wi[k].W = (uint32_t)W;
     wi[k].totient = (uint32_t)tot;
     wi[k].pc = sp[k - 1];
-    off += period + 1;
+    wi[k].pat_off = off + wi[k].period + 1;
+    wi[k].pat_period = (uint32_t)pat;
+    off = wi[k].pat_off + (pat + 1) / 2;
+    period_max = std::max<uint64_t>(period_max, wi[k].period);
   }
   int rc;
   if ((rc = dbuf_reserve(c, c->wheel, off, &c->table_bytes))) return rc;
   if ((rc = dbuf_reserve(c, c->winfo, 9, &c->table_bytes))) return rc;
-  size_t maxchunks = (period + 4095) / 4096 + 2;
+  size_t maxchunks = (period_max + 4095) / 4096 + 2;
   if ((rc = dbuf_reserve(c, c->scan_tot, std::max<size_t>(maxchunks, c->scan_tot.cap), &c->table_bytes)))
     return rc;
   if ((rc = dbuf_reserve(c, c->scan_base, std::max<size_t>(maxchunks, c->scan_base.cap), &c->table_bytes)))
     return rc;
-  for (uint32_t k = 1; k <= cmax; k++) {
+  for (uint32_t k = 1; k <= 8; k++) {
     HIPCHK(launch_wheel(c->wheel.p + wi[k].off, wi[k].period, k, c->stream));
-    HIPCHK(launch_scan_entries(c->wheel.p + wi[k].off, wi[k].period, c->scan_tot.p,
-                               c->scan_base.p, c->stream));
+    if (wi[k].period)
+      HIPCHK(launch_scan_entries(c->wheel.p + wi[k].off, wi[k].period, c->scan_tot.p,
+                                 c->scan_base.p, c->stream));
   }
   HIPCHK(hipMemcpyAsync(c->winfo.p, wi.data(), 9 * sizeof(WheelInfo), hipMemcpyHostToDevice,
                         c->stream));
@@ -353,7 +361,7 @@ int ensure_tables(cpx_ctx *c, uint64_t R, uint64_t P, uint64_t Y)
   // mu * lpf for odd m <= Y
   uint64_t nodd = (Y + 1) / 2;
   uint64_t nodd_alloc = (nodd + 4095) / 4096 * 4096;
-  if ((rc = dbuf_reserve(c, c->mlpf, nodd_alloc, &c->table_bytes))) return rc;
+  if ((rc = dbuf_reserve(c, c->mlpf, cpx_mlpf_words(nodd_alloc), &c->table_bytes))) return rc;
   HIPCHK(launch_mlpf(c->mlpf.p, nodd_alloc, c->primes.p, (uint32_t)np, c->stream));
   c->mlpf_limit = 2 * nodd_alloc - 1;
   HIPCHK(hipStreamSynchronize(c->stream));
@@ -365,11 +373,12 @@ int ensure_tables(cpx_ctx *c, uint64_t R, uint64_t P, uint64_t Y)
 
 static uint64_t ceil_div(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
 
-static const uint64_t ORD_CH = 8192, TRIV_CH = 4096, EASY_WORK = 131072, P2_CH = 65536;
+static const uint64_t ORD_CH = 2048, TRIV_CH = 4096, EASY_WORK = 131072, P2_CH = 65536;
 
-static void plan_needs(const cpx_ctx *c, const HostQuery &h, uint32_t mask, uint64_t SB,
+static void plan_needs(const cpx_ctx *c, const HostQuery &h, uint32_t mask, uint64_t seg_bits,
                        uint64_t *R, uint64_t *P, uint64_t *Y)
 {
+  const uint64_t SI = seg_bits / 8 * 30;               // integers of a segment
   if (h.small) { *R = std::max<uint64_t>(*R, (uint64_t)h.x); return; }
   *R = std::max(*R, std::max(h.sqrtx, h.y));
   *Y = std::max(*Y, h.y);
@@ -380,8 +389,8 @@ static void plan_needs(const cpx_ctx *c, const HostQuery &h, uint32_t mask, uint
       p = std::max(p, h.sqrtx);
     } else {                        // sieving primes of the last P2 segment
       uint64_t e = h.sqrtx & ~63ull;
-      uint64_t nseg = ceil_div(h.zt + 1 - e, 2 * SB);
-      p = std::max<uint64_t>(p, cpx_isqrt128((u128)e + nseg * 2 * SB) + 1);
+      uint64_t nseg = ceil_div(h.zt + 1 - e, SI) + 1;
+      p = std::max<uint64_t>(p, cpx_isqrt128((u128)e + nseg * SI) + 1);
     }
   }
   *P = std::max(*P, p);
@@ -392,7 +401,7 @@ static void plan_needs(const cpx_ctx *c, const HostQuery &h, uint32_t mask, uint
 // counters); build_plan places the shares.
 struct QPlan {
   QueryDev d{};
-  std::vector<BlockDesc> ord, triv, easy, fin, p2d;
+  std::vector<BlockDesc> ord, triv, easy, fin, p2d, dir;
   std::vector<uint32_t> fin_rows;    // rows each carry block scans (its first stage's active rows)
   std::vector<HardRowInfo> rowinfo;  // replicas and M rows are set per group
   std::vector<float> rleaves;        // estimated leaves of each hard row
@@ -407,7 +416,7 @@ struct GPlan {
 };
 
 // Where one query's descriptors and rows go in the batch arrays.
-struct PlanOff { size_t ord, triv, easy, fin, p2d, rows; };
+struct PlanOff { size_t ord, triv, easy, fin, p2d, dir, rows; };
 
 // A batch plan: queries, groups and sorted tiles; the per-query descriptors
 // and rows stay in the query shares and are written straight into the
@@ -423,7 +432,7 @@ struct Plan {
                                      // stage table from the host
   Caps base{};                       // where its entries start in each arena array (a
                                      // streaming cohort's slot; zero for a batch)
-  size_t nord = 0, ntriv = 0, neasy = 0, nfin = 0, np2d = 0, nrows = 0;
+  size_t nord = 0, ntriv = 0, neasy = 0, nfin = 0, np2d = 0, ndir = 0, nrows = 0;
   uint64_t stage_total = 0, hard_rows = 0, hard_tm = 0, p2_rows = 0, parts = 0;
   uint64_t hard_mrows = 0, hard_mm = 0;
   uint64_t hard_segments = 0, p2_segments = 0;
@@ -450,38 +459,37 @@ static inline uint16_t cost_bucket(double cost)
 static void plan_query(const cpx_ctx *c, const HostQuery &h, uint32_t i, uint32_t mask, QPlan &qp)
 // (i: the query's index in the arena's query array, which its descriptors name)
 {
-  const uint64_t SB = c->shape.seg_bits();
+  const uint64_t SI = c->shape.seg_ints();
   const uint32_t T = (uint32_t)c->shape.threads;
   QueryDev &d = qp.d;
   d.x_lo = (uint64_t)h.x;
   d.x_hi = (uint64_t)(h.x >> 64);
   d.omega = 0;
-  d.pad_o = 0;
+  d.cs = h.cs;
   if (h.small) {
     d.small = 1;
     return;
   }
   d.y = h.y; d.z = h.z; d.sqrtx = h.sqrtx; d.cbrtx = h.cbrtx; d.qrtx = h.qrtx; d.sqrtz = h.sqrtz;
   d.p2_zt = h.zt;
-  // the wheel pattern is word-aligned: segments start on a multiple of 64
   d.p2_e = h.sqrtx & ~63ull;
   d.c = h.c;
   uint64_t B = host_pi(c, h.qrtx);
   d.B = (uint32_t)B;
-  d.nstage = ((mask & TERM_HARD) && B > h.c) ? (uint32_t)(B - h.c) : 0;
+  d.nstage = ((mask & TERM_HARD) && B > h.cs) ? (uint32_t)(B - h.cs) : 0;
   d.a = (uint32_t)host_pi(c, h.y);
   d.pi_cbrt = (uint32_t)host_pi(c, std::min(h.cbrtx, h.y));
   d.pi_qrt = (uint32_t)B;
   d.pi_sqrtz = (uint32_t)host_pi(c, h.sqrtz);
-  // segments of 2*SB integers from 0: the hard leaves use [0, z]; P2 counts
+  // segments of SI integers from 0: the hard leaves use [0, z]; P2 counts
   // primes in (p2_e, zt] in the segments that hold them (a P2 epilogue of
   // the same tile), so the tiles reach z, or zt when only P2 is asked for --
   // unless P2 comes from pi-table lookups
   const bool p2 = (mask & TERM_P2) && h.y < h.sqrtx;
   d.p2tab = p2 && h.p2tab;
-  d.p2_seg0 = d.p2_e / (2 * SB);
-  d.p2_nseg = p2 && !h.p2tab ? h.zt / (2 * SB) + 1 - d.p2_seg0 : 0;
-  d.hard_nseg = d.nstage ? ceil_div(h.z + 1, 2 * SB) : (d.p2_nseg ? d.p2_seg0 + d.p2_nseg : 0);
+  d.p2_seg0 = d.p2_e / SI;
+  d.p2_nseg = p2 && !h.p2tab ? h.zt / SI + 1 - d.p2_seg0 : 0;
+  d.hard_nseg = d.nstage ? ceil_div(h.z + 1, SI) : (d.p2_nseg ? d.p2_seg0 + d.p2_nseg : 0);
   uint32_t part = 0;
   // ordinary: odd n <= y
   if (mask & TERM_ORD) {
@@ -532,7 +540,7 @@ static void plan_query(const cpx_ctx *c, const HostQuery &h, uint32_t i, uint32_
   // at the first such p.  About half of all hard leaves at 1e13..1e16.
   if (d.nstage) {
     const uint64_t sy = cpx_isqrt128((u128)h.y);                         // p > sy <=> p^2 > y
-    const uint64_t js = std::max<uint64_t>(h.c, host_pi(c, sy));         // first such stage prime
+    const uint64_t js = std::max<uint64_t>(h.cs, host_pi(c, sy));         // first such stage prime
     if (js < d.B && ((h.x / c->h_primes[js]) >> 64) == 0) {
       d.omega = 1;
       const uint64_t ky = d.a;                                          // pi(y)
@@ -550,6 +558,12 @@ static void plan_query(const cpx_ctx *c, const HostQuery &h, uint32_t i, uint32_
       }
     }
   }
+  // hard leaves of the wheel stages c < b <= cs: odd m in (y / p_cs, y]
+  if ((mask & TERM_HARD) && h.cs > h.c) {
+    const uint64_t nodd = (h.y + 1) / 2;
+    for (uint64_t b = h.y / c->h_primes[h.cs - 1] / 2; b < nodd; b += ORD_CH)
+      qp.dir.push_back({i, part++, b, std::min(nodd, b + ORD_CH)});
+  }
   d.n_hard_parts = part - d.n_ord_parts - d.n_triv_parts - d.n_easy_parts;
   // P2 by lookups: prime indices (pi(y), pi(sqrt x)] (primes[k] is the (k+1)-th prime)
   if (d.p2tab) {
@@ -564,7 +578,7 @@ static void plan_query(const cpx_ctx *c, const HostQuery &h, uint32_t i, uint32_
   std::vector<double> xps;
   if (d.hard_nseg) {
     xps.resize(d.nstage);
-    for (uint32_t k = 0; k < d.nstage; k++) xps[k] = (double)(h.x / c->h_primes[h.c + k]);
+    for (uint32_t k = 0; k < d.nstage; k++) xps[k] = (double)(h.x / c->h_primes[h.cs + k]);
   }
   const double leaf_target = 256.0 * T;
   uint32_t sparse_run = 0;
@@ -574,10 +588,10 @@ static void plan_query(const cpx_ctx *c, const HostQuery &h, uint32_t i, uint32_
   qp.rleaves.reserve(d.hard_nseg);
   qp.rleafy.reserve(d.hard_nseg);
   for (uint64_t s = 0; s < d.hard_nseg; s++) {
-    const uint64_t lo = s * 2 * SB, hi = lo + 2 * SB;
+    const uint64_t lo = s * SI, hi = lo + SI;
     // active stages: p_b^2 <= x / lo, i.e. p_b^2 * lo <= x (the kernel's test)
     while (act > 0) {
-      const u128 p = c->h_primes[h.c + act - 1];
+      const u128 p = c->h_primes[h.cs + act - 1];
       if (p * p * (u128)lo <= h.x) break;
       act--;
     }
@@ -588,7 +602,7 @@ static void plan_query(const cpx_ctx *c, const HostQuery &h, uint32_t i, uint32_
     // (a sample of at most 32 stages, scaled: the estimate only sizes replicas)
     const uint32_t kstep = act > 32 ? (uint32_t)((act + 31) / 32) : 1u;
     for (uint32_t k = 0; est && k < act; k += kstep) {
-      const double p = (double)c->h_primes[h.c + k];
+      const double p = (double)c->h_primes[h.cs + k];
       const double xp = (double)xps[k];
       double mhi = lo ? std::min(fy, std::floor(xp * inv_lo)) : fy;
       double mlo = std::max(std::floor(xp * inv_hi), std::floor(fy / p));
@@ -597,7 +611,7 @@ static void plan_query(const cpx_ctx *c, const HostQuery &h, uint32_t i, uint32_
       if (sparse && d.omega) mhi = std::min(mhi, std::floor(xp / (p * p)));
       if (mhi > mlo) {
         leafy += kstep;
-        leaves += kstep * (sparse ? (mhi - mlo) / std::log(mhi) : 0.5 * (mhi - mlo));
+        leaves += kstep * (sparse ? (mhi - mlo) / std::log(mhi) : 0.192 * (mhi - mlo));
       }
     }
     if (est) sparse_run = leaves < leaf_target / 4 ? sparse_run + 1 : 0;
@@ -635,10 +649,10 @@ static void make_groups(const cpx_ctx *c, const std::vector<HostQuery> &hq,
   uint64_t smax = 0, p2min = ~0ull;
   for (uint32_t i : hs) {
     const QueryDev &d = qps[i].d;
-    const uint64_t si = d.nstage ? c->h_primes[d.c + d.nstage - 1] : 0;
+    const uint64_t si = d.nstage ? c->h_primes[d.cs + d.nstage - 1] : 0;
     const uint64_t pi = d.p2_nseg ? d.p2_e : ~0ull;
     const bool alone = d.y >= (1ull << 28);
-    if (cur.n && (cur.n == CPX_GROUP || qps[cur.q[0]].d.c != d.c || alone || cur_alone ||
+    if (cur.n && (cur.n == CPX_GROUP || qps[cur.q[0]].d.cs != d.cs || alone || cur_alone ||
                   std::max(smax, si) > std::min(p2min, pi))) {
       groups.push_back(cur);
       cur = GroupDev{};
@@ -665,13 +679,13 @@ static void plan_group(const cpx_ctx *c, const GroupDev &g, uint32_t gi, std::ve
   const double leaf_target = 256.0 * T;
   uint64_t nseg = 0;
   for (uint32_t m = 0; m < g.n; m++) nseg = std::max(nseg, qps[g.q[m]].d.hard_nseg);
-  const uint32_t cw = qps[g.q[0]].d.c;
+  const uint32_t cw = qps[g.q[0]].d.cs;
   uint64_t mrows[CPX_GROUP] = {0}, moff[CPX_GROUP] = {0};
   uint64_t nsp_i = 0;                                  // pi(sqrt(hi)), grows with s
   gp.tiles.reserve(nseg);
   gp.tbucket.reserve(nseg);
   for (uint64_t s = 0; s < nseg; s++) {
-    const uint64_t hi = (s + 1) * 2 * SB;
+    const uint64_t hi = (s + 1) * c->shape.seg_ints();
     double leaves = 0, lcost = 0;
     uint32_t act = 0, np2 = 0;
     for (uint32_t m = 0; m < g.n; m++) {
@@ -853,9 +867,9 @@ static int build_plan(cpx_ctx *c, const std::vector<HostQuery> &hq, uint32_t mas
     pl.hard_segments += d.hard_nseg;
     pl.p2_segments += d.p2_nseg;
     pl.q[i] = d;
-    off[i] = {pl.nord, pl.ntriv, pl.neasy, pl.nfin, pl.np2d, pl.nrows};
+    off[i] = {pl.nord, pl.ntriv, pl.neasy, pl.nfin, pl.np2d, pl.ndir, pl.nrows};
     pl.nord += qp.ord.size(); pl.ntriv += qp.triv.size(); pl.neasy += qp.easy.size();
-    pl.np2d += qp.p2d.size(); pl.nfin += qp.fin.size(); pl.nrows += qp.rowinfo.size();
+    pl.np2d += qp.p2d.size(); pl.ndir += qp.dir.size(); pl.nfin += qp.fin.size(); pl.nrows += qp.rowinfo.size();
   }
   for (const GPlan &gp : gps) ntiles += gp.tiles.size();
   // longest first: counting sort on the cost buckets (descending, stable in
@@ -887,6 +901,7 @@ static int build_plan(cpx_ctx *c, const std::vector<HostQuery> &hq, uint32_t mas
   if (stream) {
     spread(CPX_TILE_ORD, pl.nord);
     spread(CPX_TILE_TRIV, pl.ntriv);
+    spread(CPX_TILE_DIR, pl.ndir);
     // a cohort of table lookups only still needs one main tile: its end
     // opens the combine phase
     if (pl.tiles.empty()) pl.tiles.push_back({CPX_TILE_NOP, 1, 0, 0});
@@ -921,6 +936,7 @@ static Layout make_layout(const Caps &k)
   L.easy = o;     o = al(o + k.easy * sizeof(BlockDesc));
   L.fin = o;      o = al(o + k.fin * sizeof(BlockDesc));
   L.p2d = o;      o = al(o + k.p2d * sizeof(BlockDesc));
+  L.dir = o;      o = al(o + k.dir * sizeof(BlockDesc));
   L.rowinfo = o;  o = al(o + k.rows * sizeof(HardRowInfo));
   L.plan_bytes = o;
   o = 0;
@@ -944,7 +960,7 @@ static Caps needed_caps(const Plan &pl)
   Caps k{};
   k.q = pl.q.size(); k.stages = pl.stage_total; k.tiles = pl.tiles.size(); k.groups = pl.groups.size();
   k.ord = pl.nord; k.triv = pl.ntriv; k.easy = pl.neasy; k.fin = pl.nfin;
-  k.p2d = pl.np2d;
+  k.p2d = pl.np2d; k.dir = pl.ndir;
   k.tm = pl.hard_tm; k.rows = pl.hard_rows; k.p2rows = pl.p2_rows; k.parts = pl.parts;
   k.mm = pl.hard_mm; k.mrows = pl.hard_mrows;
   return k;
@@ -1050,11 +1066,12 @@ static BatchDev batchdev_at(const cpx_ctx *c, const Layout &L, char *P, char *O)
   BatchDev b{};
   b.pitab = c->pitab.p; b.pitab_n = c->pitab_nent;
   b.primes = c->primes.p; b.nprimes = c->nprimes; b.prinv = c->prinv.p;
-  b.mlpf = c->mlpf.p; b.mlpf_n = c->mlpf.cap;
+  b.mlpf = c->mlpf.p; b.mlpf_n = (c->mlpf_limit + 1) / 2;
+  b.mleaf = reinterpret_cast<const int2 *>(c->mlpf.p + b.mlpf_n);
   b.wheel = c->wheel.p; b.winfo = c->winfo.p;
   uint32_t *cnt = (uint32_t *)(P + L.counters);
   b.nqueries = cnt + 0; b.ntiles = cnt + 1; b.tile_head = cnt + 2;
-  b.n_ord = cnt + 3; b.n_triv = cnt + 4; b.n_easy = cnt + 5; b.n_fin = cnt + 6; b.n_p2 = cnt + 7;
+  b.n_ord = cnt + 3; b.n_triv = cnt + 4; b.n_easy = cnt + 5; b.n_fin = cnt + 6; b.n_p2 = cnt + 7; b.n_dir = cnt + 8;
   b.queries = (QueryDev *)(P + L.queries);
   b.stages = (StageDev *)(P + L.stages);
   b.tiles = (TileDev *)(P + L.tiles);
@@ -1063,6 +1080,7 @@ static BatchDev batchdev_at(const cpx_ctx *c, const Layout &L, char *P, char *O)
   b.triv_desc = (BlockDesc *)(P + L.triv);
   b.easy_desc = (BlockDesc *)(P + L.easy);
   b.p2_desc = (BlockDesc *)(P + L.p2d);
+  b.dir_desc = (BlockDesc *)(P + L.dir);
   b.fin_desc = (BlockDesc *)(P + L.fin);
   b.rowinfo = (HardRowInfo *)(P + L.rowinfo);
   b.hard_T = (uint32_t *)(O + L.hard_T);
@@ -1092,7 +1110,7 @@ static void pack_plan(const Layout &L, const Plan &pl, char *H)
   cnt[0] = (uint32_t)pl.q.size(); cnt[1] = (uint32_t)pl.tiles.size(); cnt[2] = 0;
   cnt[3] = (uint32_t)pl.nord; cnt[4] = (uint32_t)pl.ntriv;
   cnt[5] = (uint32_t)pl.neasy; cnt[6] = (uint32_t)pl.nfin;
-  cnt[7] = (uint32_t)pl.np2d;
+  cnt[7] = (uint32_t)pl.np2d; cnt[8] = (uint32_t)pl.ndir;
   auto put = [&](size_t off, const void *src, size_t bytes) {
     if (bytes) memcpy(H + off, src, bytes);
   };
@@ -1109,6 +1127,7 @@ static void pack_plan(const Layout &L, const Plan &pl, char *H)
       case CPX_TILE_P2: t.seg += B.p2d; break;
       case CPX_TILE_ORD: t.seg += B.ord; break;
       case CPX_TILE_TRIV: t.seg += B.triv; break;
+      case CPX_TILE_DIR: t.seg += B.dir; break;
       case CPX_TILE_NOP: break;
       default: t.group += (uint32_t)B.groups; break;
     }
@@ -1128,6 +1147,7 @@ static void pack_plan(const Layout &L, const Plan &pl, char *H)
     put(L.triv + (B.triv + o.triv) * sizeof(BlockDesc), qp.triv.data(), qp.triv.size() * sizeof(BlockDesc));
     put(L.easy + (B.easy + o.easy) * sizeof(BlockDesc), qp.easy.data(), qp.easy.size() * sizeof(BlockDesc));
     put(L.p2d + (B.p2d + o.p2d) * sizeof(BlockDesc), qp.p2d.data(), qp.p2d.size() * sizeof(BlockDesc));
+    put(L.dir + (B.dir + o.dir) * sizeof(BlockDesc), qp.dir.data(), qp.dir.size() * sizeof(BlockDesc));
     put(L.rowinfo + (B.rows + o.rows) * sizeof(HardRowInfo), qp.rowinfo.data(),
         qp.rowinfo.size() * sizeof(HardRowInfo));
   });
@@ -1142,7 +1162,7 @@ static void pack_stages(const cpx_ctx *c, const Layout &L, const Plan &pl, char 
     const QueryDev &q = pl.q[i];
     const u128 x = ((u128)q.x_hi << 64) | q.x_lo;
     for (uint32_t k = 0; k < q.nstage; k++) {
-      const uint32_t p = c->h_primes[q.c + k];
+      const uint32_t p = c->h_primes[q.cs + k];
       StageDev d;
       d.p = p;
       d.ylo = (uint32_t)(q.y / p);
@@ -1183,6 +1203,7 @@ static int upload_plan(cpx_ctx *c, BatchSlot &S, const Plan &pl)
   HIPCHK(up(L.triv, pl.ntriv * sizeof(BlockDesc)));
   HIPCHK(up(L.easy, pl.neasy * sizeof(BlockDesc)));
   HIPCHK(up(L.p2d, pl.np2d * sizeof(BlockDesc)));
+  HIPCHK(up(L.dir, pl.ndir * sizeof(BlockDesc)));
   HIPCHK(up(L.fin, pl.nfin * sizeof(BlockDesc)));
   HIPCHK(up(L.rowinfo, pl.nrows * sizeof(HardRowInfo)));
   HIPCHK(hipEventRecord(S.ev[4], c->up_stream));
@@ -1194,14 +1215,15 @@ static int upload_plan(cpx_ctx *c, BatchSlot &S, const Plan &pl)
 // graph capture; the grid is cached per shape.
 static int seg_grid(cpx_ctx *c)
 {
-  static thread_local SegShape last{0, 0};
-  static thread_local int last_nb = 0;
-  if (last.threads != c->shape.threads || last.kwords != c->shape.kwords) {
-    last_nb = seg_blocks_per_cu(c->shape);
-    last = c->shape;
+  static thread_local struct { SegShape shape; int nb; } seen[2];
+  int k = 0;
+  while (k < 2 && (seen[k].shape.threads != c->shape.threads || seen[k].shape.kwords != c->shape.kwords)) k++;
+  if (k == 2) {
+    seen[1] = seen[0];
+    seen[0] = {c->shape, std::max(1, seg_blocks_per_cu(c->shape))};
+    k = 0;
   }
-  int nb = last_nb < 1 ? 1 : last_nb;
-  return nb * c->cu_count;
+  return seen[k].nb * c->cu_count;
 }
 
 static const uint32_t GRID_Q = 256, GRID_T = 2048;
@@ -1263,19 +1285,19 @@ static int ensure_graph(cpx_ctx *c, BatchSlot &S, const BatchDev &b, uint32_t nr
 uint64_t plan_bytes_estimate(const cpx_ctx *c, const HostQuery &h)
 {
   if (h.small) return 1024;
-  const uint64_t SB = c->shape.seg_bits();
+  const double SI = (double)c->shape.seg_ints();
   // stages ~ pi(x^(1/4)) <= 1.26 n / ln n
   double q = (double)h.qrtx;
   double B = q < 3 ? 1 : 1.26 * q / std::log(q);
-  double hseg = std::ceil((double)(h.z + 1) / (2.0 * SB));
-  double p2seg = std::ceil((double)(h.zt + 1) / (2.0 * SB));
-  // active (segment, stage) pairs: segment r >= 1 (lo = 2 SB r) has about
+  double hseg = std::ceil((double)(h.z + 1) / SI);
+  double p2seg = std::ceil((double)(h.zt + 1) / SI);
+  // active (segment, stage) pairs: segment r >= 1 (lo = SI r) has about
   // min(B, pi(sqrt(x / lo))) active stages; summed over log-spaced buckets
   const double X = (double)h.x;
   double pairs = B;
   for (double r = 1; r < hseg;) {
     const double r1 = std::min(hseg, std::max(r + 1, std::floor(r * 1.25)));
-    const double v = std::sqrt(X / (2.0 * SB * std::sqrt(r * r1)));
+    const double v = std::sqrt(X / (SI * std::sqrt(r * r1)));
     const double pv = v < 3 ? 0 : 1.26 * v / std::log(v);
     pairs += (r1 - r) * std::min(B, pv);
     r = r1;
@@ -1283,7 +1305,7 @@ uint64_t plan_bytes_estimate(const cpx_ctx *c, const HostQuery &h)
   // T and M per pair (M rows of replicated segments add some: a group's
   // leaf-dense segments give every member the group's replicas), rowinfo,
   // bact and the P2 rows, stage and carry descriptors, easy descriptors
-  double bytes = pairs * 8 * 1.5 + hseg * 48 + p2seg * 16 + 4096 + B * 80 + (h.y / 8192.0 + 16) * 48;
+  double bytes = pairs * 8 * 1.5 + hseg * 48 + p2seg * 16 + 4096 + B * 80 + (h.y / 2048.0 + 32) * 48;
   return (uint64_t)bytes;
 }
 
@@ -1420,6 +1442,22 @@ static int launch_passes(cpx_ctx *c, BatchSlot &S, const Plan &pl, const PassPla
   return CPX_OK;
 }
 
+// The segment shape of a solve, for the length of a scope.  One small query on
+// its own does not fill the chip with 512-thread segments: half-size blocks
+// (256 x 32 words) give it twice the tiles and end sooner (1e12: 0.56 against
+// 0.61 ms, 1e15: 1.59 against 1.85; 2e15 even, 4e15: 3.42 against 2.99).  A
+// shape the caller or the tuner chose stays.
+static const uint64_t SMALL_SHAPE_X = 2000000000000000ull;
+struct ShapeScope {
+  cpx_ctx *c;
+  SegShape keep;
+  ShapeScope(cpx_ctx *ctx, const std::vector<HostQuery> &hq) : c(ctx), keep(ctx->shape)
+  {
+    if (!c->shape_tuned && hq.size() == 1 && hq[0].x < SMALL_SHAPE_X) c->shape = SegShape{256, 32};
+  }
+  ~ShapeScope() { c->shape = keep; }
+};
+
 static int submit_impl(cpx_ctx *c, const std::vector<HostQuery> &hq_in, uint32_t mask, uint32_t p2mode,
                        bool use_graph, uint32_t *slot_out)
 {
@@ -1429,6 +1467,7 @@ static int submit_impl(cpx_ctx *c, const std::vector<HostQuery> &hq_in, uint32_t
     if (!c->slot[i].busy) { si = i; break; }
   if (si == CPX_SLOTS) return ctx_fail(c, CPX_ESTATE, "every batch slot holds an uncollected batch");
   BatchSlot &S = c->slot[si];
+  const ShapeScope shape_scope(c, hq_in);
   for (auto &ev : S.ev)
     if (!ev) HIPCHK(hipEventCreateWithFlags(&ev, hipEventDefault));
   std::vector<HostQuery> hq(hq_in);
@@ -1480,6 +1519,7 @@ static int submit_impl(cpx_ctx *c, const std::vector<HostQuery> &hq_in, uint32_t
   HIPCHK(hipEventRecord(S.ev[1], c->stream));
   S.busy = true;
   S.ticket = c->next_ticket++;
+  S.shape = c->shape;
   S.nq = hq.size();
   S.t_submit = t0;
   S.ms_tables = tt1 - tt0;
@@ -1528,8 +1568,8 @@ int collect_queries(cpx_ctx *c, uint32_t si, std::vector<ResultDev> &res, cpx_ba
     st->tiles = S.tiles;
     st->hard_segments = S.hard_segments;
     st->p2_segments = S.p2_segments;
-    st->seg_threads = (uint32_t)c->shape.threads;
-    st->seg_kwords = (uint32_t)c->shape.kwords;
+    st->seg_threads = (uint32_t)S.shape.threads;
+    st->seg_kwords = (uint32_t)S.shape.kwords;
     st->passes = S.passes;
   }
   return CPX_OK;
@@ -1589,6 +1629,7 @@ int run_queries_at(cpx_ctx *c, std::vector<HostQuery> &hq, void *d_region, uint6
   HIPCHK(up(L.triv, pl.ntriv * sizeof(BlockDesc)));
   HIPCHK(up(L.easy, pl.neasy * sizeof(BlockDesc)));
   HIPCHK(up(L.p2d, pl.np2d * sizeof(BlockDesc)));
+  HIPCHK(up(L.dir, pl.ndir * sizeof(BlockDesc)));
   HIPCHK(up(L.fin, pl.nfin * sizeof(BlockDesc)));
   HIPCHK(up(L.rowinfo, pl.nrows * sizeof(HardRowInfo)));
   const BatchDev b = batchdev_at(c, L, P0, O0);
@@ -1705,6 +1746,7 @@ int stream_plan(cpx_ctx *c, std::vector<HostQuery> &hq, BatchSlot &S, const Caps
                           {L.easy + base.easy * sizeof(BlockDesc), pl.neasy * sizeof(BlockDesc)},
                           {L.fin + base.fin * sizeof(BlockDesc), pl.nfin * sizeof(BlockDesc)},
                           {L.p2d + base.p2d * sizeof(BlockDesc), pl.np2d * sizeof(BlockDesc)},
+                          {L.dir + base.dir * sizeof(BlockDesc), pl.ndir * sizeof(BlockDesc)},
                           {L.rowinfo + base.rows * sizeof(HardRowInfo), pl.nrows * sizeof(HardRowInfo)}};
   ci->nranges = 0;
   ci->copy_bytes = 0;

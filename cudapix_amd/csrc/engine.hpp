@@ -21,7 +21,8 @@ struct DBuf {
 struct HostQuery {
   u128 x;
   uint64_t y, z, zt, sqrtx, cbrtx, qrtx, sqrtz;
-  uint32_t c;
+  uint32_t c;               // wheel of the ordinary leaves
+  uint32_t cs;              // wheel of the segment sieve (>= c): hard stages c < b <= cs need no sieve
   bool small;               // answered from the pi table (x < CPX_SMALL_X)
   bool p2tab;               // P2 by pi-table lookups of x/p (the table covers x/(y+1))
 };
@@ -38,12 +39,12 @@ enum : uint32_t {
 // Fixed-capacity batch arena: array offsets depend only on capacities, so
 // the pointers baked into a captured graph stay valid until a capacity grows.
 struct Caps {
-  uint64_t q, stages, tiles, groups, ord, triv, easy, fin, p2d, tm, rows, p2rows, parts, mm, mrows;
+  uint64_t q, stages, tiles, groups, ord, triv, easy, fin, p2d, dir, tm, rows, p2rows, parts, mm, mrows;
   uint64_t base;   // per-stage survivor totals of a run in passes (0 otherwise)
 };
 
 struct Layout {
-  size_t counters, queries, stages, tiles, groups, ord, triv, easy, fin, p2d, rowinfo, plan_bytes;
+  size_t counters, queries, stages, tiles, groups, ord, triv, easy, fin, p2d, dir, rowinfo, plan_bytes;
   size_t hard_T, hard_M, hard_bact, hard_acc, hard_base, p2_cnt, p2_np, p2_loc, parts, results, out_bytes;
 };
 
@@ -69,6 +70,7 @@ struct BatchSlot {
   // the batch in flight
   bool busy = false;
   uint64_t ticket = 0;
+  SegShape shape{0, 0};
   size_t nq = 0;
   double t_submit = 0, ms_tables = 0, ms_plan = 0;
   uint64_t tiles = 0, hard_segments = 0, p2_segments = 0;

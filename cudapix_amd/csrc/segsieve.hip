@@ -23,7 +23,8 @@ __global__ __launch_bounds__(T, 4) void k_segments(BatchDev bd)
   }
 }
 
-size_t seg_lds_bytes(SegShape shape) { return (size_t)(shape.kwords + 1) * shape.threads * 4; }
+// Units of 1024 bits with one padding word each.
+size_t seg_lds_bytes(SegShape shape) { return (size_t)(shape.seg_bits() / 1024) * 33 * 4; }
 
 // One-wavefront workgroups (T = 64) make every block barrier a single-wave
 // barrier and let ~15 independent segment workers share a CU.

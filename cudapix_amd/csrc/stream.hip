@@ -286,9 +286,10 @@ static __device__ __attribute__((noinline)) void stream_comb(const BatchDev &bd,
 template <int T>
 static __device__ __attribute__((noinline)) void stream_term(const BatchDev &bd, const TileDev &tile, uint32_t *lds)
 {
-  const bool ord = tile.group == CPX_TILE_ORD;
-  const BlockDesc d = ord ? bd.ord_desc[tile.seg] : bd.triv_desc[tile.seg];
-  const i128 v = ord ? ordinary_part<T>(bd, d, threadIdx.x) : trivial_part<T>(bd, d, threadIdx.x);
+  const bool ord = tile.group == CPX_TILE_ORD, dir = tile.group == CPX_TILE_DIR;
+  const BlockDesc d = ord ? bd.ord_desc[tile.seg] : dir ? bd.dir_desc[tile.seg] : bd.triv_desc[tile.seg];
+  const i128 v = ord ? ordinary_part<T>(bd, d, threadIdx.x)
+                     : dir ? direct_part<T>(bd, d, threadIdx.x) : trivial_part<T>(bd, d, threadIdx.x);
   const i128 s = block_sum_i128(v, reinterpret_cast<i128 *>(lds));
   if (threadIdx.x == 0) st_out(&bd.parts[bd.queries[d.query].part_off + d.part], s);
 }
@@ -309,7 +310,7 @@ static __device__ __forceinline__ void stream_main(const BatchDev &bd, const Bat
     easy_tile<T, K>(bd, (uint32_t)tile.seg, lds, sh);
   } else if (tile.group == CPX_TILE_P2) {
     p2tab_tile<T, K>(bd, (uint32_t)tile.seg, lds);
-  } else if (tile.group == CPX_TILE_ORD || tile.group == CPX_TILE_TRIV) {
+  } else if (tile.group == CPX_TILE_ORD || tile.group == CPX_TILE_TRIV || tile.group == CPX_TILE_DIR) {
     stream_term<T>(*bd_mem, tile, lds);
   } else {
     hard_segment<T, K>(bd, tile, lds, sh);

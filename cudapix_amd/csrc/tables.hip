@@ -270,12 +270,27 @@ __global__ __launch_bounds__(256) void k_mlpf(int32_t *mlpf, uint32_t *lpf_out, 
   }
 }
 
+// The leaf table from the mu*lpf table: thread i writes m = 2i + 1 if coprime to 30030.
+__global__ __launch_bounds__(256) void k_mleaf(const int32_t *__restrict__ mlpf, uint64_t nodd, int2 *out)
+{
+  const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nodd) return;
+  const uint32_t m = 2 * (uint32_t)i + 1, b = m / 30030u, k = (m - b * 30030u) >> 1;
+  const PiEntry e = cop30030_table.e[k >> 5];
+  if (!((e.bits >> (k & 31u)) & 1u)) return;
+  out[b * COP30030_TOT + e.count + cpx_popc32(e.bits & cpx_lowmask32(k & 31u))] = make_int2((int)m, mlpf[i]);
+}
+
+// mu*lpf of nodd odd m (a multiple of 4096), and after it the leaf table:
+// cpx_mlpf_words(nodd) words in all.
 hipError_t launch_mlpf(int32_t *mlpf, uint64_t nodd, const uint32_t *primes, uint32_t nsp,
                        hipStream_t s)
 {
   uint32_t g = (uint32_t)((nodd + MLPF_SEG - 1) / MLPF_SEG);
   hipLaunchKernelGGL(k_mlpf, dim3(g), dim3(256), 0, s, mlpf, (uint32_t *)nullptr,
                      (int8_t *)nullptr, (uint64_t)0, nodd, primes, nsp);
+  hipLaunchKernelGGL(k_mleaf, dim3((uint32_t)((nodd + 255) / 256)), dim3(256), 0, s, mlpf, nodd,
+                     reinterpret_cast<int2 *>(mlpf + nodd));
   return hipGetLastError();
 }
 
@@ -377,11 +392,35 @@ __global__ __launch_bounds__(256) void k_wheel(PiEntry *wheel, uint32_t period, 
   }
 }
 
+// Segment pattern of a wheel: word w holds the integers of [120 w, 120 w + 120)
+// coprime to 30 (bit 8q + i: 30q + the i-th residue), with the multiples of
+// 7 .. p_c cleared.
+__global__ __launch_bounds__(256) void k_wheel_pattern(uint32_t *pat, uint32_t period, uint32_t c)
+{
+  const uint32_t sp[8] = {2, 3, 5, 7, 11, 13, 17, 19}, res[8] = {1, 7, 11, 13, 17, 19, 23, 29};
+  for (uint32_t w = blockIdx.x * blockDim.x + threadIdx.x; w < period; w += gridDim.x * blockDim.x) {
+    uint32_t bits = 0;
+    for (uint32_t i = 0; i < 32; i++) {
+      const uint32_t n = 120 * w + 30 * (i >> 3) + res[i & 7];
+      bool ok = true;
+      for (uint32_t k = 3; k < c; k++) ok = ok && (n % sp[k] != 0);
+      bits |= (uint32_t)ok << i;
+    }
+    pat[w] = bits;
+  }
+}
+
+// The wheel of the first c primes at `wheel`: `period` entries of odd-only bits
+// (none if 0) and, from entry period + 1, the segment pattern (7 * .. * p_c words).
 hipError_t launch_wheel(PiEntry *wheel, uint32_t period, uint32_t c, hipStream_t s)
 {
-  uint32_t g = (period + 255) / 256;
-  if (g > 4096) g = 4096;
-  hipLaunchKernelGGL(k_wheel, dim3(g), dim3(256), 0, s, wheel, period, c);
+  const uint32_t sp[8] = {2, 3, 5, 7, 11, 13, 17, 19};
+  uint32_t pp = 1;
+  for (uint32_t k = 3; k < c; k++) pp *= sp[k];
+  if (period)
+    hipLaunchKernelGGL(k_wheel, dim3(std::min((period + 255) / 256, 4096u)), dim3(256), 0, s, wheel, period, c);
+  hipLaunchKernelGGL(k_wheel_pattern, dim3(std::min((pp + 255) / 256, 4096u)), dim3(256), 0, s,
+                     reinterpret_cast<uint32_t *>(wheel + period + 1), pp, c);
   return hipGetLastError();
 }
 

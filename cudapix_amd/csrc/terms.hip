@@ -36,7 +36,7 @@ __global__ __launch_bounds__(256) void k_setup(BatchDev bd)
       q.pi_e = pi_lookup(bd.pitab, q.p2_e);
     }
     for (uint32_t s = threadIdx.x; s < q.nstage; s += blockDim.x) {
-      uint32_t p = bd.primes[q.c + s];
+      uint32_t p = bd.primes[q.cs + s];
       StageDev d;
       d.p = p;
       d.ylo = (uint32_t)(q.y / p);
@@ -65,14 +65,16 @@ hipError_t launch_setup(BatchDev b, uint32_t grid, uint32_t, hipStream_t s)
 }
 
 // ----------------------------------------------------------- ordinary
-// S0 (ordinary_part, cpx_terms.hpp), one descriptor per block iteration.
+// S0 (ordinary_part, cpx_terms.hpp) and the hard leaves of the wheel stages
+// (direct_part), one descriptor per block iteration.
 __global__ __launch_bounds__(256) void k_ordinary(BatchDev bd)
 {
   __shared__ i128 red[4];
-  const uint32_t nd = *bd.n_ord;
+  const uint32_t no = *bd.n_ord, nd = no + *bd.n_dir;
   for (uint32_t di = blockIdx.x; di < nd; di += gridDim.x) {
-    const BlockDesc d = bd.ord_desc[di];
-    i128 t = block_sum_i128(ordinary_part<256>(bd, d, threadIdx.x), red);
+    const BlockDesc d = di < no ? bd.ord_desc[di] : bd.dir_desc[di - no];
+    const i128 v = di < no ? ordinary_part<256>(bd, d, threadIdx.x) : direct_part<256>(bd, d, threadIdx.x);
+    i128 t = block_sum_i128(v, red);
     if (threadIdx.x == 0) bd.parts[bd.queries[d.query].part_off + d.part] = t;
   }
 }
