@@ -63,6 +63,17 @@ __device__ __forceinline__ uint64_t cpx_div_leaf_r(uint64_t a, double af, uint32
   return q;
 }
 
+// floor(sqrt(v)) for any v: the f64 root of the f64 nearest to v is within one
+// of it (and below 2^32 after the clamp, so no square wraps), then one exact
+// step either way.
+__device__ __forceinline__ uint64_t isqrt64_dev(uint64_t v)
+{
+  uint64_t s = min((uint64_t)__builtin_sqrt((double)v), 0xffffffffull);
+  if (s * s > v) s--;
+  else if (s < 0xffffffffull && (s + 1) * (s + 1) <= v) s++;
+  return s;
+}
+
 // Sum of 32-bit values over the wavefront, in every lane (DPP scan, then lane 63).
 __device__ __forceinline__ uint32_t wave_sum(uint32_t v)
 {

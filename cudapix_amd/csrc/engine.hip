@@ -373,7 +373,13 @@ int ensure_tables(cpx_ctx *c, uint64_t R, uint64_t P, uint64_t Y)
 
 static uint64_t ceil_div(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
 
-static const uint64_t ORD_CH = 2048, TRIV_CH = 4096, EASY_WORK = 131072, P2_CH = 65536;
+static const uint64_t ORD_CH = 2048, TRIV_CH = 4096, P2_CH = 65536;
+// Lookups of one easy-leaf tile: EASY_WORK where the batch has plenty, fewer
+// (to EASY_MIN) where the batch's tiles would not give every block of the
+// grid a few: a tile of 131072 lookups takes about 100 us on its own, as
+// long as all of the easy leaves of one query at 1e13 (V at 1e14 alone: 240 us
+// with 131072, 220 with 32768; 8192 to 32768 are even).
+static const uint64_t EASY_WORK = 131072, EASY_MIN = 32768, EASY_TILES = 2048;
 
 static void plan_needs(const cpx_ctx *c, const HostQuery &h, uint32_t mask, uint64_t seg_bits,
                        uint64_t *R, uint64_t *P, uint64_t *Y)
@@ -456,8 +462,29 @@ static inline uint16_t cost_bucket(double cost)
   return (uint16_t)std::min(std::max(b, 0), PLAN_NB - 1);
 }
 
-static void plan_query(const cpx_ctx *c, const HostQuery &h, uint32_t i, uint32_t mask, QPlan &qp)
-// (i: the query's index in the arena's query array, which its descriptors name)
+// Cuts the primes [j0, j0 + w.size()) with work w each into descriptors of
+// `unit` work at least (the last one less).
+static void cut_work(const std::vector<uint32_t> &w, uint64_t j0, uint64_t unit, uint32_t i, uint32_t &part,
+                     std::vector<BlockDesc> &out)
+{
+  uint64_t b = 0, work = 0;
+  for (uint64_t k = 0; k < w.size(); k++) {
+    work += w[k];
+    if (work >= unit || k + 1 == w.size()) {
+      out.push_back({i, part++, j0 + b, j0 + k + 1});
+      b = k + 1;
+      work = 0;
+    }
+  }
+}
+
+static uint64_t easy_unit(uint64_t total, size_t nq)
+{
+  return std::min(EASY_WORK, std::max(EASY_MIN, total * nq / EASY_TILES));
+}
+
+static void plan_query(const cpx_ctx *c, const HostQuery &h, uint32_t i, uint32_t mask, QPlan &qp, size_t nq)
+// (i: the query's index in the arena's query array, which its descriptors name; nq: queries of the batch)
 {
   const uint64_t SI = c->shape.seg_ints();
   const uint32_t T = (uint32_t)c->shape.threads;
@@ -509,22 +536,23 @@ static void plan_query(const cpx_ctx *c, const HostQuery &h, uint32_t i, uint32_
   if (mask & TERM_EASY_A) ej1 = std::min<uint64_t>(ej1, d.pi_sqrtz);
   if (mask & TERM_EASY_B) ej0 = std::max<uint64_t>(ej0, d.pi_sqrtz);
   if ((mask & TERM_EASY) && ej1 > ej0) {
-    // work estimate only: q-count pi(min(y, x/p^2)) - j - 1, with x/p^2 in
-    // doubles and pi by a pointer that only moves down as p grows
-    uint64_t j0 = ej0, work = 0;
+    // work estimate only: lookups pi(min(y, x/p^2, sqrt(x/p))) - j - 1, with
+    // the bounds in doubles and pi by a pointer that only moves down as p grows
+    std::vector<uint32_t> w(ej1 - ej0);
+    uint64_t total = 0;
     const double fx = (double)h.x;
     uint64_t k1 = d.a;                                  // pi(y)
     for (uint64_t j = ej0; j < ej1; j++) {
       const double p = (double)c->h_primes[j];
-      const double qm = std::min((double)h.y, fx / (p * p));
-      while (k1 > 0 && (double)c->h_primes[k1 - 1] > qm) k1--;
-      work += (k1 > j + 1 ? k1 - j - 1 : 0) + 64;
-      if (work >= EASY_WORK || j + 1 == ej1) {
-        qp.easy.push_back({i, part++, j0, j + 1});
-        j0 = j + 1;
-        work = 0;
+      const double xp = fx / p, qm = std::min((double)h.y, xp / p);
+      for (; k1 > 0; k1--) {
+        const double r = (double)c->h_primes[k1 - 1];
+        if (r <= qm && r * r <= xp) break;
       }
+      w[j - ej0] = (uint32_t)((k1 > j + 1 ? k1 - j - 1 : 0) + 64);
+      total += w[j - ej0];
     }
+    cut_work(w, ej0, easy_unit(total, nq), i, part, qp.easy);
   }
   d.n_easy_parts = part - d.n_ord_parts - d.n_triv_parts;
   // hard carry: one block per CPX_FIN_STAGES stages
@@ -544,18 +572,19 @@ static void plan_query(const cpx_ctx *c, const HostQuery &h, uint32_t i, uint32_
     if (js < d.B && ((h.x / c->h_primes[js]) >> 64) == 0) {
       d.omega = 1;
       const uint64_t ky = d.a;                                          // pi(y)
-      uint64_t j0 = js, work = 0;
+      std::vector<uint32_t> w(d.B - js);
+      uint64_t total = 0;
       for (uint64_t j = js; j < d.B; j++) {
         const uint64_t p = c->h_primes[j];
         const u128 t3 = h.x / ((u128)p * p * p);
         const uint64_t k0 = std::max<uint64_t>(j + 1, t3 >= h.y ? ky : host_pi(c, (uint64_t)t3));
-        work += (ky > k0 ? ky - k0 : 0) + 64;
-        if (work >= EASY_WORK || j + 1 == d.B) {
-          qp.easy.push_back({i, part++, j0, j + 1});
-          j0 = j + 1;
-          work = 0;
-        }
+        // lookups to min(y, sqrt(x/p)) (the y's prime index scaled: an estimate)
+        const double sc = std::min(1.0, std::sqrt((double)h.x / (double)p) / (double)h.y);
+        const uint64_t ke = sc < 1.0 ? std::max<uint64_t>(k0, (uint64_t)((double)ky * sc)) : ky;
+        w[j - js] = (uint32_t)((ke > k0 ? ke - k0 : 0) + 64);
+        total += w[j - js];
       }
+      cut_work(w, js, easy_unit(total, nq), i, part, qp.easy);
     }
   }
   // hard leaves of the wheel stages c < b <= cs: odd m in (y / p_cs, y]
@@ -836,7 +865,7 @@ static int build_plan(cpx_ctx *c, const std::vector<HostQuery> &hq, uint32_t mas
   std::vector<QPlan> &qps = pl.qps;
   qps.assign(nq, QPlan());
   const unsigned nt = plan_threads(nq);
-  parallel_for(nq, nt, [&](size_t i) { plan_query(c, hq[i], (uint32_t)(B.q + i), mask, qps[i]); });
+  parallel_for(nq, nt, [&](size_t i) { plan_query(c, hq[i], (uint32_t)(B.q + i), mask, qps[i], nq); });
   pl.groups.clear();
   make_groups(c, hq, qps, pl.groups);
   std::vector<GPlan> gps(pl.groups.size());
@@ -1305,7 +1334,12 @@ uint64_t plan_bytes_estimate(const cpx_ctx *c, const HostQuery &h)
   // T and M per pair (M rows of replicated segments add some: a group's
   // leaf-dense segments give every member the group's replicas), rowinfo,
   // bact and the P2 rows, stage and carry descriptors, easy descriptors
-  double bytes = pairs * 8 * 1.5 + hseg * 48 + p2seg * 16 + 4096 + B * 80 + (h.y / 2048.0 + 32) * 48;
+  // easy-leaf descriptors (with a part and a tile each): a few per EASY_MIN
+  // pairs up to about EASY_TILES each for V and the hard leaves, then per EASY_WORK
+  const double cb = (double)h.cbrtx + 3, fy = (double)h.y + 3;
+  const double lookups = 1.6 * cb / std::log(cb) * fy / std::log(fy);
+  const double edesc = 4 + std::min(lookups / EASY_MIN, 2.0 * EASY_TILES) + lookups / EASY_WORK;
+  double bytes = pairs * 8 * 1.5 + hseg * 48 + p2seg * 16 + 4096 + B * 80 + (h.y / 2048.0 + 32) * 48 + edesc * 64;
   return (uint64_t)bytes;
 }
 

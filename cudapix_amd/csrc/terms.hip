@@ -147,14 +147,6 @@ hipError_t launch_combine(BatchDev b, uint32_t grid, hipStream_t s)
 // then thread 0 stores the four per-p parts {A_p, pi(x/(p y)) if p <= sqrt z,
 // pi(min(y, x/p^2)) if p > sqrt z, -pi(sqrt(x/p))^2}.  Needs x/p < 2^64,
 // the prime list to sqrt(x/p) and the pi table to sqrt(x).
-static __device__ __forceinline__ uint64_t isqrt64_dev(uint64_t v)
-{
-  uint64_t s = (uint64_t)sqrt((double)v);
-  while ((u128)s * s > v) s--;
-  while ((u128)(s + 1) * (s + 1) <= v) s++;
-  return s;
-}
-
 __global__ __launch_bounds__(256) void k_sigma(uint64_t x_lo, uint64_t x_hi, uint64_t y, uint64_t sz,
                                                const uint32_t *__restrict__ primes,
                                                const PiEntry *__restrict__ pitab, uint64_t j0,
