@@ -487,7 +487,6 @@ static void plan_query(const cpx_ctx *c, const HostQuery &h, uint32_t i, uint32_
 // (i: the query's index in the arena's query array, which its descriptors name; nq: queries of the batch)
 {
   const uint64_t SI = c->shape.seg_ints();
-  const uint32_t T = (uint32_t)c->shape.threads;
   QueryDev &d = qp.d;
   d.x_lo = (uint64_t)h.x;
   d.x_hi = (uint64_t)(h.x >> 64);
@@ -601,16 +600,16 @@ static void plan_query(const cpx_ctx *c, const HostQuery &h, uint32_t i, uint32_
   }
   d.n_p2_parts = part - d.n_ord_parts - d.n_triv_parts - d.n_easy_parts - d.n_hard_parts;
   qp.parts = part;
-  // hard rows: active stages per segment and, for the low (leaf-dense)
-  // segments, an estimate of the leaves to evaluate (replicas are chosen per
-  // group, from the members' leaves of the segment)
+  // hard rows: active stages per segment, and an estimate of the leaves to
+  // evaluate (replicas are chosen per group, from the members' leaves of the
+  // segment), taken at segments about a twelfth of their number apart and
+  // linear between them
   std::vector<double> xps;
   if (d.hard_nseg) {
     xps.resize(d.nstage);
     for (uint32_t k = 0; k < d.nstage; k++) xps[k] = (double)(h.x / c->h_primes[h.cs + k]);
   }
-  const double leaf_target = 256.0 * T;
-  uint32_t sparse_run = 0;
+  uint64_t knot = 0, prev = 0;
   uint64_t toff = 0;
   uint64_t act = d.nstage;                             // non-increasing in the segment
   qp.rowinfo.reserve(d.hard_nseg);
@@ -624,8 +623,8 @@ static void plan_query(const cpx_ctx *c, const HostQuery &h, uint32_t i, uint32_
       if (p * p * (u128)lo <= h.x) break;
       act--;
     }
+    const bool est = s == knot || s + 1 == d.hard_nseg;
     double leaves = 0, leafy = 0;
-    const bool est = sparse_run < 4;
     const double inv_lo = lo ? 1.0 / (double)lo : 0.0, inv_hi = 1.0 / (double)hi;
     const double fy = (double)h.y;
     // (a sample of at most 32 stages, scaled: the estimate only sizes replicas)
@@ -643,11 +642,19 @@ static void plan_query(const cpx_ctx *c, const HostQuery &h, uint32_t i, uint32_
         leaves += kstep * (sparse ? (mhi - mlo) / std::log(mhi) : 0.192 * (mhi - mlo));
       }
     }
-    if (est) sparse_run = leaves < leaf_target / 4 ? sparse_run + 1 : 0;
     qp.rowinfo.push_back({0u, 0u, (uint32_t)act, 0u, toff, 0u});
     qp.rleaves.push_back((float)leaves);
     qp.rleafy.push_back((float)leafy);
     toff += act;
+    if (est) {
+      for (uint64_t r = prev + 1; r < s; r++) {
+        const float f = (float)(r - prev) / (float)(s - prev);
+        qp.rleaves[r] = qp.rleaves[prev] + f * ((float)leaves - qp.rleaves[prev]);
+        qp.rleafy[r] = qp.rleafy[prev] + f * ((float)leafy - qp.rleafy[prev]);
+      }
+      prev = s;
+      knot = s + 1 + s / 12;
+    }
   }
   qp.tm = toff;
   // carry blocks: rows with their first stage active (act is non-increasing)
@@ -696,16 +703,21 @@ static void make_groups(const cpx_ctx *c, const std::vector<HostQuery> &hq,
   if (cur.n) groups.push_back(cur);
 }
 
+// Weights of the replica rule: a stage of a segment costs a block about what
+// STAGE_LEAVES leaf candidates do, and a replica (which sieves the segment
+// again) is not made for less than REP_SIEVE times its sieve where the chip is
+// full anyway.
+static const double STAGE_LEAVES = 143.0, REP_SIEVE = 16.0;
+
 // Replicas, M rows and tiles of one group: a segment's replica count comes
 // from all members' leaves there; every member with the segment in its hard
 // range gets that many M rows.  Tile cost: the shared sieve once, each
 // member's leaves, and on replica 0 the P2 sieve and counts.
 static void plan_group(const cpx_ctx *c, const GroupDev &g, uint32_t gi, std::vector<QPlan> &qps,
-                       GPlan &gp)
+                       double block_work, GPlan &gp)
 {
   const uint64_t SB = c->shape.seg_bits();
   const uint32_t T = (uint32_t)c->shape.threads;
-  const double leaf_target = 256.0 * T;
   uint64_t nseg = 0;
   for (uint32_t m = 0; m < g.n; m++) nseg = std::max(nseg, qps[g.q[m]].d.hard_nseg);
   const uint32_t cw = qps[g.q[0]].d.cs;
@@ -724,7 +736,9 @@ static void plan_group(const cpx_ctx *c, const GroupDev &g, uint32_t gi, std::ve
       act = std::max(act, qp.rowinfo[s].act);
       if (s >= qp.d.p2_seg0 && s < qp.d.p2_seg0 + qp.d.p2_nseg) np2++;
     }
-    const uint32_t nrep = (uint32_t)std::min(64.0, std::max(1.0, std::ceil(leaves / leaf_target)));
+    const double most = std::max(524288.0, REP_SIEVE * STAGE_LEAVES * (double)act);
+    const double per = std::max(16384.0, std::min(block_work, most));
+    const uint32_t nrep = (uint32_t)std::min(64.0, std::max(1.0, std::ceil(leaves / per)));
     for (uint32_t m = 0; m < g.n; m++) {
       QPlan &qp = qps[g.q[m]];
       if (s >= qp.d.hard_nseg) continue;
@@ -868,9 +882,26 @@ static int build_plan(cpx_ctx *c, const std::vector<HostQuery> &hq, uint32_t mas
   parallel_for(nq, nt, [&](size_t i) { plan_query(c, hq[i], (uint32_t)(B.q + i), mask, qps[i], nq); });
   pl.groups.clear();
   make_groups(c, hq, qps, pl.groups);
+  // leaves of one tile (a segment with more becomes replicas): 16 K at least,
+  // 512 K at most, between them four fifths of the work of one of 512 blocks,
+  // so that no tile outlasts the others' work and none is sieved more often
+  // than that needs.  Best of {32 .. 2048} x 512 measured: 1e13 32 K, 1e15 and
+  // 256 queries to 1e13 64 K, 64 queries to 1e15 256 K, 1e16 and 512 queries
+  // to 1e15 512 K; a fixed 128 K cost 1e16 9 %, the 512 queries 25 % and 64
+  // queries to 1e12 90 %.
+  double work = 0;
+  for (const QPlan &qp : qps)
+    for (float l : qp.rleaves) work += l;
+  for (const GroupDev &g : pl.groups) {
+    const QPlan *longest = &qps[g.q[0]];
+    for (uint32_t m = 1; m < g.n; m++)
+      if (qps[g.q[m]].tm > longest->tm) longest = &qps[g.q[m]];
+    work += STAGE_LEAVES * (double)longest->tm;
+  }
+  const double block_work = 0.8 * work / 512.0;
   std::vector<GPlan> gps(pl.groups.size());
   parallel_for(pl.groups.size(), nt,
-               [&](size_t g) { plan_group(c, pl.groups[g], (uint32_t)g, qps, gps[g]); });
+               [&](size_t g) { plan_group(c, pl.groups[g], (uint32_t)g, qps, block_work, gps[g]); });
   // place the shares: global offsets of every query's rows, parts and counters
   std::vector<PlanOff> &off = pl.off;
   off.resize(nq);
