@@ -103,10 +103,12 @@ static __device__ __forceinline__ bool slot_of(const StreamPub *pub, uint32_t ns
 // host may reuse the record, so a head read before a record's reuse no longer
 // matches at the compare-and-swap.  A claim at or past the count (read again
 // after the claim) is no work.
-// A claim takes a run of up to (count / (2 * grid), at most 64) units: a
-// cohort's carry has thousands of units of a few microseconds each, and one
-// compare-and-swap (plus its accounting) per unit made the claims, not the
-// units, the cost of the phase.
+// A claim takes a run of 16 to 64 units (two shares of the count): a cohort's
+// carry has thousands of units of a few microseconds each, every idle block
+// contends for the one head, and a claim reads pinned memory between its load
+// and its compare-and-swap, so about one succeeds per bus round trip and the
+// claims are the cost of the phase.  (A burst of 100 requests below 1e14, whose
+// carry is about 3000 units: 23 ms with runs of 2, 4 ms with 16.)
 static __device__ __forceinline__ bool claim_phase(uint64_t *head, const uint64_t *count, uint64_t *idx,
                                                    uint32_t *n)
 {
@@ -117,8 +119,8 @@ static __device__ __forceinline__ bool claim_phase(uint64_t *head, const uint64_
     order_acquire();
     const uint64_t cnt = ld_sys(count);
     if (i >= cnt) return false;
-    uint64_t k = cnt / (2ull * gridDim.x);
-    k = k < 1 ? 1 : (k > 64 ? 64 : k);
+    uint64_t k = 2 * cnt / gridDim.x;
+    k = k < 16 ? 16 : (k > 64 ? 64 : k);
     if (k > cnt - i) k = cnt - i;
     if (cas_dev(head, v, v + k)) {
       order_acquire();
@@ -151,9 +153,13 @@ static __device__ __forceinline__ bool claim_fifo(uint64_t *head, uint64_t end, 
 // (each claim a compare-and-swap at device scope), so while many tiles are
 // left a claim takes a run of up to 16 consecutive tiles (1 near the end,
 // where the longest-first order leaves the short tiles to balance the grid).
+// Two shares of what is left: the same burst's main phase took 17 ms with a
+// quarter share, 11 with a half, 9 with one; at three the largest cohorts'
+// last long runs show (16 requests to 1e16: 12.5 ms with one share, 14.4 with
+// two, 15-17 with three; 512 requests to 1e13: 22, 16.5 and 16 ms).
 static __device__ __forceinline__ uint64_t main_claim_run(uint64_t left)
 {
-  const uint64_t k = left / (4ull * gridDim.x);
+  const uint64_t k = 2 * left / gridDim.x;
   return k < 1 ? 1 : (k > 16 ? 16 : k);
 }
 
