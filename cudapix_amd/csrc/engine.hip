@@ -1081,6 +1081,7 @@ static int ensure_arena_caps(cpx_ctx *c, BatchSlot &S, const Caps &need, uint64_
   if ((e = cpx_dev_malloc(&S.d_out, L.out_bytes)) != hipSuccess) { S.d_out = nullptr; (void)hipGetLastError(); return fail(hip_fail(c, e, "hipMalloc(out)")); }
   if ((e = hipHostMalloc(&S.h_plan, L.plan_bytes, hipHostMallocDefault)) != hipSuccess) { S.h_plan = nullptr; return fail(hip_fail(c, e, "hipHostMalloc")); }
   if ((e = hipHostMalloc(&S.h_res, kk.q * sizeof(ResultDev), hipHostMallocDefault)) != hipSuccess) { S.h_res = nullptr; return fail(hip_fail(c, e, "hipHostMalloc")); }
+  if ((e = hipHostGetDevicePointer((void **)&S.d_res, S.h_res, 0)) != hipSuccess) return fail(hip_fail(c, e, "hipHostGetDevicePointer"));
   S.L = L;
   return CPX_OK;
 }
@@ -1242,14 +1243,26 @@ static void pack_stages(const cpx_ctx *c, const Layout &L, const Plan &pl, char 
   });
 }
 
-// Writes the plan into the slot's pinned staging and queues its copy on the
-// upload stream; the batch stream waits for it (event ev[4]).
-static int upload_plan(cpx_ctx *c, BatchSlot &S, const Plan &pl)
+// Plans up to this many bytes go up in one copy, gaps included (a copy costs
+// about 5 us of host and 3 us of device time, 256 KB of bus about 6 us).
+static const size_t UPLOAD_ONE = 256u << 10;
+
+// Writes the plan into the slot's pinned staging and queues its copy: on the
+// batch stream if no other batch is in flight and the plan is small, else on
+// the upload stream, for which the batch stream waits (event ev[4]).
+static int upload_plan(cpx_ctx *c, BatchSlot &S, const Plan &pl, bool passes)
 {
   CpxRange range("cpx:upload");
   const Layout &L = S.L;
   char *H = (char *)S.h_plan;
   pack_plan(L, pl, H);
+  bool alone = !passes;
+  for (const BatchSlot &o : c->slot) alone = alone && !o.busy;
+  const size_t end = L.rowinfo + pl.nrows * sizeof(HardRowInfo);   // (the last plan array)
+  if (alone && end <= UPLOAD_ONE) {
+    HIPCHK(hipMemcpyAsync(S.d_plan, H, end, hipMemcpyHostToDevice, c->stream));
+    return CPX_OK;
+  }
   // copy only the used prefix of each array
   auto up = [&](size_t off, size_t bytes) -> hipError_t {
     if (!bytes) return hipSuccess;
@@ -1293,30 +1306,30 @@ static const uint32_t GRID_FIN = 16384;
 
 // The launch sequence in three parts; events between the parts time the
 // persistent segment kernel on its own stream (also when replayed as graphs).
-//   part 0: clear results + queue head, setup, ordinary, trivial
+//   part 0: setup, ordinary, wheel-stage and trivial leaves
 //   part 1: persistent segment kernel (hard + P2 segment tiles, easy-leaf
 //           and P2-lookup tiles)
 //   part 2: hard-leaf carry, combine
-static int enqueue_part(cpx_ctx *c, const BatchDev &b, int part, uint32_t nres_words)
+// pl: the plan the launches are for, whose counts bound their grids (null
+// for a captured sequence, which serves every plan of the arena).
+static int enqueue_part(cpx_ctx *c, const BatchDev &b, int part, const Plan *pl)
 {
   CpxRange range(part == 0 ? "cpx:enqueue setup, ordinary, trivial"
                  : part == 1 ? "cpx:enqueue segment kernel" : "cpx:enqueue carry, combine");
+  auto grid = [&](uint32_t most, size_t units) { return pl ? (uint32_t)std::min<size_t>(most, units) : most; };
+  const size_t nq = pl ? pl->q.size() : 1, ntiles = pl ? pl->tiles.size() : 1, nfin = pl ? pl->nfin : 1;
   if (part == 0) {
-    HIPCHK(launch_zero_u32((uint32_t *)b.results, nres_words, c->stream));
-    HIPCHK(launch_zero_u32(b.tile_head, 1, c->stream));
-    HIPCHK(launch_setup(b, GRID_Q, 0, c->stream));
-    HIPCHK(launch_ordinary(b, GRID_T, c->stream));
-    HIPCHK(launch_trivial(b, GRID_T, c->stream));
+    HIPCHK(launch_setup(b, grid(GRID_T, nq + (pl ? pl->nord + pl->ndir + pl->ntriv : 0)), 0, c->stream));
   } else if (part == 1) {
-    HIPCHK(launch_segments(b, c->shape, (uint32_t)seg_grid(c), c->stream));
+    if (ntiles) HIPCHK(launch_segments(b, c->shape, grid((uint32_t)seg_grid(c), ntiles), c->stream));
   } else {
-    HIPCHK(launch_hard_finalize(b, GRID_FIN, c->stream));
-    HIPCHK(launch_combine(b, GRID_Q, c->stream));
+    if (nfin) HIPCHK(launch_hard_finalize(b, grid(GRID_FIN, nfin), c->stream));
+    HIPCHK(launch_combine(b, grid(GRID_Q, nq), c->stream));
   }
   return CPX_OK;
 }
 
-static int ensure_graph(cpx_ctx *c, BatchSlot &S, const BatchDev &b, uint32_t nres_words)
+static int ensure_graph(cpx_ctx *c, BatchSlot &S, const BatchDev &b)
 {
   if (S.gexec[0] && S.graph_gen == c->generation && S.graph_arena_gen == S.arena_gen &&
       S.graph_shape.threads == c->shape.threads && S.graph_shape.kwords == c->shape.kwords)
@@ -1328,7 +1341,7 @@ static int ensure_graph(cpx_ctx *c, BatchSlot &S, const BatchDev &b, uint32_t nr
   for (int part = 0; part < 3; part++) {
     hipGraph_t g;
     HIPCHK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
-    int rc = enqueue_part(c, b, part, nres_words);
+    int rc = enqueue_part(c, b, part, nullptr);
     hipError_t e2 = hipStreamEndCapture(c->stream, &g);
     if (rc) return rc;
     if (e2 != hipSuccess) return hip_fail(c, e2, "hipStreamEndCapture");
@@ -1469,11 +1482,10 @@ static bool plan_passes(const cpx_ctx *c, Plan &pl, PassPlan &pp)
 // so the host waits for the previous pass before it stages the next), the
 // segment kernel over its tiles and the carry blocks over its rows; then the
 // combine.
-static int launch_passes(cpx_ctx *c, BatchSlot &S, const Plan &pl, const PassPlan &pp, const BatchDev &b0,
-                         uint32_t nres_words)
+static int launch_passes(cpx_ctx *c, BatchSlot &S, const Plan &pl, const PassPlan &pp, const BatchDev &b0)
 {
   HIPCHK(hipEventRecord(S.ev[0], c->stream));
-  int rc = enqueue_part(c, b0, 0, nres_words);
+  int rc = enqueue_part(c, b0, 0, &pl);
   if (rc) return rc;
   BatchDev b = b0;
   b.hard_base = (uint64_t *)((char *)S.d_out + S.L.hard_base);
@@ -1524,7 +1536,7 @@ struct ShapeScope {
 };
 
 static int submit_impl(cpx_ctx *c, const std::vector<HostQuery> &hq_in, uint32_t mask, uint32_t p2mode,
-                       bool use_graph, uint32_t *slot_out)
+                       bool use_graph, bool timed, uint32_t *slot_out)
 {
   const double t0 = now_ms();
   uint32_t si = CPX_SLOTS;
@@ -1562,25 +1574,22 @@ static int submit_impl(cpx_ctx *c, const std::vector<HostQuery> &hq_in, uint32_t
   }
   if ((rc = ensure_arena(c, S, need))) return rc;
   const double tp = now_ms();
-  if ((rc = upload_plan(c, S, pl))) return rc;
+  if ((rc = upload_plan(c, S, pl, passes))) return rc;
   BatchDev b = make_batchdev(c, S);
+  b.results = S.d_res;
   const bool graph = use_graph && c->opts.use_graphs && !passes;
-  // results region of the arena, in 32-bit words (capacity, so graphs stay valid)
-  const uint32_t nres_words = (uint32_t)(S.caps.q * sizeof(ResultDev) / 4);
-  if (graph && (rc = ensure_graph(c, S, b, nres_words))) return rc;
+  if (graph && (rc = ensure_graph(c, S, b))) return rc;
   if (passes) {
-    if ((rc = launch_passes(c, S, pl, pp, b, nres_words))) return rc;
+    if ((rc = launch_passes(c, S, pl, pp, b))) return rc;
   } else {
-    HIPCHK(hipEventRecord(S.ev[0], c->stream));
+    if (timed) HIPCHK(hipEventRecord(S.ev[0], c->stream));
     for (int part = 0; part < 3; part++) {
-      if (part == 1) HIPCHK(hipEventRecord(S.ev[2], c->stream));
+      if (timed && part == 1) HIPCHK(hipEventRecord(S.ev[2], c->stream));
       if (graph) HIPCHK(hipGraphLaunch(S.gexec[part], c->stream));
-      else if ((rc = enqueue_part(c, b, part, nres_words))) return rc;
-      if (part == 1) HIPCHK(hipEventRecord(S.ev[3], c->stream));
+      else if ((rc = enqueue_part(c, b, part, &pl))) return rc;
+      if (timed && part == 1) HIPCHK(hipEventRecord(S.ev[3], c->stream));
     }
   }
-  HIPCHK(hipMemcpyAsync(S.h_res, (char *)S.d_out + S.L.results, hq.size() * sizeof(ResultDev),
-                        hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipEventRecord(S.ev[1], c->stream));
   S.busy = true;
   S.ticket = c->next_ticket++;
@@ -1598,10 +1607,10 @@ static int submit_impl(cpx_ctx *c, const std::vector<HostQuery> &hq_in, uint32_t
 }
 
 int submit_queries(cpx_ctx *c, const std::vector<HostQuery> &hq, uint32_t mask, uint32_t p2mode,
-                   bool use_graph, uint32_t *slot)
+                   bool use_graph, uint32_t *slot, bool timed)
 {
   if (hq.empty()) return ctx_fail(c, CPX_EINVAL, "empty batch");
-  const int rc = submit_impl(c, hq, mask, p2mode, use_graph, slot);
+  const int rc = submit_impl(c, hq, mask, p2mode, use_graph, timed, slot);
   if (rc) {
     // a failed submission may have queued part of its upload or launches:
     // let them drain before the slot is reused
@@ -1645,7 +1654,7 @@ int run_queries(cpx_ctx *c, const std::vector<HostQuery> &hq, uint32_t mask, uin
 {
   if (hq.empty()) { res.clear(); return CPX_OK; }
   uint32_t si = 0;
-  const int rc = submit_queries(c, hq, mask, p2mode, use_graph, &si);
+  const int rc = submit_queries(c, hq, mask, p2mode, use_graph, &si, st != nullptr);
   if (rc) return rc;
   return collect_queries(c, si, res, st);
 }
@@ -1698,9 +1707,8 @@ int run_queries_at(cpx_ctx *c, std::vector<HostQuery> &hq, void *d_region, uint6
   HIPCHK(up(L.fin, pl.nfin * sizeof(BlockDesc)));
   HIPCHK(up(L.rowinfo, pl.nrows * sizeof(HardRowInfo)));
   const BatchDev b = batchdev_at(c, L, P0, O0);
-  const uint32_t nres_words = (uint32_t)(k.q * sizeof(ResultDev) / 4);
   for (int part = 0; part < 3; part++)
-    if ((rc = enqueue_part(c, b, part, nres_words))) return rc;
+    if ((rc = enqueue_part(c, b, part, &pl))) return rc;
   res.resize(hq.size());
   HIPCHK(hipMemcpyAsync(res.data(), O0 + L.results, hq.size() * sizeof(ResultDev), hipMemcpyDeviceToHost,
                         c->stream));

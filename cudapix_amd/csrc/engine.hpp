@@ -58,7 +58,8 @@ struct BatchSlot {
   void *d_plan = nullptr;           // plan arena (device)
   void *h_plan = nullptr;           // its pinned staging copy
   void *d_out = nullptr;            // counters, partial sums and results (device)
-  void *h_res = nullptr;            // pinned results
+  void *h_res = nullptr;            // pinned results, written by the combine kernel
+  ResultDev *d_res = nullptr;       // their device address
   Caps caps{};
   Layout L{};
   uint64_t arena_gen = 0;           // bumps when the arena is reallocated
@@ -130,8 +131,9 @@ int ensure_tables(cpx_ctx *c, uint64_t R, uint64_t P, uint64_t Y);
 // waiting (CPX_ESTATE when every slot holds an uncollected batch);
 // collect_queries waits for a slot's batch and frees the slot; run_queries
 // does both.
+// timed: record the events that collect_queries' statistics read.
 int submit_queries(cpx_ctx *c, const std::vector<HostQuery> &hq, uint32_t mask, uint32_t p2mode,
-                   bool use_graph, uint32_t *slot);
+                   bool use_graph, uint32_t *slot, bool timed = true);
 int collect_queries(cpx_ctx *c, uint32_t slot, std::vector<ResultDev> &res, cpx_batch_stats *st);
 int run_queries(cpx_ctx *c, const std::vector<HostQuery> &hq, uint32_t mask, uint32_t p2mode,
                 std::vector<ResultDev> &res, cpx_batch_stats *st, bool use_graph);

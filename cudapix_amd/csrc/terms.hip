@@ -22,85 +22,65 @@ hipError_t launch_zero_u32(uint32_t *p, size_t n, hipStream_t s)
   return hipGetLastError();
 }
 
-// --------------------------------------------------------------- setup
-// Block per query: pi(sqrt x), pi(p2_e), and the stage table
-// {p_b, floor(x / p_b)} with the emulated 128/64 divide.
+// ------------------------------------------- setup, ordinary, trivial
+// One query's record: pi(sqrt x), pi(p2_e), its result cleared, and the
+// stage table {p_b, floor(x / p_b)} with the emulated 128/64 divide.
+static __device__ __forceinline__ void setup_query(const BatchDev &bd, uint32_t qi)
+{
+  QueryDev &q = bd.queries[qi];
+  const u128 x = ((u128)q.x_hi << 64) | q.x_lo;
+  if (threadIdx.x == 0) {
+    q.pi_sqrtx = pi_lookup(bd.pitab, q.sqrtx);
+    q.pi_e = pi_lookup(bd.pitab, q.p2_e);
+    bd.results[qi].status = 0;
+  }
+  for (uint32_t s = threadIdx.x; s < q.nstage; s += blockDim.x) {
+    uint32_t p = bd.primes[q.cs + s];
+    StageDev d;
+    d.p = p;
+    d.ylo = (uint32_t)(q.y / p);
+    d.inv_p = 1.0 / (double)p;
+    d.magic = ~0ull / p + 1;
+    uint64_t rem;
+    const u128 xq = cpx_div128_64(x, p, &rem);
+    d.xp = (uint64_t)xq;
+    d.xph = (uint32_t)(xq >> 64);
+    d.pad = 0;
+    d.xp3 = ~0ull;
+    if (q.omega && (uint64_t)p * p > q.y) {
+      uint64_t r3;
+      const u128 t = cpx_div128_64(xq, (uint64_t)p * p, &r3);
+      d.xp3 = t < (u128)q.y ? (uint64_t)t : q.y;
+    }
+    bd.stages[q.stage_off + s] = d;
+  }
+}
+
+// What a solve needs before its segment kernel, in one launch (five small
+// launches of 2-20 us each, one after the other, were a tenth of a solve at
+// 1e12): S0 (ordinary_part, cpx_terms.hpp), the hard leaves of the wheel
+// stages (direct_part) and U (trivial_part), one descriptor per block
+// iteration, and the queries' records.
 __global__ __launch_bounds__(256) void k_setup(BatchDev bd)
 {
-  const uint32_t nq = *bd.nqueries;
-  for (uint32_t qi = blockIdx.x; qi < nq; qi += gridDim.x) {
-    QueryDev &q = bd.queries[qi];
-    const u128 x = ((u128)q.x_hi << 64) | q.x_lo;
-    if (threadIdx.x == 0) {
-      q.pi_sqrtx = pi_lookup(bd.pitab, q.sqrtx);
-      q.pi_e = pi_lookup(bd.pitab, q.p2_e);
+  __shared__ i128 red[4];
+  const uint32_t n0 = *bd.n_ord, n1 = n0 + *bd.n_dir, n2 = n1 + *bd.n_triv, n3 = n2 + *bd.nqueries;
+  for (uint32_t i = blockIdx.x; i < n3; i += gridDim.x) {
+    if (i >= n2) {
+      setup_query(bd, i - n2);
+      continue;
     }
-    for (uint32_t s = threadIdx.x; s < q.nstage; s += blockDim.x) {
-      uint32_t p = bd.primes[q.cs + s];
-      StageDev d;
-      d.p = p;
-      d.ylo = (uint32_t)(q.y / p);
-      d.inv_p = 1.0 / (double)p;
-      d.magic = ~0ull / p + 1;
-      uint64_t rem;
-      const u128 xq = cpx_div128_64(x, p, &rem);
-      d.xp = (uint64_t)xq;
-      d.xph = (uint32_t)(xq >> 64);
-      d.pad = 0;
-      d.xp3 = ~0ull;
-      if (q.omega && (uint64_t)p * p > q.y) {
-        uint64_t r3;
-        const u128 t = cpx_div128_64(xq, (uint64_t)p * p, &r3);
-        d.xp3 = t < (u128)q.y ? (uint64_t)t : q.y;
-      }
-      bd.stages[q.stage_off + s] = d;
-    }
+    const BlockDesc d = i < n0 ? bd.ord_desc[i] : i < n1 ? bd.dir_desc[i - n0] : bd.triv_desc[i - n1];
+    const i128 v = i < n0 ? ordinary_part<256>(bd, d, threadIdx.x)
+                   : i < n1 ? direct_part<256>(bd, d, threadIdx.x) : trivial_part<256>(bd, d, threadIdx.x);
+    const i128 t = block_sum_i128(v, red);
+    if (threadIdx.x == 0) bd.parts[bd.queries[d.query].part_off + d.part] = t;
   }
 }
 
 hipError_t launch_setup(BatchDev b, uint32_t grid, uint32_t, hipStream_t s)
 {
   hipLaunchKernelGGL(k_setup, dim3(grid), dim3(256), 0, s, b);
-  return hipGetLastError();
-}
-
-// ----------------------------------------------------------- ordinary
-// S0 (ordinary_part, cpx_terms.hpp) and the hard leaves of the wheel stages
-// (direct_part), one descriptor per block iteration.
-__global__ __launch_bounds__(256) void k_ordinary(BatchDev bd)
-{
-  __shared__ i128 red[4];
-  const uint32_t no = *bd.n_ord, nd = no + *bd.n_dir;
-  for (uint32_t di = blockIdx.x; di < nd; di += gridDim.x) {
-    const BlockDesc d = di < no ? bd.ord_desc[di] : bd.dir_desc[di - no];
-    const i128 v = di < no ? ordinary_part<256>(bd, d, threadIdx.x) : direct_part<256>(bd, d, threadIdx.x);
-    i128 t = block_sum_i128(v, red);
-    if (threadIdx.x == 0) bd.parts[bd.queries[d.query].part_off + d.part] = t;
-  }
-}
-
-hipError_t launch_ordinary(BatchDev b, uint32_t grid, hipStream_t s)
-{
-  hipLaunchKernelGGL(k_ordinary, dim3(grid), dim3(256), 0, s, b);
-  return hipGetLastError();
-}
-
-// ------------------------------------------------------------ trivial U
-// U (trivial_part, cpx_terms.hpp), one descriptor per block iteration.
-__global__ __launch_bounds__(256) void k_trivial(BatchDev bd)
-{
-  __shared__ i128 red[4];
-  const uint32_t nd = *bd.n_triv;
-  for (uint32_t di = blockIdx.x; di < nd; di += gridDim.x) {
-    const BlockDesc d = bd.triv_desc[di];
-    i128 t = block_sum_i128(trivial_part<256>(bd, d, threadIdx.x), red);
-    if (threadIdx.x == 0) bd.parts[bd.queries[d.query].part_off + d.part] = t;
-  }
-}
-
-hipError_t launch_trivial(BatchDev b, uint32_t grid, hipStream_t s)
-{
-  hipLaunchKernelGGL(k_trivial, dim3(grid), dim3(256), 0, s, b);
   return hipGetLastError();
 }
 
