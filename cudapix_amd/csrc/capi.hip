@@ -405,14 +405,17 @@ int cpx_count_primes(cpx_ctx *c, uint64_t lo, uint64_t hi, uint64_t *out)
       uint64_t r = cpx_isqrt128((u128)hi) + 1;
       if ((rc = ensure_tables(c, r, r, 64))) break;
       hipError_t e = launch_zero_u32((uint32_t *)d, 2, c->stream);
-      if (!e) e = launch_count_primes_sieve(lo, hi, c->primes.p, (uint32_t)c->nprimes, d, c->stream);
+      const WheelInfo &wi = c->h_winfo[8];
+      if (!e) e = launch_count_primes_sieve(lo, hi, c->primes.p, (uint32_t)c->nprimes,
+                                            (const uint32_t *)(c->wheel.p + wi.pat_off), wi.pat_period, d, c->stream);
       if (e) { rc = hip_fail(c, e, "count_primes_sieve"); break; }
     }
     hipError_t e = hipMemcpyAsync(&h, d, sizeof(h), hipMemcpyDeviceToHost, c->stream);
     if (!e) e = hipStreamSynchronize(c->stream);
     if (e) { rc = hip_fail(c, e, "count copy"); break; }
-    // the sieve counts odd primes >= 3; add the prime 2
-    if (!from_table && lo <= 2 && hi > 2) h += 1;
+    // the sieve counts the primes above 19; add those of its wheel
+    if (!from_table)
+      for (uint64_t p : {2, 3, 5, 7, 11, 13, 17, 19}) h += lo <= p && p < hi;
   } while (0);
   (void)hipFree(d);
   if (!rc) *out = h;

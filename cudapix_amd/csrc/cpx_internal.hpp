@@ -265,8 +265,9 @@ hipError_t launch_phi_count(const int32_t *mlpf, uint64_t lo_idx, uint64_t hi_id
                             uint32_t pa, unsigned long long *out, hipStream_t s);
 hipError_t launch_count_range(const PiEntry *tab, uint64_t lo, uint64_t hi,
                               unsigned long long *out, hipStream_t s);
-hipError_t launch_count_primes_sieve(uint64_t lo, uint64_t hi, const uint32_t *sprimes,
-                                     uint32_t nsp, unsigned long long *out, hipStream_t s);
+hipError_t launch_count_primes_sieve(uint64_t lo, uint64_t hi, const uint32_t *sprimes, uint32_t nsp,
+                                     const uint32_t *pat, uint32_t period, unsigned long long *out,
+                                     hipStream_t s);
 hipError_t launch_div_x_by_y(uint64_t x_lo, uint64_t x_hi, uint64_t *d_y, size_t len,
                              hipStream_t s);
 

@@ -111,55 +111,6 @@ struct SegShared {
 #define HARD_RECOUNT_P 128
 #endif
 
-// Residues coprime to 30 as a bit mask.
-#define COP30 0x208A2882u
-
-// Integers 0 <= j <= d coprime to 30.
-__device__ __forceinline__ uint32_t cop30_upto(uint32_t d)
-{
-  const uint32_t q = d / 30u, r = d - 30u * q;
-  return 8 * q + cpx_popc32(COP30 & ((2u << r) - 1u));
-}
-
-// The residue coprime to 30 of class i (0..7): one byte each.
-__device__ __forceinline__ uint32_t cop30_residue(uint32_t i)
-{
-  return (uint32_t)(0x1d1713110d0b0701ull >> (8 * i)) & 255u;
-}
-
-// A lane's class constants for crossing off: the multiples p k of a prime p =
-// 30 a + b with k = r (mod 30), r the residue of lane & 7, are the bits
-//   8 (a r + floor(b r / 30)) + index(b r mod 30) + 8 p u,  u = 0, 1, ...
-// counted from 0; eb holds the part that depends on b, one byte per class of b.
-struct CrossLane {
-  uint32_t r8;          // 8 r
-  uint64_t eb;
-  __device__ __forceinline__ explicit CrossLane(uint32_t lane)
-  {
-    const uint32_t r = cop30_residue(lane & 7u);
-    r8 = 8 * r;
-    eb = 0;
-#pragma unroll
-    for (uint32_t i = 0; i < 8; i++) {
-      const uint32_t br = cop30_residue(i) * r, q = br / 30u, m = br - 30u * q;
-      eb |= (uint64_t)(8 * q + cpx_popc32(COP30 & ((1u << m) - 1u))) << (8 * i);
-    }
-  }
-  // first bit at or above zero of this lane's class, with d8 = 8 (base mod p)
-  // for a window that starts at the integer 30 base; pb8 = 8 class(p mod 30)
-  __device__ __forceinline__ uint32_t first(uint32_t a, uint32_t pb8, uint32_t p8, uint32_t d8) const
-  {
-    const uint32_t j = a * r8 + ((uint32_t)(eb >> pb8) & 255u) - d8;   // in (-8p, 8p)
-    return min(j, j + p8);
-  }
-};
-// 8 * (class of p mod 30), for p coprime to 30.
-__device__ __forceinline__ uint32_t cop30_class8(uint32_t p)
-{
-  const uint32_t b = p % 30u;
-  return 8 * cpx_popc32(COP30 & ((1u << b) - 1u));
-}
-
 // Word of bit j of a bitmap in padded units.
 __device__ __forceinline__ uint32_t unit_word(uint32_t j) { return (j >> 5) + (j >> 10); }
 

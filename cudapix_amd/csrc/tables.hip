@@ -498,54 +498,145 @@ hipError_t launch_count_range(const PiEntry *tab, uint64_t lo, uint64_t hi,
   return hipGetLastError();
 }
 
-// Plain segmented-Eratosthenes count of the primes in [lo, hi) (the
+// Plain segmented-Eratosthenes count of the primes in [lo, hi) above 19 (the
 // CudaSieve::countPrimes replacement; also the brute-force check of pi(x)).
-// Segment k covers integers [base + k*2*SB, ...), base = lo & ~1.
-template <int T, int K>
-__global__ __launch_bounds__(T) void k_count_sieve(uint64_t lo, uint64_t hi,
-                                                   const uint32_t *__restrict__ sp, uint32_t nsp,
-                                                   unsigned long long *out)
+// Block b sieves `words` words of the integers coprime to 30 (120 integers a
+// word, layout as the segment sieve's) from start + 120 words b, start a
+// multiple of 120 at or below lo: the wheel pattern without the multiples of
+// 7 .. 19, then every prime from 23 up,
+//   below 1024     by every wave in its own part of the bitmap, eight classes
+//                  of multiples by eight in step;
+//   below 16384    by one wave over the whole bitmap;
+//   below 2^18     by one lane, class after class;
+//   above          by one lane, multiple after multiple (at most 15 of them,
+//                  of which those coprime to 30 are crossed).
+// Bound by the work per (prime, segment) once the primes outnumber the
+// segment's integers (664,000 of them at 1e14): hence one block of 1024
+// threads per CU with all of its LDS, 4.9e6 integers.  2^32 integers at 1e14:
+// 12.1 -> 3.2 ms, against 2^19 odd bits per block and a 64-bit remainder per
+// prime (1e15: 50 -> 8.8 ms for 6e9 integers, 4.5 -> 1.6 ms for 1e6).
+#define CS_T 1024
+#define CS_WORDS 40960u
+__global__ __launch_bounds__(CS_T) void k_count_sieve(uint64_t lo, uint64_t hi, uint64_t start, uint32_t words,
+                                                      const uint32_t *__restrict__ sp, uint32_t nsp,
+                                                      const uint32_t *__restrict__ pat, uint32_t period,
+                                                      unsigned long long *out)
 {
   extern __shared__ uint32_t lds[];
-  const uint32_t t = threadIdx.x;
-  const uint64_t SB = 32ull * K * T;
-  const uint64_t base = lo & ~1ull;
-  const uint64_t s0 = base + (uint64_t)blockIdx.x * 2 * SB;
-  for (uint32_t g = t; g < (uint32_t)(K * T); g += T) lds[seg_addr(g, K, T)] = 0xffffffffu;
-  __syncthreads();
-  seg_cross_primes(lds, K, T, s0, SB, sp, 1, nsp);
-  __syncthreads();
-  // count bits whose integer is an odd prime in [max(lo, 3), hi)
-  unsigned long long c = 0;
-  for (uint32_t j = 0; j < (uint32_t)K; j++) {
-    uint32_t w = lds[own_addr(t, j, K)];
-    uint64_t g = (uint64_t)t * K + j;
-    uint64_t n0 = s0 + 64 * g + 1;                 // integer of bit 0 of this word
-    if (n0 + 62 < lo || n0 >= hi) continue;
-    if (n0 < lo || n0 + 62 >= hi || n0 < 3) {
-      for (int i = 0; i < 32; i++) {
-        uint64_t n = n0 + 2 * i;
-        if (((w >> i) & 1u) && n >= lo && n < hi && n >= 3) c++;
-      }
-    } else {
-      c += cpx_popc32(w);
+  constexpr uint32_t NW = CS_T / CPX_WAVE, P0 = 8;      // sp[8] = 23
+  const uint32_t t = threadIdx.x, lane = lane_id();
+  const uint32_t wv = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_id());
+  const uint64_t base = start + (uint64_t)blockIdx.x * words * 120, end = base + (uint64_t)words * 120;
+  const uint64_t b30 = base / 30;
+  const bool small = end < (1ull << 58);
+  const uint32_t nbits = 32 * words;
+  {
+    const uint32_t step = CS_T % period;
+    uint32_t idx = (uint32_t)((base / 120 + t) % period);
+#pragma unroll 4
+    for (uint32_t w = t; w < words; w += CS_T) {
+      lds[w] = pat[idx];
+      idx += step;
+      if (idx >= period) idx -= period;
     }
   }
+  __syncthreads();
+  const CrossLane cl(lane);
+  // bits [j0, j1) of the multiples of p by this wave; b = the bitmap's start / 30 + j0 / 8
+  auto cross = [&](uint32_t p, uint32_t j0, uint32_t j1, uint64_t b, uint64_t d) {
+    const uint32_t p8 = 8 * p, p64 = 64 * p;
+    uint32_t j = j0 + cl.first(p / 30u, cop30_class8(p), p8, 8 * (uint32_t)d) + (lane >> 3) * p8;
+    if (lane == 0 && p >= 30 * b) j += p64;             // p itself
+    for (; j < j1; j += p64) atomicAnd(&lds[j >> 5], ~(1u << (j & 31u)));
+  };
+  uint32_t k = P0;
+  {
+    const uint32_t part = (words + NW - 1) / NW * 32;   // bits of a wave's part
+    const uint32_t j0 = min(nbits, wv * part), j1 = min(nbits, j0 + part);
+    const uint64_t b = b30 + j0 / 8;
+    for (; k < nsp; k++) {
+      const uint32_t p = sp[k];
+      if (p >= 1024 || (uint64_t)p * p >= end) break;
+      // (b / p < 2^50 below 2^58: the reciprocal divide)
+      cross(p, j0, j1, b, small ? b - cpx_div_leaf(b, (double)b, p) * p : b % p);
+    }
+  }
+  __syncthreads();
+  uint32_t kk = k + wv;
+  for (; kk < nsp; kk += NW) {
+    const uint32_t p = sp[kk];
+    if (p >= 16384 || (uint64_t)p * p >= end) break;
+    cross(p, 0, nbits, b30, b30 - cpx_div_leaf(b30, (double)b30, p) * p);
+  }
+  const double bf = (double)base, b30f = (double)b30;
+  uint32_t pn = k + t < nsp ? sp[k + t] : ~0u;          // the lane's next prime, loaded ahead
+  for (kk = k + t; kk < nsp; kk += CS_T) {
+    const uint32_t p = pn;
+    pn = kk + CS_T < nsp ? sp[kk + CS_T] : ~0u;
+    if ((uint64_t)p * p >= end) break;
+    if (p < 16384) continue;
+    if (p < (1u << 18)) {
+      const uint32_t p8 = 8 * p, a = p / 30u, pr = p - 30u * a;
+      const uint32_t d8 = 8 * (uint32_t)(b30 - cpx_div_leaf(b30, b30f, p) * p);
+#pragma unroll
+      for (uint32_t i = 0; i < 8; i++) {
+        const uint32_t r = cop30_residue(i), br = pr * r, q = br / 30u, m = br - 30u * q;
+        uint32_t j = 8 * (a * r + q) + cpx_popc32(COP30 & ((1u << m) - 1u)) - d8;
+        j = min(j, j + p8);
+        if (i == 0 && p >= base) j += p8;               // p itself
+        for (; j < nbits; j += p8) atomicAnd(&lds[j >> 5], ~(1u << (j & 31u)));
+      }
+    } else {
+      // the multiples p m at or above base (base / p < 2^50: base < 2^64, p >= 2^18), m >= 2
+      uint64_t q = cpx_div_leaf(base, bf, p);
+      uint64_t off = base - q * p;
+      if (off) { q++; off = p - off; }
+      if (q < 2) { off += (2 - q) * p; q = 2; }
+      if (off >= 120ull * words) continue;
+      uint32_t m = ((uint32_t)(q >> 32) * 16u + (uint32_t)q % 30u) % 30u;   // 2^32 = 16 (mod 30)
+      for (; off < 120ull * words; off += p, m = m == 29 ? 0u : m + 1) {
+        if (!((COP30 >> m) & 1u)) continue;
+        const uint32_t d = (uint32_t)off, dq = d / 30u;
+        const uint32_t j = 8 * dq + cpx_popc32(COP30 & ((1u << (d - 30u * dq)) - 1u));
+        atomicAnd(&lds[j >> 5], ~(1u << (j & 31u)));
+      }
+    }
+  }
+  __syncthreads();
+  // count the bits whose integer lies in [max(lo, 2), hi)
+  unsigned long long c = 0;
+  const uint64_t from = max(lo, (uint64_t)2);
+  for (uint32_t w = t; w < words; w += CS_T) {
+    const uint64_t n0 = base + 120ull * w;
+    uint32_t b = lds[w];
+    if (n0 >= hi || n0 + 120 <= from) continue;
+    if (n0 < from) b &= ~cpx_lowmask32(cop30_upto((uint32_t)(from - n0) - 1));
+    if (n0 + 120 > hi) b &= cpx_lowmask32(cop30_upto((uint32_t)(hi - n0) - 1));
+    c += cpx_popc32(b);
+  }
   c = wave_sum(c);
-  if (lane_id() == 0) atomicAdd(out, c);
+  if (lane == 0) atomicAdd(out, c);
 }
 
-hipError_t launch_count_primes_sieve(uint64_t lo, uint64_t hi, const uint32_t *sprimes,
-                                     uint32_t nsp, unsigned long long *out, hipStream_t s)
+// pat, period: the segment pattern of the wheel of eight primes.
+hipError_t launch_count_primes_sieve(uint64_t lo, uint64_t hi, const uint32_t *sprimes, uint32_t nsp,
+                                     const uint32_t *pat, uint32_t period, unsigned long long *out,
+                                     hipStream_t s)
 {
   if (hi <= lo) return hipSuccess;
-  constexpr int T = 256, K = 64;                   // 2^19 odd bits per segment
-  const uint64_t SB = 32ull * K * T;
-  uint64_t base = lo & ~1ull;
-  uint64_t nseg = (hi - base + 2 * SB - 1) / (2 * SB);
+  const uint64_t start = lo / 120 * 120;
+  const uint64_t nw = (hi - start + 119) / 120;
+  // equal segments, a multiple of 256 of them once there are that many
+  uint64_t nseg = (nw + CS_WORDS - 1) / CS_WORDS;
+  if (nseg > 256) nseg = (nseg + 255) / 256 * 256;
   if (nseg > 0x7fffffffull) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((k_count_sieve<T, K>), dim3((uint32_t)nseg), dim3(T), (size_t)(K + 1) * T * 4, s,
-                     lo, hi, sprimes, nsp, out);
+  const uint32_t words = (uint32_t)((nw + nseg - 1) / nseg);
+  nseg = (nw + words - 1) / words;
+  const hipError_t e = hipFuncSetAttribute((const void *)k_count_sieve,
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, CS_WORDS * 4);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(k_count_sieve, dim3((uint32_t)nseg), dim3(CS_T), (size_t)words * 4, s, lo, hi, start,
+                     words, sprimes, nsp, pat, period, out);
   return hipGetLastError();
 }
 
