@@ -202,6 +202,26 @@ __device__ __forceinline__ uint32_t cop30_residue(uint32_t i)
   return (uint32_t)(0x1d1713110d0b0701ull >> (8 * i)) & 255u;
 }
 
+// e[i] byte k: 8 floor(r_i r_k / 30) + index(r_i r_k mod 30), for the residues
+// r coprime to 30 (symmetric in i and k).
+struct Cop30Products {
+  uint64_t e[8];
+};
+constexpr Cop30Products make_cop30_products()
+{
+  const uint32_t r[8] = {1, 7, 11, 13, 17, 19, 23, 29};
+  Cop30Products t{};
+  for (int i = 0; i < 8; i++)
+    for (int k = 0; k < 8; k++) {
+      const uint32_t q = r[i] * r[k] / 30, m = r[i] * r[k] % 30;
+      uint64_t n = 0;
+      for (int l = 0; l < 8; l++) n += r[l] < m;
+      t.e[i] |= (8 * q + n) << (8 * k);
+    }
+  return t;
+}
+static __device__ const Cop30Products cop30_products = make_cop30_products();
+
 // A lane's class constants for crossing off: the multiples p k of a prime p =
 // 30 a + b with k = r (mod 30), r the residue of lane & 7, are the bits
 //   8 (a r + floor(b r / 30)) + index(b r mod 30) + 8 p u,  u = 0, 1, ...
@@ -211,20 +231,14 @@ struct CrossLane {
   uint64_t eb;
   __device__ __forceinline__ explicit CrossLane(uint32_t lane)
   {
-    const uint32_t r = cop30_residue(lane & 7u);
-    r8 = 8 * r;
-    eb = 0;
-#pragma unroll
-    for (uint32_t i = 0; i < 8; i++) {
-      const uint32_t br = cop30_residue(i) * r, q = br / 30u, m = br - 30u * q;
-      eb |= (uint64_t)(8 * q + cpx_popc32(COP30 & ((1u << m) - 1u))) << (8 * i);
-    }
+    r8 = 8 * cop30_residue(lane & 7u);
+    eb = cop30_products.e[lane & 7u];
   }
   // first bit at or above zero of this lane's class, with d8 = 8 (base mod p)
   // for a window that starts at the integer 30 base; pb8 = 8 class(p mod 30)
   __device__ __forceinline__ uint32_t first(uint32_t a, uint32_t pb8, uint32_t p8, uint32_t d8) const
   {
-    const uint32_t j = a * r8 + ((uint32_t)(eb >> pb8) & 255u) - d8;   // in (-8p, 8p)
+    const uint32_t j = __umul24(a, r8) + ((uint32_t)(eb >> pb8) & 255u) - d8;   // in (-8p, 8p)
     return min(j, j + p8);
   }
 };

@@ -283,7 +283,6 @@ hipError_t launch_combine(BatchDev b, uint32_t maxq, hipStream_t s);
 // segsieve.hip
 hipError_t launch_segments(BatchDev b, SegShape shape, uint32_t grid, hipStream_t s);
 hipError_t launch_selftest_wave(const uint32_t *in, uint32_t n, uint32_t *bad, hipStream_t s);
-size_t seg_lds_bytes(SegShape shape);
 bool seg_shape_supported(SegShape shape);
 hipError_t launch_scan_entries(PiEntry *tab, uint64_t nent, uint32_t *tot, uint64_t *base,
                                hipStream_t s);

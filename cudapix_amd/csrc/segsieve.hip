@@ -4,11 +4,11 @@
 #include "segtiles.hpp"
 
 template <int T, int K>
-// (at least 4 waves per SIMD: two 512-thread blocks per CU need <= 128 VGPRs)
-__global__ __launch_bounds__(T, 4) void k_segments(BatchDev bd)
+__global__ __launch_bounds__(T, (SegLds<T, K>::waves())) void k_segments(BatchDev bd)
 {
-  extern __shared__ uint32_t lds[];
-  __shared__ SegShared<T, K> sh;
+  __shared__ SegLds<T, K> mem;
+  SegShared<T, K> &sh = mem.sh;
+  uint32_t *const lds = mem.bits;
   const uint32_t ntiles = *bd.ntiles;
   for (;;) {
     if (threadIdx.x == 0) sh.tile = atomicAdd(bd.tile_head, 1u);
@@ -22,9 +22,6 @@ __global__ __launch_bounds__(T, 4) void k_segments(BatchDev bd)
     __syncthreads();
   }
 }
-
-// Units of 1024 bits with one padding word each.
-size_t seg_lds_bytes(SegShape shape) { return (size_t)(shape.seg_bits() / 1024) * 33 * 4; }
 
 // One-wavefront workgroups (T = 64) make every block barrier a single-wave
 // barrier and let ~15 independent segment workers share a CU.
@@ -42,13 +39,10 @@ bool seg_shape_supported(SegShape s)
 
 int seg_blocks_per_cu(SegShape shape)
 {
-  size_t lds = seg_lds_bytes(shape);
   int nb = 0;
 #define X(TT, KK)                                                                            \
   if (shape.threads == TT && shape.kwords == KK) {                                           \
-    (void)hipFuncSetAttribute((const void *)k_segments<TT, KK>,                              \
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);         \
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_segments<TT, KK>, TT, lds) !=   \
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_segments<TT, KK>, TT, 0) !=     \
         hipSuccess)                                                                          \
       nb = 0;                                                                                \
   }
@@ -59,11 +53,9 @@ int seg_blocks_per_cu(SegShape shape)
 
 hipError_t launch_segments(BatchDev b, SegShape shape, uint32_t grid, hipStream_t s)
 {
-  size_t lds = seg_lds_bytes(shape);
 #define X(TT, KK)                                                                            \
   if (shape.threads == TT && shape.kwords == KK) {                                           \
-    /* the >64 KiB LDS attribute is set by seg_blocks_per_cu before any launch */           \
-    hipLaunchKernelGGL((k_segments<TT, KK>), dim3(grid), dim3(TT), lds, s, b);               \
+    hipLaunchKernelGGL((k_segments<TT, KK>), dim3(grid), dim3(TT), 0, s, b);                 \
     return hipGetLastError();                                                                \
   }
   CPX_SEG_SHAPES(X)

@@ -74,11 +74,11 @@ struct SegShared {
   static constexpr uint32_t NW = T / CPX_WAVE, NU = T * (K / 32);
   // items of a chunk: as many as the LDS left by two blocks per CU holds
   static constexpr uint32_t NI = NW >= 8 ? 96 : 128;
-  // survivors of each unit's two halves (low and high 16 bits), kept in the
-  // stages that count their removals one by one
+  // survivors of each unit's four quarters, a byte each (a quarter's 256 bits
+  // lose at least the multiples of 7 and 11), kept in the stages that count
+  // their removals one by one and published at a stage with leaves
   uint32_t cnt[NU];
-  // published at a stage with leaves: the unit's in-wave exclusive prefix (18
-  // bits) and the count of its first half (above)
+  // published at a stage with leaves: the unit's in-wave exclusive prefix
   uint32_t ipre[NU];
   long long acc[NW][CPX_GROUP];  // sum of mu * phi by wave and member
   GroupMember gm[CPX_GROUP];
@@ -101,65 +101,83 @@ struct SegShared {
   uint32_t tile;
 };
 
+// A block's LDS, one object at a fixed address, so that the bitmap's and the
+// tables' addresses are instruction offsets: units of 32 words and one of padding.
+template <int T, int K>
+struct SegLds {
+  SegShared<T, K> sh;
+  __attribute__((aligned(16))) uint32_t bits[SegShared<T, K>::NU * 33];
+  // waves per SIMD that a CU's LDS holds: the register budget (4 for 512 threads x 32 words)
+  static constexpr int waves()
+  {
+    return 163840 / (int)sizeof(SegLds) * (T / CPX_WAVE) / 4 > 0 ? 163840 / (int)sizeof(SegLds) * (T / CPX_WAVE) / 4 : 1;
+  }
+};
+
 #define HARD_NC_MASK 0x7fffffffu
 #define HARD_SPARSE 0x80000000u    // p^2 > y: candidates are primes
-#define HARD_PRE_BITS 18
 // Stages with p below this cross without returns and recount the wave's
 // bits afterwards (a popcount per word of the thread); above, each removal
-// is taken off its half unit's count.  Steps of a wave per stage: 1024/p.
+// is taken off its quarter's count.  Steps of a wave per stage: 1024/p.
 #ifndef HARD_RECOUNT_P
 #define HARD_RECOUNT_P 128
 #endif
 
-// Word of bit j of a bitmap in padded units.
-__device__ __forceinline__ uint32_t unit_word(uint32_t j) { return (j >> 5) + (j >> 10); }
-
-// Survivors of the two halves of a unit, packed low | high << 16.
-__device__ __forceinline__ uint32_t unit_counts(const uint32_t *w)
+// Word of bit j of a bitmap in padded units.  (One shift-add forms the byte
+// offset; the compiler's own form takes two shifts, two masks and an add.)
+__device__ __forceinline__ uint32_t *unit_word(uint32_t *bits, uint32_t j)
 {
-  uint32_t lo = 0, hi = 0;
-#pragma unroll
-  for (uint32_t j = 0; j < 16; j++) lo += cpx_popc32(w[j]);
-#pragma unroll
-  for (uint32_t j = 16; j < 32; j++) hi += cpx_popc32(w[j]);
-  return lo | (hi << 16);
+  const uint32_t w = j >> 5, u = j >> 10;
+  uint32_t o;
+  asm("v_add_lshl_u32 %0, %1, %2, 2" : "=v"(o) : "v"(w), "v"(u));
+  return (uint32_t *)((char *)bits + o);
 }
 
-// Publish the wave's prefix counts from its threads' packed unit counts.
+// Survivors of the four quarters of a unit, a byte each.
+__device__ __forceinline__ uint32_t unit_counts(const uint32_t *w)
+{
+  uint32_t q[4] = {0, 0, 0, 0};
+#pragma unroll
+  for (uint32_t j = 0; j < 32; j++) q[j >> 3] += cpx_popc32(w[j]);
+  return q[0] | q[1] << 8 | q[2] << 16 | q[3] << 24;
+}
+__device__ __forceinline__ uint32_t unit_total(uint32_t c) { return __builtin_amdgcn_sad_u8(c, 0u, 0u); }
+
+// Publish the wave's prefix counts from its threads' unit counts.
 template <int UPT>
 __device__ __forceinline__ uint32_t publish_units(const uint32_t (&c)[UPT], uint32_t *ipre)
 {
   uint32_t s = 0;
 #pragma unroll
-  for (int u = 0; u < UPT; u++) s += (c[u] & 0xffffu) + (c[u] >> 16);
+  for (int u = 0; u < UPT; u++) s = __builtin_amdgcn_sad_u8(c[u], 0u, s);
   const uint32_t incl = wave_incl_scan(s);
   uint32_t ex = incl - s;
 #pragma unroll
   for (int u = 0; u < UPT; u++) {
-    ipre[threadIdx.x * UPT + u] = ex | (c[u] << HARD_PRE_BITS);   // (the high half's bits shift out)
-    ex += (c[u] & 0xffffu) + (c[u] >> 16);
+    ipre[threadIdx.x * UPT + u] = ex;
+    ex = __builtin_amdgcn_sad_u8(c[u], 0u, ex);
   }
   return (uint32_t)__builtin_amdgcn_readlane((int)incl, CPX_WAVE - 1);
 }
 
-// Survivors below bit jb (0 .. 1024) of a unit, plus its published prefix.
-// The 16 words of the bit's half, the published word and the partial word are
-// loaded before any is used, so the count costs one LDS round trip; words at
-// or above the bit are masked out.  (At jb = 1024 the partial word is the
-// unit's padding word, masked to nothing.)
-__device__ __forceinline__ uint32_t unit_count_below(const uint32_t *w, uint32_t e, uint32_t jb)
+// Survivors at or below bit g of the units from `bits`, of which ipre and cnt
+// hold the published prefixes and quarter counts.  The quarter's eight words,
+// the published words and the bit's own word are loaded before any is used, so
+// the count costs one LDS round trip; words at or above the bit's are masked out.
+__device__ __forceinline__ uint32_t unit_count_to(const uint32_t *bits, const uint32_t *ipre, const uint32_t *cnt,
+                                                  uint32_t g)
 {
-  const bool upper = jb >= 512;
-  const uint32_t *ow = w + (upper ? 16u : 0u);
-  const uint32_t nf = (jb >> 5) - (upper ? 16u : 0u);   // whole words below the bit: 0 .. 16
-  uint32_t wd[16];
+  const uint32_t u = g >> 10, nf = (g >> 5) & 7u;
+  const uint32_t *w = bits + ((g >> 5) & ~7u) + u;
+  uint32_t wd[8];
 #pragma unroll
-  for (uint32_t r = 0; r < 16; r++) wd[r] = ow[r];
-  const uint32_t part = ow[nf];
-  uint32_t c = (e & ((1u << HARD_PRE_BITS) - 1u)) + (upper ? e >> HARD_PRE_BITS : 0u);
+  for (uint32_t r = 0; r < 8; r++) wd[r] = w[r];
+  const uint32_t part = w[nf], pre = ipre[u], q = cnt[u];
+  const uint32_t full = (1u << nf) - 1u;
+  uint32_t c = __builtin_amdgcn_sad_u8(q & ((1u << ((g >> 5) & 24u)) - 1u), 0u, pre);
 #pragma unroll
-  for (uint32_t r = 0; r < 16; r++) c += cpx_popc32(r < nf ? wd[r] : 0u);
-  return c + cpx_popc32(part & cpx_lowmask32(jb & 31u));
+  for (uint32_t r = 0; r < 8; r++) c += cpx_popc32(wd[r] & (uint32_t)__builtin_amdgcn_sbfe((int)full, r, 1u));
+  return c + cpx_popc32(part & ((2u << (g & 31u)) - 1u));
 }
 
 // Number of table entries m <= M: primes (sparse) or leaf-table m's.
@@ -359,7 +377,7 @@ __device__ __forceinline__ void p2_cross_wave(uint32_t *lds, uint32_t p, uint64_
   const uint32_t d8 = 8 * (uint32_t)(base - cpx_div_leaf(base, (double)base, p) * p);
   uint32_t j = cl.first(p / 30u, cop30_class8(p), p8, d8) + (lane >> 3) * p8;
   if (base == 0 && lane == 0) j += p64;                 // p itself
-  for (; j < SB; j += p64) atomicAnd(&lds[unit_word(j)], ~(1u << (j & 31u)));
+  for (; j < SB; j += p64) atomicAnd(unit_word(lds, j), ~(1u << (j & 31u)));
 }
 
 // P2 leaves of a segment (replaces the windowed upper_bound count of
@@ -400,22 +418,23 @@ __device__ __forceinline__ void p2_epilogue(const BatchDev &bd, const GroupDev &
     const uint32_t p = sp[k];
     if ((uint64_t)p * p >= hi) break;
     if (p < P2_WAVE_P) continue;
-    const uint32_t p8 = 8 * p, a = p / 30u, b = p - 30u * a;
+    const uint32_t p8 = 8 * p, a = p / 30u;
     const uint32_t d8 = 8 * (uint32_t)(base - cpx_div_leaf(base, (double)base, p) * p);
+    // (the table is symmetric: the lane constants of p's own class are its bytes by class of multiple)
+    const uint64_t eb = cop30_products.e[cop30_class8(p) >> 3];
 #pragma unroll
     for (uint32_t i = 0; i < 8; i++) {
-      const uint32_t r = cop30_residue(i), br = b * r, q = br / 30u, m = br - 30u * q;
-      uint32_t j = 8 * (a * r + q) + cpx_popc32(COP30 & ((1u << m) - 1u)) - d8;
+      uint32_t j = a * (8 * cop30_residue(i)) + ((uint32_t)(eb >> (8 * i)) & 255u) - d8;
       j = min(j, j + p8);
       if (i == 0 && base == 0) j += p8;                 // p itself
-      for (; j < SB; j += p8) atomicAnd(&lds[unit_word(j)], ~(1u << (j & 31u)));   // SB + 8p < 2^32
+      for (; j < SB; j += p8) atomicAnd(unit_word(lds, j), ~(1u << (j & 31u)));   // SB + 8p < 2^32
     }
   }
   __syncthreads();
   {
     uint32_t c[UPT];
 #pragma unroll
-    for (uint32_t u = 0; u < UPT; u++) c[u] = unit_counts(lds + (t * UPT + u) * 33);
+    for (uint32_t u = 0; u < UPT; u++) c[u] = sh.cnt[t * UPT + u] = unit_counts(lds + (t * UPT + u) * 33);
     const uint32_t ws = publish_units<(int)UPT>(c, sh.ipre);
     if (lane == 0) sh.wtot[wv] = ws;
   }
@@ -425,12 +444,11 @@ __device__ __forceinline__ void p2_epilogue(const BatchDev &bd, const GroupDev &
   for (uint32_t w = 0; w < NW; w++) { wp[w] = tot; tot += sh.wtot[w]; }
   // survivors at or below n (lo <= n < hi)
   auto count_to = [&](uint64_t n) {
-    const uint32_t bit = cop30_upto((uint32_t)(n - lo));
-    const uint32_t u = min(bit >> 10, SegShared<T, K>::NU - 1);
+    const uint32_t bits = cop30_upto((uint32_t)(n - lo)), b = max(bits, 1u) - 1, wave = (b >> 10) / WU;
     uint32_t pre = 0;
 #pragma unroll
-    for (uint32_t w = 0; w < NW; w++) pre = u / WU == w ? wp[w] : pre;
-    return pre + unit_count_below(lds + u * 33, sh.ipre[u], bit - u * 1024);
+    for (uint32_t w = 0; w < NW; w++) pre = wave == w ? wp[w] : pre;
+    return bits ? pre + unit_count_to(lds, sh.ipre, sh.cnt, b) : 0u;
   };
   for (uint32_t g = 0; g < grp.n; g++) {
     if (!(sh.gm[g].on & 2u)) continue;
@@ -502,11 +520,15 @@ __device__ __forceinline__ void p2_epilogue(const BatchDev &bd, const GroupDev &
 // crossing its own bits instead, one multiple or none each, a stage cost the
 // wave about 50 instructions to find the lanes' first multiples.)
 //
-// Bound by VALU issue and the latency of a wave's chain of stages, not by the
-// bits: what counts is instructions per (wave, stage).  Against odd-only bits,
-// own-bits crossing, candidates from every odd m and groups of 8, on MI355X:
-// 512 queries to 1e15 64.2 -> 35.5 ms for two batches, 1e16 7.7 -> 5.4 ms,
-// 1e18 153 -> 97 ms, 2e19 1215 -> 802 ms.
+// Bound by VALU issue: at x = 1e17 the SIMDs have a VALU instruction in flight
+// 87 % of the time (7.5e9 of them in 14.6 ms, 4 cycles each), so what counts is
+// instructions per (wave, stage).  Against odd-only bits, own-bits crossing,
+// candidates from every odd m and groups of 8, the layout above took two
+// 512-query batches to 1e15 from 64.2 to 35.5 ms, 1e16 from 7.7 to 5.4 ms, 1e18
+// from 153 to 97 ms.  First multiples of eight stages at a time, four stages'
+// operations in flight, removals taken off byte counters and one LDS object at a
+// fixed address took a stage of a prime above 1024 from 35 to 20 VALU
+// instructions: 1e16 4.36 -> 4.05 ms, 1e18 79.2 -> 68.4 ms, 1e12 431 -> 402 us.
 template <int T, int K, int GS>
 __device__ __forceinline__ void hard_chunks(const BatchDev &bd, SegShared<T, K> &sh, uint32_t *lds,
                                             uint32_t cs, uint32_t nst, uint32_t rep, uint32_t cstep,
@@ -521,8 +543,7 @@ __device__ __forceinline__ void hard_chunks(const BatchDev &bd, SegShared<T, K> 
   const double inv_lo_w = lo_w ? 1.0 / (double)lo_w : 0.0, inv_hi_w = 1.0 / (double)hi_w;
   const double inv_lo = lo ? 1.0 / (double)lo : 0.0, inv_hi = 1.0 / (double)hi;
   const uint64_t base_w = lo_w / 30;
-  uint32_t *const wl = lds + wv * WU * 33;              // the wave's bits
-  uint32_t *const wc = sh.cnt + wv * WU;                // ... its units' counts
+  const uint32_t wbit = wv * WB;                        // the wave's bits start here
   const CrossLane cl(lane);
 
   // survivors: the thread's units, the wave, the segment
@@ -531,7 +552,7 @@ __device__ __forceinline__ void hard_chunks(const BatchDev &bd, SegShared<T, K> 
 #pragma unroll
   for (uint32_t u = 0; u < UPT; u++) {
     cr[u] = unit_counts(lds + (t * UPT + u) * 33);
-    wcur += (cr[u] & 0xffffu) + (cr[u] >> 16);
+    wcur += unit_total(cr[u]);
   }
   wcur = wave_sum(wcur);
   if (lane == 0) sh.wsum[wv] = (int32_t)wcur;
@@ -544,11 +565,12 @@ __device__ __forceinline__ void hard_chunks(const BatchDev &bd, SegShared<T, K> 
   for (uint32_t s0 = 0; s0 < nst;) {
     const uint32_t se = min(SST, nst - s0);
     // stage constants, stage k in lane k: p, 8 (base mod p), p / 30 and the class of p
+    // (p < 2^21: the pi table's reach bounds x^(1/4))
     const uint32_t pk = bd.primes[cs + s0 + min(lane, se - 1)];
     uint32_t ni;
     const uint32_t n = hard_items<T, K, GS>(bd, sh, s0, se, lo, hi, inv_lo, inv_hi, &ni);
     const uint32_t d8k = 8 * (uint32_t)(base_w - cpx_div_leaf(base_w, (double)base_w, pk) * pk);
-    const uint32_t ak = pk / 30u, ck = cop30_class8(pk);
+    const uint32_t ack = pk / 30u << 6 | cop30_class8(pk);
     const uint32_t istk = sh.ist[lane];
     if (lane == 0) sh.c0[wv] = wcur;
     // the wave's candidates [ia, ia + in) of the items lane and lane + 64
@@ -645,8 +667,48 @@ __device__ __forceinline__ void hard_chunks(const BatchDev &bd, SegShared<T, K> 
     };
     prepare();
 
-    for (uint32_t k = 0; k < n; k++) {
+    uint32_t dwk = 0;                                   // the wave's removals of stage k, in lane k
+    auto removed = [&](uint32_t k, uint32_t wd) {
+      wcur -= wd;
+      dwk = lane == k ? wd : dwk;
+    };
+    // first multiples as bits of the segment, class by class: of the eight
+    // stages from 8 fg (fj) and from 8 fg + 8 (fn), stage (lane >> 3), class lane & 7
+    uint32_t fg = 0, fj, fn;
+    auto firsts = [&](uint32_t g) {
+      const uint32_t st = 8 * g + (lane >> 3), ac = lane_get(ack, st);
+      return cl.first(ac >> 6, ac & 63u, 8 * lane_get(pk, st), lane_get(d8k, st)) + wbit;
+    };
+    fj = firsts(0);
+    fn = firsts(1);
+    // this lane's first multiple of the primes of stages k, k + 1, .. (at most eight)
+    auto first_of = [&](uint32_t k, uint32_t count, uint32_t *j) {
+      while (k >> 3 > fg) {
+        fg++;
+        fj = fn;
+        fn = firsts(fg + 1);
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < count; u++)
+        j[u] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(4 * (lane & 7u) + 32 * ((k + u) & 7u)),
+                                                      (int)((k + u) >> 3 > fg ? fn : fj));
+#pragma unroll
+      for (uint32_t u = 0; u < count; u++) j[u] += __umul24(lane >> 3, 8 * lane_read(pk, k + u));
+    };
+    // one multiple j: whether its bit (m) was still set, taken off its quarter's count
+    auto hit = [&](uint32_t j, uint32_t m, uint32_t old) {
+      const bool h = (old & m) != 0;
+      const uint64_t all = __builtin_amdgcn_ballot_w64(h);
+      if (h) atomicSub(&sh.cnt[j >> 10], 1u << ((j >> 5) & 24u));
+      return all;
+    };
+    for (uint32_t k = 0; k < n;) {
       const uint32_t p = lane_read(pk, k);
+      if (!counted && p >= HARD_RECOUNT_P) {            // from here on removals are counted one by one
+#pragma unroll
+        for (uint32_t u = 0; u < UPT; u++) sh.cnt[t * UPT + u] = cr[u];
+        counted = true;
+      }
       if (k == nk) {
         // ---- leaves of p whose n falls in this wave's bits (state: crossed
         //      by p_1 .. p_{b-1}), all members' in one list; the wave
@@ -654,9 +716,10 @@ __device__ __forceinline__ void hard_chunks(const BatchDev &bd, SegShared<T, K> 
         int64_t as = 0;                                 // this item lane's sums (GS > 1)
         int32_t ws = 0;                                 // sum of mu: the item lane's, or the wave's (GS = 1)
         if (ntot > rep * CPX_WAVE) {
-          if (counted) {
 #pragma unroll
-            for (uint32_t u = 0; u < UPT; u++) cr[u] = sh.cnt[t * UPT + u];
+          for (uint32_t u = 0; u < UPT; u++) {
+            if (counted) cr[u] = sh.cnt[t * UPT + u];
+            else sh.cnt[t * UPT + u] = cr[u];
           }
           (void)publish_units<(int)UPT>(cr, sh.ipre);
           for (uint32_t fb = rep * CPX_WAVE; fb < ntot; fb += cstep) {   // every lane runs every window
@@ -677,9 +740,9 @@ __device__ __forceinline__ void hard_chunks(const BatchDev &bd, SegShared<T, K> 
                 const uint64_t xp = sh.xp[fi];
                 const double xpf = (double)xp + (double)sh.xph[fi] * 0x1p64;
                 const uint64_t nn = cpx_div_leaf(xp, xpf, (uint32_t)pf.x);   // lo_w <= nn < hi_w
-                const uint32_t bit = cop30_upto((uint32_t)nn - (uint32_t)lo_w);
-                const uint32_t u = min(bit >> 10, WU - 1);
-                const int32_t cn = (int32_t)unit_count_below(wl + u * 33, sh.ipre[wv * WU + u], bit - u * 1024);
+                const uint32_t bits = cop30_upto((uint32_t)nn - (uint32_t)lo_w);   // 0 .. WB
+                const uint32_t ct = unit_count_to(lds, sh.ipre, sh.cnt, max(bits, 1u) - 1 + wbit);
+                const int32_t cn = bits ? (int32_t)ct : 0;
                 val = sg > 0 ? cn : -cn;
               }
             }
@@ -700,61 +763,81 @@ __device__ __forceinline__ void hard_chunks(const BatchDev &bd, SegShared<T, K> 
         }
         prepare();
       }
-      // ---- cross off the multiples of p in the wave's bits
-      {
-        const uint32_t p8 = 8 * p, p64 = 64 * p;
-        uint32_t j = cl.first(lane_read(ak, k), lane_read(ck, k), p8, lane_read(d8k, k)) + (lane >> 3) * p8;
-        uint32_t wd;
-        if (p < HARD_RECOUNT_P) {
-          for (; j + 3 * p64 < WB; j += 4 * p64) {
-            const uint32_t j1 = j + p64, j2 = j1 + p64, j3 = j2 + p64;
-            atomicAnd(&wl[unit_word(j)], ~(1u << (j & 31u)));
-            atomicAnd(&wl[unit_word(j1)], ~(1u << (j1 & 31u)));
-            atomicAnd(&wl[unit_word(j2)], ~(1u << (j2 & 31u)));
-            atomicAnd(&wl[unit_word(j3)], ~(1u << (j3 & 31u)));
-          }
-          for (; j < WB; j += p64) atomicAnd(&wl[unit_word(j)], ~(1u << (j & 31u)));
-          uint32_t s = 0;
+      // ---- cross off the multiples of p in the wave's bits, and of the
+      //      stages after it that have no leaves here: with at most one multiple
+      //      per lane four stages go together, the LDS taking the wave's
+      //      operations in order, so that their round trips overlap
+      const uint32_t kend = min(nk, n);                 // (> k)
+      const uint32_t jend = wbit + WB;
+      if (64 * p >= WB) {
+        for (; k + 3 < kend; k += 4) {
+          uint32_t j[4], m[4], old[4];
+          first_of(k, 4, j);
 #pragma unroll
-          for (uint32_t u = 0; u < UPT; u++) {
-            cr[u] = unit_counts(lds + (t * UPT + u) * 33);
-            s += (cr[u] & 0xffffu) + (cr[u] >> 16);
+          for (uint32_t u = 0; u < 4; u++) {
+            m[u] = 1u << (j[u] & 31u);
+            old[u] = 0;
+            if (j[u] < jend) old[u] = atomicAnd(unit_word(lds, j[u]), ~m[u]);
           }
-          s = wave_sum(s);
-          wd = wcur - s;
-        } else {
-          if (!counted) {                               // from here on removals are counted one by one
+          // the four stages' removals (below 2^16) to lanes k .. k + 3
+          uint64_t wd4 = 0;
 #pragma unroll
-            for (uint32_t u = 0; u < UPT; u++) sh.cnt[t * UPT + u] = cr[u];
-            counted = true;
+          for (uint32_t u = 0; u < 4; u++) {
+            const uint32_t wd = (uint32_t)__popcll(hit(j[u], m[u], old[u]));
+            wcur -= wd;
+            wd4 |= (uint64_t)wd << (16 * u);
           }
-          // one multiple: whether its bit was still set
-          auto hit = [&](uint32_t jj, uint32_t old) {
-            const bool h = (old >> (jj & 31u)) & 1u;
-            if (h) atomicSub(&wc[jj >> 10], jj & 512u ? 0x10000u : 1u);
-            return h;
-          };
-          if (p64 >= WB) {                              // at most one multiple per lane
-            bool h = false;
-            if (j < WB) h = hit(j, atomicAnd(&wl[unit_word(j)], ~(1u << (j & 31u))));
-            wd = (uint32_t)__popcll(__ballot(h));
-          } else {
-            uint32_t d = 0;
-            for (; j + p64 < WB; j += 2 * p64) {
-              const uint32_t j1 = j + p64;
-              const uint32_t o0 = atomicAnd(&wl[unit_word(j)], ~(1u << (j & 31u)));
-              const uint32_t o1 = atomicAnd(&wl[unit_word(j1)], ~(1u << (j1 & 31u)));
-              d += hit(j, o0) ? 1u : 0u;
-              d += hit(j1, o1) ? 1u : 0u;
-            }
-            if (j < WB) d += hit(j, atomicAnd(&wl[unit_word(j)], ~(1u << (j & 31u)))) ? 1u : 0u;
-            wd = wave_sum(d);
-          }
+          const uint32_t to = lane - k;
+          dwk = to < 4 ? (uint32_t)(wd4 >> (16 * to)) & 0xffffu : dwk;
         }
-        wcur -= wd;
-        if (lane == 0) sh.dw[k][wv] = (uint16_t)wd;     // this wave's removals
+        for (; k < kend; k++) {
+          uint32_t j, old = 0;
+          first_of(k, 1, &j);
+          const uint32_t m = 1u << (j & 31u);
+          if (j < jend) old = atomicAnd(unit_word(lds, j), ~m);
+          removed(k, (uint32_t)__popcll(hit(j, m, old)));
+        }
+        continue;
       }
+      const uint32_t p64 = 64 * p;                      // (64 p bits: whole words, so a lane keeps its bit)
+      uint32_t j, wd;
+      first_of(k, 1, &j);
+      const uint32_t m = 1u << (j & 31u);
+      if (p < HARD_RECOUNT_P) {
+        const uint32_t p2 = 2 * p, we = jend >> 5;
+        uint32_t w = j >> 5;
+        for (; w + 3 * p2 < we; w += 4 * p2) {
+          const uint32_t w1 = w + p2, w2 = w1 + p2, w3 = w2 + p2;
+          atomicAnd(&lds[w + (w >> 5)], ~m);
+          atomicAnd(&lds[w1 + (w1 >> 5)], ~m);
+          atomicAnd(&lds[w2 + (w2 >> 5)], ~m);
+          atomicAnd(&lds[w3 + (w3 >> 5)], ~m);
+        }
+        for (; w < we; w += p2) atomicAnd(&lds[w + (w >> 5)], ~m);
+        uint32_t s = 0;
+#pragma unroll
+        for (uint32_t u = 0; u < UPT; u++) {
+          cr[u] = unit_counts(lds + (t * UPT + u) * 33);
+          s += unit_total(cr[u]);
+        }
+        wd = wcur - wave_sum(s);
+      } else {
+        // (every lane takes every step: the ballots count the removals)
+        wd = 0;
+        const uint32_t steps = (WB + p64 - 1) / p64;    // (first multiples are below 64 p)
+        for (uint32_t i = 0; i < steps; i += 2, j += 2 * p64) {
+          const uint32_t j1 = j + p64;
+          uint32_t o0 = 0, o1 = 0;
+          if (j < jend) o0 = atomicAnd(unit_word(lds, j), ~m);
+          if (j1 < jend) o1 = atomicAnd(unit_word(lds, j1), ~m);
+          wd += (uint32_t)__popcll(hit(j, m, o0));
+          wd += (uint32_t)__popcll(hit(j1, m, o1));
+        }
+      }
+      removed(k, wd);
+      k++;
     }
+    if (lane < n) sh.dw[lane][wv] = (uint16_t)dwk;
     hard_flush<T, K, GS>(bd, sh, s0, n, ni, kk, running, rep == 0, acc);
     s0 += n;
   }

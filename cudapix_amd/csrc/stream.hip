@@ -406,10 +406,11 @@ static __device__ __attribute__((noinline)) void stream_account(const StreamArgs
 }
 
 template <int T, int K>
-__global__ __launch_bounds__(T, 4) void k_stream(const StreamArgs a)
+__global__ __launch_bounds__(T, (SegLds<T, K>::waves())) void k_stream(const StreamArgs a)
 {
-  extern __shared__ uint32_t lds[];
-  __shared__ SegShared<T, K> sh;
+  __shared__ SegLds<T, K> mem;
+  SegShared<T, K> &sh = mem.sh;
+  uint32_t *const lds = mem.bits;
   __shared__ StreamWork w;
   uint64_t idle_since = wall_clock64();
   uint32_t backoff = 1;
@@ -514,13 +515,10 @@ bool stream_shape_supported(SegShape s)
 
 int stream_blocks_per_cu(SegShape shape)
 {
-  size_t lds = seg_lds_bytes(shape);
   int nb = 0;
 #define X(TT, KK)                                                                            \
   if (shape.threads == TT && shape.kwords == KK) {                                           \
-    (void)hipFuncSetAttribute((const void *)k_stream<TT, KK>,                                \
-                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);         \
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_stream<TT, KK>, TT, lds) !=     \
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_stream<TT, KK>, TT, 0) !=       \
         hipSuccess)                                                                          \
       nb = 0;                                                                                \
   }
@@ -531,10 +529,9 @@ int stream_blocks_per_cu(SegShape shape)
 
 hipError_t launch_stream(const StreamArgs &a, SegShape shape, uint32_t grid, hipStream_t s)
 {
-  size_t lds = seg_lds_bytes(shape);
 #define X(TT, KK)                                                                            \
   if (shape.threads == TT && shape.kwords == KK) {                                           \
-    hipLaunchKernelGGL((k_stream<TT, KK>), dim3(grid), dim3(TT), lds, s, a);                 \
+    hipLaunchKernelGGL((k_stream<TT, KK>), dim3(grid), dim3(TT), 0, s, a);                   \
     return hipGetLastError();                                                                \
   }
   CPX_STREAM_SHAPES(X)
