@@ -65,7 +65,7 @@ struct QueryDev {
   uint32_t nstage;        // B - cs: the sieved ones
   uint32_t a;             // pi(y)
   uint32_t pi_cbrt, pi_qrt, pi_sqrtz, small;   // small: answered by one pi-table lookup
-  uint64_t hard_nseg, hard_row0;      // hard segments and first output row (T, bact, rowinfo)
+  uint64_t hard_nseg, hard_row0;      // hard segments and first output row (T, rowinfo)
   uint64_t m_off;                     // first element of this query in hard_M
   uint64_t mrow_base, hard_nmrow;     // first M-row (acc slot) and M-row count (>= segments)
   uint64_t p2_nseg, p2_row0;          // segments holding P2 leaves and their first output row
@@ -176,10 +176,10 @@ struct HardRowInfo {
   uint64_t moff;
 };
 
-// Hard-leaf stages per carry block (k_hard_fin): a row's T and sum(mu) of
-// consecutive stages are adjacent, so a block that takes several stages
-// reads them from the same cache lines.
-#define CPX_FIN_STAGES 8
+// Hard-leaf stages per carry block (k_hard_fin), one column of its threads
+// each: a row's T and sum(mu) of consecutive stages are adjacent, so 16 of them
+// are one 64-byte access.
+#define CPX_FIN_STAGES 16
 
 // Block descriptor of the grid-stride term kernels (ordinary, trivial, easy).
 struct BlockDesc {
@@ -214,14 +214,13 @@ struct BatchDev {
   BlockDesc *ord_desc;   uint32_t *n_ord;
   BlockDesc *triv_desc;  uint32_t *n_triv;
   BlockDesc *easy_desc;  uint32_t *n_easy;
-  BlockDesc *fin_desc;   uint32_t *n_fin;     // hard carry blocks (begin = the stage)
+  BlockDesc *fin_desc;   uint32_t *n_fin;     // hard carry blocks (begin = stage | rows << 32)
   BlockDesc *p2_desc;    uint32_t *n_p2;      // P2 lookups (prime index ranges)
   BlockDesc *dir_desc;   uint32_t *n_dir;     // hard leaves of the wheel stages (odd m)
   HardRowInfo *rowinfo;                       // [row]
   // outputs
   uint32_t *hard_T;                           // per row, active stages: survivors before stage
   int32_t *hard_M;                            // per mrow, active stages: sum of mu of the leaves
-  uint32_t *hard_bact;                        // [row]   active stages
   int64_t *hard_acc;                          // [mrow]  sum of mu * local phi
   uint32_t *p2_cnt;      uint32_t *p2_np;     uint64_t *p2_loc;   // [row]
   i128 *parts;           // partial sums

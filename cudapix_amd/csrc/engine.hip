@@ -663,6 +663,7 @@ static void plan_query(const cpx_ctx *c, const HostQuery &h, uint32_t i, uint32_
   for (size_t k = 0; k < qp.fin.size(); k++) {
     while (r > 0 && qp.rowinfo[r - 1].act <= qp.fin[k].begin) r--;
     qp.fin_rows[k] = (uint32_t)r;
+    qp.fin[k].begin |= r << 32;                        // rows the block walks
   }
 }
 
@@ -1002,7 +1003,6 @@ static Layout make_layout(const Caps &k)
   o = 0;
   L.hard_T = o;    o = al(o + k.tm * 4);
   L.hard_M = o;    o = al(o + k.mm * 4);
-  L.hard_bact = o; o = al(o + k.rows * 4);
   L.hard_acc = o;  o = al(o + k.mrows * 8);
   L.hard_base = o; o = al(o + k.base * 8);
   L.p2_cnt = o;    o = al(o + k.p2rows * 4);
@@ -1146,7 +1146,6 @@ static BatchDev batchdev_at(const cpx_ctx *c, const Layout &L, char *P, char *O)
   b.rowinfo = (HardRowInfo *)(P + L.rowinfo);
   b.hard_T = (uint32_t *)(O + L.hard_T);
   b.hard_M = (int32_t *)(O + L.hard_M);
-  b.hard_bact = (uint32_t *)(O + L.hard_bact);
   b.hard_acc = (int64_t *)(O + L.hard_acc);
   b.hard_base = nullptr;                 // (a run in passes points it at L.hard_base)
   b.pass_r0 = 0; b.pass_r1 = ~0ull; b.pass_toff = 0; b.pass_moff = 0; b.pass_add = 0; b.pass_pad = 0;
@@ -1300,9 +1299,9 @@ static int seg_grid(cpx_ctx *c)
 }
 
 static const uint32_t GRID_Q = 256, GRID_T = 2048;
-// carry kernel: 128-thread blocks whose time is a latency chain, so many of
-// them in flight (extra blocks of a small batch exit at once)
-static const uint32_t GRID_FIN = 16384;
+// carry kernel: blocks whose time is a latency chain, so many of them in
+// flight (extra blocks of a small batch exit at once)
+static const uint32_t GRID_FIN = 4096;
 
 // The launch sequence in three parts; events between the parts time the
 // persistent segment kernel on its own stream (also when replayed as graphs).
@@ -1376,8 +1375,8 @@ uint64_t plan_bytes_estimate(const cpx_ctx *c, const HostQuery &h)
     r = r1;
   }
   // T and M per pair (M rows of replicated segments add some: a group's
-  // leaf-dense segments give every member the group's replicas), rowinfo,
-  // bact and the P2 rows, stage and carry descriptors, easy descriptors
+  // leaf-dense segments give every member the group's replicas), rowinfo and
+  // the P2 rows, stage and carry descriptors, easy descriptors
   // easy-leaf descriptors (with a part and a tile each): a few per EASY_MIN
   // pairs up to about EASY_TILES each for V and the hard leaves, then per EASY_WORK
   const double cb = (double)h.cbrtx + 3, fy = (double)h.y + 3;

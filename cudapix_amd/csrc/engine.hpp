@@ -45,7 +45,7 @@ struct Caps {
 
 struct Layout {
   size_t counters, queries, stages, tiles, groups, ord, triv, easy, fin, p2d, dir, rowinfo, plan_bytes;
-  size_t hard_T, hard_M, hard_bact, hard_acc, hard_base, p2_cnt, p2_np, p2_loc, parts, results, out_bytes;
+  size_t hard_T, hard_M, hard_acc, hard_base, p2_cnt, p2_np, p2_loc, parts, results, out_bytes;
 };
 
 // Batch slots per context: one batch can be planned and uploaded while the

@@ -913,7 +913,6 @@ __device__ __forceinline__ void hard_segment(const BatchDev &bd, const TileDev &
     long long tt = 0;
     for (uint32_t w = 0; w < NW; w++) tt += sh.acc[w][g];
     st_out(&bd.hard_acc[q.mrow_base + bd.rowinfo[row].mrow + rep], (int64_t)tt);
-    if (rep == 0) st_out(&bd.hard_bact[row], sh.gm[g].nst);
   }
   if (rep == 0 && p2any) p2_epilogue<T, K>(bd, grp, seg, lo, cs + nst, lds, sh);
 }

@@ -85,9 +85,8 @@ hipError_t launch_setup(BatchDev b, uint32_t grid, uint32_t, hipStream_t s)
 }
 
 // -------------------------------------------------------- hard carry
-// hard_fin_desc (cpx_terms.hpp) per carry descriptor: 128-thread blocks,
-// whose time is a latency chain over the segment chunks, so many in flight.
-#define FIN_T 128          // carry-block threads: segments per chunk
+// hard_fin_desc (cpx_terms.hpp) per carry descriptor.
+#define FIN_T 512
 __global__ __launch_bounds__(FIN_T) void k_hard_fin(BatchDev bd)
 {
   __shared__ FinShared<FIN_T> fs;

@@ -58,3 +58,15 @@ def test_shapes_term_by_term(ctx, shape):
         for t, u in zip(c.pi_batch(xs, terms=True), want):
             _same(t, u, shape)
         _same(c.pi(10 ** 16, terms=True), ctx.pi(10 ** 16, terms=True), shape)
+
+
+# the hard carry takes a stage's rows in 32 runs, four rows of a run at a time: numbers of
+# segments on both sides of one row a run, four rows a run and their remainders (y on both
+# sides of the least it can be, so that the numbers of stages differ)
+@pytest.mark.parametrize("nseg", [1, 2, 4, 31, 32, 33, 63, 65, 127, 128, 129, 133])
+@pytest.mark.parametrize("extra", [2, 301])
+def test_carry_runs(ctx, oracle, nseg, extra):
+    z = SEG * nseg - 7
+    y = max(int(z ** 0.5) + extra, 100)
+    x = y * z + 3
+    _same(ctx.pi(x, y=y, terms=True), oracle.pi_dr(x, y, 6), (x, y))
