@@ -181,6 +181,13 @@ struct HardRowInfo {
 // are one 64-byte access.
 #define CPX_FIN_STAGES 16
 
+// A segment's P2 primes are shared among its replicas when they span more than
+// this many pi-table entries a thread (every sharing replica sieves the
+// segment's primes for itself); otherwise replica 0 counts them all.
+#ifndef CPX_P2_SHARE
+#define CPX_P2_SHARE 8
+#endif
+
 // Block descriptor of the grid-stride term kernels (ordinary, trivial, easy).
 struct BlockDesc {
   uint32_t query;
@@ -222,7 +229,8 @@ struct BatchDev {
   uint32_t *hard_T;                           // per row, active stages: survivors before stage
   int32_t *hard_M;                            // per mrow, active stages: sum of mu of the leaves
   int64_t *hard_acc;                          // [mrow]  sum of mu * local phi
-  uint32_t *p2_cnt;      uint32_t *p2_np;     uint64_t *p2_loc;   // [row]
+  uint32_t *p2_cnt;                           // [P2 row] primes of the segment
+  uint32_t *p2_np;       uint64_t *p2_loc;    // [mrow]   P2 primes counted by the replica, sum of their counts
   i128 *parts;           // partial sums
   ResultDev *results;
   // one query's hard segments in passes over segment ranges (its rows of

@@ -189,7 +189,8 @@ __device__ __forceinline__ void hard_fin_desc(const BatchDev &bd, const BlockDes
 // the record (the streaming path has no setup kernel).
 template <uint32_t NT>
 struct CombShared {
-  i128 red[NT / CPX_WAVE];
+  i128 red[5][NT / CPX_WAVE];
+  i128 sum[5];
   uint64_t wtot[NT / CPX_WAVE];
 };
 
@@ -218,34 +219,52 @@ __device__ __forceinline__ void combine_query(const BatchDev &bd, uint32_t qi, C
   const QueryDev &q = bd.queries[qi];
   const uint64_t pi_e = table_pi ? pi_lookup(bd.pitab, q.p2_e) : q.pi_e;
   const uint64_t pi_sqrtx = table_pi ? pi_lookup(bd.pitab, q.sqrtx) : q.pi_sqrtx;
-  // P2: sum over segments of loc + np * (pi(p2_e) + primes in earlier segments)
+  // P2: sum over segments of loc + np * (pi(p2_e) + primes in earlier segments),
+  // a run of consecutive segments a thread, then the runs' totals.  (A latency
+  // chain: four rows in flight.  At 1e18, one row a thread and a scan for every
+  // 256 rows, each a chain of its own, took 430 us.)
   i128 p2 = 0;
-  uint64_t base = pi_e;
-  for (uint64_t r0 = 0; r0 < q.p2_nseg; r0 += NT) {
-    uint64_t r = r0 + t;
-    uint64_t c = 0, np = 0, loc = 0;
-    if (r < q.p2_nseg) {
-      c = bd.p2_cnt[q.p2_row0 + r];
-      np = bd.p2_np[q.p2_row0 + r];
-      loc = bd.p2_loc[q.p2_row0 + r];
+  {
+    constexpr uint32_t U = 4;
+    const uint64_t per = (q.p2_nseg + NT - 1) / NT, ra = per * t, rb = min(ra + per, q.p2_nseg);
+    const HardRowInfo *__restrict__ info = bd.rowinfo + q.hard_row0 + q.p2_seg0;
+    const uint32_t *__restrict__ cnt = bd.p2_cnt + q.p2_row0, *__restrict__ nps = bd.p2_np + q.mrow_base;
+    const uint64_t *__restrict__ locs = bd.p2_loc + q.mrow_base;
+    uint64_t pre = 0, nsum = 0;
+    for (uint64_t r = ra; r < rb; r += U) {
+      uint32_t mr[U], nr[U];
+      uint64_t c[U], np[U], loc[U];
+#pragma unroll
+      for (uint32_t u = 0; u < U; u++) {
+        const bool in = r + u < rb;
+        mr[u] = in ? info[r + u].mrow : 0u;
+        nr[u] = in ? info[r + u].nrep : 0u;
+        c[u] = in ? cnt[r + u] : 0u;
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < U; u++) {
+        np[u] = nr[u] ? nps[mr[u]] : 0u;
+        loc[u] = nr[u] ? locs[mr[u]] : 0ull;
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < U; u++) {
+        for (uint32_t k = 1; k < nr[u]; k++) { np[u] += nps[mr[u] + k]; loc[u] += locs[mr[u] + k]; }
+        p2 += (i128)loc[u] + (i128)np[u] * pre;
+        pre += c[u];
+        nsum += np[u];
+      }
     }
-    uint64_t incl = wave_incl_scan(c);
+    const uint64_t incl = wave_incl_scan(pre);
     if (lane_id() == CPX_WAVE - 1) cs.wtot[wave_id()] = incl;
     __syncthreads();
-    uint64_t pre = incl - c, tot = 0;
-    for (uint32_t w = 0; w < NT / CPX_WAVE; w++) {
-      tot += cs.wtot[w];
-      if (w < wave_id()) pre += cs.wtot[w];
-    }
-    p2 += (i128)loc + (i128)np * (i128)(base + pre);
-    base += tot;
-    __syncthreads();
+    uint64_t base = pi_e + incl - pre;
+    for (uint32_t w = 0; w < wave_id(); w++) base += cs.wtot[w];
+    p2 += (i128)nsum * base;
   }
   // hard: local sums
   i128 hacc = 0;
+#pragma unroll 4
   for (uint64_t r = t; r < q.hard_nmrow; r += NT) hacc += bd.hard_acc[q.mrow_base + r];
-  i128 p2s = block_sum_i128(p2, cs.red);
-  i128 hs = block_sum_i128(hacc, cs.red);
   if (t == 0 && q.small) {
     ResultDev res;
     i128 pi = (i128)pi_lookup(bd.pitab, q.x_lo);
@@ -261,11 +280,12 @@ __device__ __forceinline__ void combine_query(const BatchDev &bd, uint32_t qi, C
   }
   // the term partial sums, by term (ordinary | trivial U | easy | hard carry
   // | P2 lookups)
-  i128 ps0 = 0, psu = 0, psv = 0, psh = 0, psp = 0;
+  i128 ps0 = 0, psu = 0, psv = 0, psh = hacc, psp = p2;
   if (!q.small) {
     const i128 *pp = bd.parts + q.part_off;
     const uint32_t n0 = q.n_ord_parts, n1 = n0 + q.n_triv_parts, n2 = n1 + q.n_easy_parts,
                    n3 = n2 + q.n_hard_parts, n4 = n3 + q.n_p2_parts;
+#pragma unroll 2
     for (uint32_t i = t; i < n4; i += NT) {
       const i128 v = pp[i];
       if (i < n0) ps0 += v;
@@ -275,22 +295,31 @@ __device__ __forceinline__ void combine_query(const BatchDev &bd, uint32_t qi, C
       else psp += v;
     }
   }
-  psp = block_sum_i128(psp, cs.red);
-  ps0 = block_sum_i128(ps0, cs.red);
-  psu = block_sum_i128(psu, cs.red);
-  psv = block_sum_i128(psv, cs.red);
-  psh = block_sum_i128(psh, cs.red);
+  // the block's five sums behind one pair of barriers
+  const i128 part[5] = {ps0, psu, psv, psh, psp};
+#pragma unroll
+  for (uint32_t j = 0; j < 5; j++) {
+    const i128 s = wave_sum_i128(part[j]);
+    if (lane_id() == 0) cs.red[j][wave_id()] = s;
+  }
+  __syncthreads();
+  if (t < 5) {
+    i128 s = 0;
+    for (uint32_t w = 0; w < NT / CPX_WAVE; w++) s += cs.red[t][w];
+    cs.sum[t] = s;
+  }
+  __syncthreads();
   if (t == 0 && !q.small) {
-    const i128 s0 = ps0, u = psu, v = psv, hc = psh;
+    const i128 s0 = cs.sum[0], u = cs.sum[1], v = cs.sum[2];
     // S1 = C(pi(y) - pi(cbrt x), 2)
     i128 kk = (i128)q.a - (i128)q.pi_cbrt;
     i128 s1 = kk > 0 ? kk * (kk - 1) / 2 : 0;
     i128 triv = s1 + u;
-    i128 hard = -(hs + hc);
+    i128 hard = -cs.sum[3];
     // P2 = sum pi(x/p) - sum_{p} (pi(p) - 1), pi(p) = a+1 .. A
     i128 A = (i128)pi_sqrtx, a = (i128)q.a;
     i128 P2 = 0;
-    if (A > a) P2 = p2s + psp - (A * (A - 1) / 2 - a * (a - 1) / 2);
+    if (A > a) P2 = cs.sum[4] - (A * (A - 1) / 2 - a * (a - 1) / 2);
     i128 pi = s0 + triv + v + hard + a - 1 - P2;
     ResultDev res;
     put_i128(res.pi, pi);

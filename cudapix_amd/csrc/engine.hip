@@ -710,10 +710,20 @@ static void make_groups(const cpx_ctx *c, const std::vector<HostQuery> &hq,
 // full anyway.
 static const double STAGE_LEAVES = 143.0, REP_SIEVE = 16.0;
 
+// pi-table entries that hold a query's P2 primes of the segment [lo, hi), and
+// the leaf candidates that counting the primes of one costs as much as.
+static const double P2_LEAVES = 6.0;
+static double p2_entries(const QueryDev &d, double x, double lo, double hi)
+{
+  const double pmax = lo > 0 ? std::min((double)d.sqrtx, x / lo) : (double)d.sqrtx;
+  return std::max(0.0, pmax - std::max((double)d.y, x / hi)) / 64.0;
+}
+
 // Replicas, M rows and tiles of one group: a segment's replica count comes
 // from all members' leaves there; every member with the segment in its hard
 // range gets that many M rows.  Tile cost: the shared sieve once, each
-// member's leaves, and on replica 0 the P2 sieve and counts.
+// member's leaves, and on replica 0, or on all where they share them, the P2
+// sieve and counts.
 static void plan_group(const cpx_ctx *c, const GroupDev &g, uint32_t gi, std::vector<QPlan> &qps,
                        double block_work, GPlan &gp)
 {
@@ -724,19 +734,31 @@ static void plan_group(const cpx_ctx *c, const GroupDev &g, uint32_t gi, std::ve
   const uint32_t cw = qps[g.q[0]].d.cs;
   uint64_t mrows[CPX_GROUP] = {0}, moff[CPX_GROUP] = {0};
   uint64_t nsp_i = 0;                                  // pi(sqrt(hi)), grows with s
+  double xd[CPX_GROUP];
+  bool few[CPX_GROUP] = {false};       // P2 primes of the segment below one entry a thread (they fall with s)
+  for (uint32_t m = 0; m < g.n; m++) xd[m] = 0x1p64 * (double)qps[g.q[m]].d.x_hi + (double)qps[g.q[m]].d.x_lo;
   gp.tiles.reserve(nseg);
   gp.tbucket.reserve(nseg);
   for (uint64_t s = 0; s < nseg; s++) {
     const uint64_t hi = (s + 1) * c->shape.seg_ints();
-    double leaves = 0, lcost = 0;
+    double leaves = 0, lcost = 0, p2e = 0;
     uint32_t act = 0, np2 = 0;
     for (uint32_t m = 0; m < g.n; m++) {
       const QPlan &qp = qps[g.q[m]];
       if (s >= qp.d.hard_nseg) continue;
       leaves += qp.rleaves[s];
       act = std::max(act, qp.rowinfo[s].act);
-      if (s >= qp.d.p2_seg0 && s < qp.d.p2_seg0 + qp.d.p2_nseg) np2++;
+      if (s >= qp.d.p2_seg0 && s < qp.d.p2_seg0 + qp.d.p2_nseg) {
+        np2++;
+        if (!few[m]) {
+          const double e = p2_entries(qp.d, xd[m], (double)(hi - c->shape.seg_ints()), (double)hi);
+          few[m] = e < (double)T;
+          p2e += e;
+        }
+      }
     }
+    const bool share = p2e > (double)(CPX_P2_SHARE * T);
+    if (share) leaves += P2_LEAVES * p2e;
     const double most = std::max(524288.0, REP_SIEVE * STAGE_LEAVES * (double)act);
     const double per = std::max(16384.0, std::min(block_work, most));
     const uint32_t nrep = (uint32_t)std::min(64.0, std::max(1.0, std::ceil(leaves / per)));
@@ -753,7 +775,8 @@ static void plan_group(const cpx_ctx *c, const GroupDev &g, uint32_t gi, std::ve
     }
     const double cost = 1.0 + (double)act * (0.5 + 4.0 * SB / (64.0 * 1024.0 * T)) + lcost;
     // replica 0 of a segment of a P2 range also crosses the primes from
-    // p_(c+act+1) to sqrt(hi) and counts the P2 leaves there
+    // p_(c+act+1) to sqrt(hi) and counts the P2 leaves there; replicas that
+    // share the leaves all cross
     double p2cost = 0;
     if (np2) {
       const double sq = std::min(std::sqrt((double)hi), (double)c->prime_limit);
@@ -761,9 +784,10 @@ static void plan_group(const cpx_ctx *c, const GroupDev &g, uint32_t gi, std::ve
       const double nsp = (double)nsp_i - (double)(cw + act);
       p2cost = 2.0 * np2 + std::max(nsp, 0.0) * 8.0 / T;
     }
+    const double p2count = 2.0 * P2_LEAVES * p2e / T / (share ? nrep : 1);
     for (uint32_t r = 0; r < nrep; r++) {
       gp.tiles.push_back({gi, (uint16_t)nrep, (uint16_t)r, s});
-      gp.tbucket.push_back(cost_bucket(r == 0 ? cost + p2cost : cost));
+      gp.tbucket.push_back(cost_bucket(r == 0 || share ? cost + p2cost + p2count : cost));
     }
   }
   for (uint32_t m = 0; m < g.n; m++) {
@@ -899,6 +923,8 @@ static int build_plan(cpx_ctx *c, const std::vector<HostQuery> &hq, uint32_t mas
       if (qps[g.q[m]].tm > longest->tm) longest = &qps[g.q[m]];
     work += STAGE_LEAVES * (double)longest->tm;
   }
+  for (const QPlan &qp : qps)
+    if (qp.d.p2_nseg) work += P2_LEAVES * ((double)qp.d.sqrtx - (double)qp.d.y) / 64.0;
   const double block_work = 0.8 * work / 512.0;
   std::vector<GPlan> gps(pl.groups.size());
   parallel_for(pl.groups.size(), nt,
@@ -1006,8 +1032,8 @@ static Layout make_layout(const Caps &k)
   L.hard_acc = o;  o = al(o + k.mrows * 8);
   L.hard_base = o; o = al(o + k.base * 8);
   L.p2_cnt = o;    o = al(o + k.p2rows * 4);
-  L.p2_np = o;     o = al(o + k.p2rows * 4);
-  L.p2_loc = o;    o = al(o + k.p2rows * 8);
+  L.p2_np = o;     o = al(o + k.mrows * 4);
+  L.p2_loc = o;    o = al(o + k.mrows * 8);
   L.parts = o;     o = al(o + k.parts * sizeof(i128));
   L.results = o;   o = al(o + k.q * sizeof(ResultDev));
   L.out_bytes = o;

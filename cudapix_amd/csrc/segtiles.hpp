@@ -40,7 +40,7 @@
 //   src/sieve/S2_hard_device.cu:357-375).
 //
 // P2: the segments holding x/p for a member's P2 primes p in (y, sqrt x]
-// get, on replica 0 of their tile, the rest of a prime sieve (primes above
+// get, on replica 0 of their tile (on all of them where the primes are many), the rest of a prime sieve (primes above
 // the last stage up to sqrt(hi)) and each such member's P2 counts; see
 // p2_epilogue.
 #pragma once
@@ -49,6 +49,7 @@
 #ifndef P2_WAVE_P
 #define P2_WAVE_P 1024     // P2 sieve: primes below this are crossed by a whole wave
 #endif
+#define P2_U 4             // P2 primes of a lane in flight (1, 2 and 4 are even)
 static_assert(CPX_GROUP == 32, "member slots: 1, 8 or 32");
 
 // Stages of a chunk at most, by member slots (one item per thread is tested).
@@ -122,6 +123,16 @@ struct SegLds {
 #ifndef HARD_RECOUNT_P
 #define HARD_RECOUNT_P 128
 #endif
+
+// threadIdx.x, opaque: what one part of a tile derives from it is not kept in
+// registers through the others (20 -> 6 spilled registers in the 512-thread
+// kernel; two 512-query batches 30.8 -> 29.7 ms).
+__device__ __forceinline__ uint32_t own_thread()
+{
+  uint32_t t = threadIdx.x;
+  asm("" : "+v"(t));
+  return t;
+}
 
 // Word of bit j of a bitmap in padded units.  (One shift-add forms the byte
 // offset; the compiler's own form takes two shifts, two masks and an add.)
@@ -204,7 +215,8 @@ __device__ __forceinline__ uint32_t hard_items(const BatchDev &bd, SegShared<T, 
                                                double inv_hi, uint32_t *ni)
 {
   constexpr uint32_t NW = T / CPX_WAVE, NI = SegShared<T, K>::NI;
-  const uint32_t t = threadIdx.x, lane = lane_id(), wv = wave_id();
+  const uint32_t t = own_thread();
+  const uint32_t lane = t % CPX_WAVE, wv = t / CPX_WAVE;
   const uint32_t k = t / GS, g = t % GS;
   uint32_t nc = 0, cb = 0, xph = 0;
   uint64_t xp = 0;
@@ -367,21 +379,8 @@ __device__ __forceinline__ void hard_flush(const BatchDev &bd, SegShared<T, K> &
   __syncthreads();
 }
 
-// Cross the multiples of p (from its first multiple at or above the bitmap's
-// start; not p itself) out of the segment at lo, by one wave.
-template <int T>
-__device__ __forceinline__ void p2_cross_wave(uint32_t *lds, uint32_t p, uint64_t base, uint32_t SB,
-                                              const CrossLane &cl, uint32_t lane)
-{
-  const uint32_t p8 = 8 * p, p64 = 64 * p;
-  const uint32_t d8 = 8 * (uint32_t)(base - cpx_div_leaf(base, (double)base, p) * p);
-  uint32_t j = cl.first(p / 30u, cop30_class8(p), p8, d8) + (lane >> 3) * p8;
-  if (base == 0 && lane == 0) j += p64;                 // p itself
-  for (; j < SB; j += p64) atomicAnd(unit_word(lds, j), ~(1u << (j & 31u)));
-}
-
 // P2 leaves of a segment (replaces the windowed upper_bound count of
-// src/P2.cu:76-133), run by replica 0 of a hard tile after its stages: the
+// src/P2.cu:76-133), run by a hard tile after its stages: the
 // bitmap already holds [lo, hi) sieved by the wheel and by the stage primes
 // below primes[kfirst]; the primes from index kfirst with p^2 < hi are
 // crossed here, which leaves exactly the primes above the largest
@@ -390,27 +389,79 @@ __device__ __forceinline__ void p2_cross_wave(uint32_t *lds, uint32_t p, uint64_
 // (pi-table bits, block-strided), the count of primes in (p2_e, x/p] held in
 // this segment; per member and segment: primes in (p2_e, hi), number of p,
 // sum of the counts.  The carry is applied in the combine kernel.
+//
+// Replica 0 does this alone, or where the P2 primes are many (CPX_P2_SHARE) all
+// replicas do, each the sieve and its share of the primes.  The first segments
+// of a small x hold most of them: at 1e12 segment 0 counts 37 K, 74 us of one
+// block bound by VALU issue (about 100 instructions a count) while the others
+// are done.  Shared, pi(1e12) takes 325 us instead of 400, 1e13 with fresh tables
+// 735 instead of 820 (100 of it the table's); with the threshold at 2 to 8
+// entries a thread the same, at 32 or more nothing is shared at 1e12.
 template <int T, int K>
 __device__ __forceinline__ void p2_epilogue(const BatchDev &bd, const GroupDev &grp, uint64_t seg,
-                                            uint64_t lo, uint32_t kfirst, uint32_t *lds,
-                                            SegShared<T, K> &sh)
+                                            uint32_t rep, uint32_t nrep, uint64_t lo, uint32_t kfirst,
+                                            uint32_t *lds, SegShared<T, K> &sh)
 {
   constexpr uint32_t NW = T / CPX_WAVE, UPT = K / 32, WU = CPX_WAVE * UPT;
   constexpr uint32_t SB = 32u * K * T;
-  const uint32_t t = threadIdx.x, lane = lane_id(), wv = wave_id();
+  const uint32_t t = own_thread();
+  const uint32_t lane = t % CPX_WAVE, wv = (uint32_t)__builtin_amdgcn_readfirstlane((int)(t / CPX_WAVE));
   const uint64_t hi = lo + SB / 8 * 30, base = lo / 30;
   const uint32_t *__restrict__ sp = bd.primes;
   const uint32_t np_all = (uint32_t)bd.nprimes;
 
+  // (the same f64 estimate in every replica)
+  bool share = false;
+  if (nrep > 1) {
+    double ents = 0;
+    if (lane < grp.n && (sh.gm[lane].on & 2u)) {
+      const QueryDev &q = bd.queries[grp.q[lane]];
+      const double xf = (double)q.x_hi * 0x1p64 + (double)q.x_lo, sq = (double)q.sqrtx;
+      const double pm = lo ? fmin(sq, xf / (double)lo) : sq;
+      ents = fmax(0.0, pm - fmax((double)q.y, xf / (double)hi)) * (1.0 / 64);
+    }
+    share = wave_sum((unsigned long long)ents) > (unsigned long long)CPX_P2_SHARE * T;
+  }
+  if (rep && !share) {
+    if (t < grp.n && (sh.gm[t].on & 2u)) {
+      const QueryDev &q = bd.queries[grp.q[t]];
+      const uint64_t mr = q.mrow_base + bd.rowinfo[q.hard_row0 + seg].mrow + rep;
+      st_out(&bd.p2_np[mr], 0u);
+      st_out(&bd.p2_loc[mr], (uint64_t)0);
+    }
+    return;
+  }
+  // member g's P2 primes of the segment, (pmin, pmax], in lane g of every wave
+  uint64_t pmin = 0, pmax = 0;
+  if (lane < grp.n && (sh.gm[lane].on & 2u)) {
+    const QueryDev &q = bd.queries[grp.q[lane]];
+    const u128 x = ((u128)q.x_hi << 64) | q.x_lo;
+    pmax = lo ? min(q.sqrtx, cpx_div128_to64(x, lo)) : q.sqrtx;
+    pmin = max(q.y, cpx_div128_to64(x, hi));
+    pmin = min(pmin, pmax);
+  }
+  const uint32_t e0 = share ? rep * T + t : t, estep = share ? nrep * T : T;
+
   __syncthreads();
   // primes below P2_WAVE_P have many multiples: one prime per wave, eight
-  // classes of multiples times eight in step, so no lane walks a long chain alone
+  // classes of multiples times eight in step, so no lane walks a long chain
+  // alone.  (The wave's next 64 primes and their constants sit in its lanes;
+  // fetched one by one they cost pi(1e9) 6 us of 160.)
   {
     const CrossLane cl(lane);
-    for (uint32_t k = kfirst + (uint32_t)__builtin_amdgcn_readfirstlane((int)wv); k < np_all; k += NW) {
-      const uint32_t p = sp[k];
-      if (p >= P2_WAVE_P || (uint64_t)p * p >= hi) break;
-      p2_cross_wave<T>(lds, p, base, SB, cl, lane);
+    uint32_t n = CPX_WAVE;
+    for (uint32_t k0 = kfirst + wv; n == CPX_WAVE && k0 < np_all; k0 += NW * CPX_WAVE) {
+      const uint32_t k = k0 + NW * lane, pk = sp[min(k, np_all - 1)];
+      n = (uint32_t)__popcll(__ballot(k < np_all && pk < P2_WAVE_P && (uint64_t)pk * pk < hi));
+      const uint32_t d8k = 8 * (uint32_t)(base - cpx_div_leaf(base, (double)base, pk) * pk);
+      const uint32_t ack = pk / 30u << 6 | cop30_class8(pk);
+      for (uint32_t i = 0; i < n; i++) {
+        const uint32_t p = lane_read(pk, i), ac = lane_read(ack, i);
+        const uint32_t p8 = 8 * p, p64 = 64 * p;
+        uint32_t j = cl.first(ac >> 6, ac & 63u, p8, lane_read(d8k, i)) + (lane >> 3) * p8;
+        if (base == 0 && lane == 0) j += p64;             // p itself
+        for (; j < SB; j += p64) atomicAnd(unit_word(lds, j), ~(1u << (j & 31u)));
+      }
     }
   }
   // the rest: one prime per lane, class after class
@@ -463,34 +514,38 @@ __device__ __forceinline__ void p2_epilogue(const BatchDev &bd, const GroupDev &
 
     unsigned long long loc = 0;
     uint32_t np = 0;
-    uint64_t pmax = q.sqrtx;
-    if (lo) {
-      const uint64_t v = cpx_div128_to64(x, lo);
-      if (v < pmax) pmax = v;
-    }
-    uint64_t pmin = cpx_div128_to64(x, hi);
-    if (pmin < q.y) pmin = q.y;
-    if (pmax > pmin) {
-      const uint64_t e_lo = (pmin + 1) >> 6, e_hi = pmax >> 6;
-      for (uint64_t e = e_lo + t; e <= e_hi; e += T) {
+    const uint64_t p_lo = lane_read((uint32_t)pmin, g) | (uint64_t)lane_read((uint32_t)(pmin >> 32), g) << 32;
+    const uint64_t p_hi = lane_read((uint32_t)pmax, g) | (uint64_t)lane_read((uint32_t)(pmax >> 32), g) << 32;
+    if (p_hi > p_lo) {
+      const uint64_t e_lo = (p_lo + 1) >> 6, e_hi = p_hi >> 6;
+      for (uint64_t e = e_lo + e0; e <= e_hi; e += estep) {
         const PiEntry pe = bd.pitab[e];
         uint32_t b = pe.bits;
         const uint64_t base64 = 64 * e;
-        // keep odd integers base64 + 2i + 1 in (pmin, pmax]
-        if (pmax < base64 + 63) b &= cpx_lowmask32((uint32_t)((pmax - base64 + 1) >> 1));
-        if (pmin > base64) {
-          const uint64_t kk = (pmin - base64 + 1) >> 1;     // bits for integers <= pmin
+        // keep odd integers base64 + 2i + 1 in (p_lo, p_hi]
+        if (p_hi < base64 + 63) b &= cpx_lowmask32((uint32_t)((p_hi - base64 + 1) >> 1));
+        if (p_lo > base64) {
+          const uint64_t kk = (p_lo - base64 + 1) >> 1;     // bits for integers <= p_lo
           b = kk >= 32 ? 0u : (b & ~cpx_lowmask32((uint32_t)kk));
         }
-        while (b) {
-          const uint32_t i = __builtin_ctz(b);
-          b &= b - 1;
-          const uint64_t p = base64 + 2 * i + 1;
-          const uint64_t v = fastdiv ? cpx_div_leaf(q.x_lo, xf, (uint32_t)p)
-                                     : cpx_div128_to64(x, p);   // lo <= v < hi
-          loc += (unsigned long long)(count_to(v) - ce);
-          np++;
+        np += cpx_popc32(b);
+        while (b && fastdiv) {                              // lo <= x / p < hi
+          bool on[P2_U];
+          uint64_t v[P2_U];
+#pragma unroll
+          for (uint32_t u = 0; u < P2_U; u++) {
+            on[u] = b != 0;
+            const uint32_t i = on[u] ? __builtin_ctz(b) : 0u;
+            b &= b - 1;
+            v[u] = on[u] ? cpx_div_leaf(q.x_lo, xf, (uint32_t)(base64 + 2 * i + 1)) : lo;
+          }
+#pragma unroll
+          for (uint32_t u = 0; u < P2_U; u++) {
+            const uint32_t ct = count_to(v[u]);
+            loc += on[u] ? ct - ce : 0u;
+          }
         }
+        for (; b; b &= b - 1) loc += count_to(cpx_div128_to64(x, base64 + 2 * __builtin_ctz(b) + 1)) - ce;
       }
     }
     loc = wave_sum(loc);
@@ -501,10 +556,10 @@ __device__ __forceinline__ void p2_epilogue(const BatchDev &bd, const GroupDev &
       unsigned long long L = 0;
       uint32_t N = 0;
       for (uint32_t w = 0; w < NW; w++) { L += sh.red_u[w]; N += (uint32_t)sh.wsum[w]; }
-      const uint64_t row = q.p2_row0 + (seg - q.p2_seg0);
-      st_out(&bd.p2_cnt[row], (uint32_t)(tot - ce));
-      st_out(&bd.p2_np[row], (uint32_t)N);
-      st_out(&bd.p2_loc[row], (uint64_t)L);
+      const uint64_t mr = q.mrow_base + bd.rowinfo[q.hard_row0 + seg].mrow + rep;
+      if (rep == 0) st_out(&bd.p2_cnt[q.p2_row0 + (seg - q.p2_seg0)], (uint32_t)(tot - ce));
+      st_out(&bd.p2_np[mr], (uint32_t)N);
+      st_out(&bd.p2_loc[mr], (uint64_t)L);
     }
     __syncthreads();
   }
@@ -537,7 +592,8 @@ __device__ __forceinline__ void hard_chunks(const BatchDev &bd, SegShared<T, K> 
   constexpr uint32_t NW = T / CPX_WAVE, UPT = K / 32, WU = CPX_WAVE * UPT, WB = WU * 1024;
   constexpr uint32_t NI = SegShared<T, K>::NI;
   constexpr uint32_t SST = ChunkStages<GS>::SST < T / GS ? ChunkStages<GS>::SST : T / GS;
-  const uint32_t t = threadIdx.x, lane = lane_id();
+  const uint32_t t = own_thread();
+  const uint32_t lane = t % CPX_WAVE;
   const uint32_t wv = (uint32_t)__builtin_amdgcn_readfirstlane((int)wave_id());
   const uint64_t lo_w = lo + (uint64_t)wv * (WB / 8 * 30), hi_w = lo_w + WB / 8 * 30;
   const double inv_lo_w = lo_w ? 1.0 / (double)lo_w : 0.0, inv_hi_w = 1.0 / (double)hi_w;
@@ -856,7 +912,7 @@ __device__ __forceinline__ void hard_segment(const BatchDev &bd, const TileDev &
                                              SegShared<T, K> &sh)
 {
   constexpr uint32_t NW = T / CPX_WAVE, G = CPX_GROUP, SB = 32u * K * T;
-  const uint32_t t = threadIdx.x;
+  const uint32_t t = own_thread();
   const uint64_t seg = tile.seg;
   const uint64_t lo = seg * (SB / 8 * 30), hi = lo + SB / 8 * 30;
   const GroupDev &grp = bd.groups[tile.group];
@@ -914,7 +970,7 @@ __device__ __forceinline__ void hard_segment(const BatchDev &bd, const TileDev &
     for (uint32_t w = 0; w < NW; w++) tt += sh.acc[w][g];
     st_out(&bd.hard_acc[q.mrow_base + bd.rowinfo[row].mrow + rep], (int64_t)tt);
   }
-  if (rep == 0 && p2any) p2_epilogue<T, K>(bd, grp, seg, lo, cs + nst, lds, sh);
+  if (p2any) p2_epilogue<T, K>(bd, grp, seg, rep, tile.nrep, lo, cs + nst, lds, sh);
 }
 
 // Easy leaves (replaces S2_a / V_a / V_b, src/Deleglise-Rivat/S2.cu:72-99,
@@ -946,7 +1002,7 @@ __device__ __forceinline__ void easy_tile(const BatchDev &bd, uint32_t di, uint3
   uint32_t *sk1 = lds + 2 * T;                          // pi(min(y, x / p^2)): q indices end here
   uint32_t *sk0 = lds + 3 * T;                          // max(j + 1, pi(x / p^3)): and start here
   uint32_t *skr = lds + 4 * T;                          // and from here on count twice
-  const uint32_t t = threadIdx.x;
+  const uint32_t t = own_thread();
   const BlockDesc d = bd.easy_desc[di];
   const QueryDev &q = bd.queries[d.query];
   const u128 x = ((u128)q.x_hi << 64) | q.x_lo;
@@ -1058,7 +1114,7 @@ template <int T, int K>
 __device__ __forceinline__ void p2tab_tile(const BatchDev &bd, uint32_t di, uint32_t *lds)
 {
   constexpr uint32_t U = 4;
-  const uint32_t t = threadIdx.x;
+  const uint32_t t = own_thread();
   const BlockDesc d = bd.p2_desc[di];
   const QueryDev &q = bd.queries[d.query];
   const uint64_t x = q.x_lo;

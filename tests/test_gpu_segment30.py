@@ -70,3 +70,23 @@ def test_carry_runs(ctx, oracle, nseg, extra):
     y = max(int(z ** 0.5) + extra, 100)
     x = y * z + 3
     _same(ctx.pi(x, y=y, terms=True), oracle.pi_dr(x, y, 6), (x, y))
+
+
+# the P2 primes of a segment: counted by its first replica or shared by all of them, on both
+# sides of the rule, with y near and far from sqrt(x) and groups of several queries
+@pytest.mark.parametrize("x", [10 ** 9, 3 * 10 ** 10 + 1, 10 ** 11, 7 * 10 ** 11 + 9, 10 ** 12, 10 ** 13 + 37])
+@pytest.mark.parametrize("alpha", [1.0, 4.0, 17.0])
+def test_p2_shared(ctx, oracle, x, alpha):
+    y = oracle.choose_y(x, alpha)
+    ref = oracle.pi_dr(x, y, 6)
+    _same(ctx.pi(x, y=y, terms=True), ref, (x, y))
+    assert ctx.P2(x, y) == ref["p2"], (x, y)
+
+
+# the prime sieve of a P2 range by waves: 64 primes a wave at a time (all stage counts from
+# none, and the last prime below and at the square root of the segment's end)
+@pytest.mark.parametrize("x", [SEG, SEG + 1, 10 ** 7 + 19, 1400 ** 3, 1409 ** 3 - 1, 10 ** 10 - 33])
+def test_p2_wave_primes(ctx, oracle, x):
+    for alpha in (1.0, 2.0, 6.0):
+        y = oracle.choose_y(x, alpha)
+        _same(ctx.pi(x, y=y, c=4, terms=True), oracle.pi_dr(x, y, 4), (x, y))
