@@ -146,18 +146,31 @@ static hipError_t scan_entries(PiEntry *tab, uint64_t nent, uint32_t *tot, uint6
   return hipGetLastError();
 }
 
+static const uint64_t PITAB_SMALL = 1ull << 22;   // entries
+
+template <int K>
+static hipError_t pitab_seg(PiEntry *tab, uint64_t nent, const uint32_t *sprimes, uint32_t nsprimes, hipStream_t s)
+{
+  constexpr int T = 256;
+  const uint64_t nseg = (nent + K * T - 1) / (K * T);
+  hipLaunchKernelGGL((k_pitab_seg<T, K>), dim3((uint32_t)nseg), dim3(T), (size_t)(K + 1) * T * 4, s, tab, nent,
+                     sprimes, nsprimes);
+  return hipGetLastError();
+}
+
 // seg_tot / seg_base must hold ceil(nent / SCAN_CHUNK) entries.
 hipError_t launch_pitab_segments(PiEntry *tab, uint64_t nent, const uint32_t *sprimes,
                                  uint32_t nsprimes, uint32_t *seg_tot, uint64_t *seg_base,
                                  hipStream_t s)
 {
-  constexpr int T = 256, K = 32;                   // 2^18 odd bits per segment
-  const uint64_t ent_per_seg = (uint64_t)K * T;
-  uint64_t nseg = (nent + ent_per_seg - 1) / ent_per_seg;
-  size_t lds = (size_t)(K + 1) * T * 4;
-  hipLaunchKernelGGL((k_pitab_seg<T, K>), dim3((uint32_t)nseg), dim3(T), lds, s, tab, nent,
-                     sprimes, nsprimes);
-  hipError_t e = hipGetLastError();
+  // A block goes through the primes below 32 K one after another (0.8 us each:
+  // two 64-bit remainders and a barrier-free pass), so a small table takes the
+  // smallest segment, and only a large one, whose blocks queue, saves the set-up
+  // of every prime with a longer one: 57 K entries 163 us with K = 32, 51 with 8,
+  // 25 with 2; 0.5 M entries 171, 58, 39; 5 M entries 295, 197, 199; 54 M entries
+  // 1.67, 1.58, 2.26 ms.
+  hipError_t e = nent <= PITAB_SMALL ? pitab_seg<2>(tab, nent, sprimes, nsprimes, s)
+                                     : pitab_seg<8>(tab, nent, sprimes, nsprimes, s);
   if (e != hipSuccess) return e;
   return scan_entries(tab, nent, seg_tot, seg_base, s);
 }

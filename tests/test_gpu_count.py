@@ -29,3 +29,20 @@ def test_windows_at_squares(fresh, oracle, root, n):
     for lo in (root * root - n, root * root - n // 2, root * root):
         lo = max(lo, 0)
         assert fresh.countPrimes(lo, lo + n) == oracle.count_primes(lo, lo + n), (lo, n)
+
+
+# the pi table's segments (32768 integers for a table of up to 2^28, 131072 above): counts from
+# the table beside and across their ends and at its end, against the sieve of a context without it
+@pytest.mark.parametrize("x", [10 ** 10, 10 ** 15, 7 * 10 ** 16, 8 * 10 ** 16])
+def test_table_segments(oracle, x):
+    import cudapix_amd as C
+    top = int(x ** 0.5)
+    ends = [k * 32768 for k in (1, 2, 3, 4, 8)] + [top // 131072 * 131072, top // 32768 * 32768]
+    with C.Context(device=0) as c, C.Context(device=0) as d:
+        c.pi(x)
+        for e in ends:
+            if e > top:
+                continue
+            for lo, hi in ((e - 1000, e), (e - 1, e + 2), (max(e - 131072, 0), min(e + 32768, top))):
+                assert c.countPrimes(lo, hi) == d.countPrimes(lo, hi), (x, lo, hi)
+        assert c.countPrimes(0, top) == d.countPrimes(0, top), x
