@@ -68,7 +68,7 @@ def primes_upto(n):
     return np.nonzero(s)[0]
 
 
-GROUP = 8   # queries per shared segment sieve (the library's group capacity)
+GROUP = 32  # queries per shared segment sieve (the library's group capacity)
 
 # Tuning of the batched runs (segment threads, words per thread, alpha factor,
 # wheel primes): the fastest of the autotuner's choices on the 512-query
@@ -76,8 +76,13 @@ GROUP = 8   # queries per shared segment sieve (the library's group capacity)
 BENCH_TUNING = "512,32,0.3,8"
 
 
+def sieve_wheel(t):
+    """Primes of the segment sieve's pattern: those up to x^(1/4), at most 8."""
+    return sum(p <= iroot(t["x"], 4) for p in (2, 3, 5, 7, 11, 13, 17, 19))
+
+
 def sieve_groups(queries, primes):
-    """The library's query groups: increasing x, the same wheel c, at most
+    """The library's query groups: increasing x, the same sieve wheel, at most
     GROUP members, every member's P2 start (isqrt(x) rounded down to a
     multiple of 64) at or above every member's largest stage prime (the
     largest prime <= x^(1/4)), and a query with y >= 2^28 alone."""
@@ -86,10 +91,10 @@ def sieve_groups(queries, primes):
     groups, cur, smax, p2min = [], [], 0, None
     for t in order:
         qi = np.searchsorted(primes, iroot(t["x"], 4), side="right")
-        si = int(primes[qi - 1]) if qi > int(t["c"]) else 0
+        si = int(primes[qi - 1]) if qi > sieve_wheel(t) else 0
         pi = iroot(t["x"], 2) & ~63
         alone = t["y"] >= 1 << 28
-        if cur and (len(cur) == GROUP or int(cur[0]["c"]) != int(t["c"]) or alone
+        if cur and (len(cur) == GROUP or sieve_wheel(cur[0]) != sieve_wheel(t) or alone
                     or cur[-1]["y"] >= 1 << 28 or max(smax, si) > min(p2min, pi)):
             groups.append(cur)
             cur, smax, p2min = [], 0, None
@@ -105,20 +110,21 @@ def algorithmic_lds_bytes(queries, primes):
     """Segment-sieve LDS work of the DR staged sieve, per group of queries
     that share it (a single query is a group of one): with z and p_h the
     largest of the members' z = x/y and floor(x^(1/4)),
-    W = B_h * ceil(z/2)/8 + 8 * sum_{b=c+1}^{c+B_h} ceil((z/2)/p_b),
-    one popcount/prefix pass over the odd-only bitmap per stage plus one
-    32-bit read-modify-write per cross-off.  (Leaf evaluations are not in W:
+    W = B_h * ceil(8z/30)/8 + 8 * sum_{b=w+1}^{w+B_h} ceil((8z/30)/p_b),
+    one popcount/prefix pass over the bitmap of the integers coprime to 30 per
+    stage plus one 32-bit read-modify-write per cross-off, over the stages above
+    the sieve's wheel of w primes.  (Leaf evaluations are not in W:
     they read a few words each.)"""
     import numpy as np
     tot = 0
     for g in sieve_groups(queries, primes):
-        c = int(g[0]["c"])
+        c = sieve_wheel(g[0])
         z = max(t["x"] // t["y"] for t in g)
         ph = max(iroot(t["x"], 4) for t in g)
         ps = primes[c:np.searchsorted(primes, ph, side="right")]
         bh = len(ps)
-        half = (z + 1) // 2
-        tot += bh * half / 8.0 + 8.0 * float(np.sum(np.ceil(half / ps.astype(np.float64))))
+        bits = (8 * z + 29) // 30
+        tot += bh * bits / 8.0 + 8.0 * float(np.sum(np.ceil(bits / ps.astype(np.float64))))
     return tot
 
 
@@ -157,24 +163,26 @@ LDS_PEAK_GBS = 256 * CU_COUNT * CLOCK_GHZ       # GB/s
 
 
 def hbm_model_bytes(terms, primes, seg_bits):
-    """W_HBM of one batch launch (a model, labelled as such): 4 B per hard-leaf
-    candidate (the packed mu*lpf word of each odd m in (y/p, y], or the prime
-    list entry when p^2 > y), 8 B per easy-leaf pair (one pi-table entry),
-    8 B per P2 prime (one pi-table entry at x/p), and 8 B per wheel word
-    filled into each segment of each query group (seg_bits odd numbers per
-    segment; replicas of a segment not counted).  Tables are resident and
+    """W_HBM of one batch launch (a model, labelled as such): 8 B per hard-leaf
+    candidate of the sieved stages (the leaf table's entry of each m coprime to
+    30030 in (y/p, y]), 4 B when p^2 > y (the prime list's entry), 8 B per
+    easy-leaf pair (one pi-table entry; pairs above sqrt(x/p) are counted from
+    the smaller side with fewer), 8 B per P2 prime (one pi-table entry at x/p),
+    and 4 B per pattern word filled into each segment of each query group
+    (seg_bits integers coprime to 30 per segment; replicas of a segment not
+    counted).  Tables are resident and
     not rebuilt inside the launch."""
     import numpy as np
-    nseg = sum(-(-((max(t["x"] // t["y"] for t in g) + 1) // 2) // seg_bits)
+    nseg = sum(-(-(max(t["x"] // t["y"] for t in g) + 1) // (seg_bits // 8 * 30))
                for g in sieve_groups(terms, primes))
     pi_at = lambda v: int(np.searchsorted(primes, v, side="right"))
-    l_hard = l_easy = n_p2 = 0
+    l_hard = l_dense = l_easy = n_p2 = 0
     for t in terms:
-        x, y, c = t["x"], t["y"], int(t["c"])
+        x, y, c = t["x"], t["y"], sieve_wheel(t)
         q4, c3, sq = iroot(x, 4), iroot(x, 3), iroot(x, 2)
         ps = primes[c:pi_at(q4)].astype(np.int64)
         dense = ps[ps * ps <= y]
-        l_hard += int(np.sum((y - y // dense + 1) // 2))
+        l_dense += int(np.sum((y - y // dense) * 5760 // 30030))
         for p in ps[ps * ps > y]:
             l_hard += max(0, pi_at(y) - pi_at(max(int(p), y // int(p))))
         for p in primes[pi_at(q4):pi_at(c3)]:
@@ -183,8 +191,8 @@ def hbm_model_bytes(terms, primes, seg_bits):
                 l_easy += pi_at(hi) - pi_at(int(p))
         n_p2 += max(0, pi_at(sq) - pi_at(y))
     wheel = nseg * seg_bits // 32
-    w = 4 * l_hard + 8 * l_easy + 8 * n_p2 + 8 * wheel
-    return w, {"hard_candidates": l_hard, "easy_pairs": l_easy, "p2_primes": n_p2,
+    w = 8 * l_dense + 4 * l_hard + 8 * l_easy + 8 * n_p2 + 4 * wheel
+    return w, {"hard_candidates": l_dense + l_hard, "easy_pairs": l_easy, "p2_primes": n_p2,
                "group_segments": nseg, "wheel_words": wheel}
 
 
@@ -704,7 +712,7 @@ def main():
             "lds": {"counted_bytes": lds_counted,
                     "counted_GBs": round(lds_counted / seg_avg_s / 1e9, 1) if lds_counted else None,
                     "model_bytes": w_lds,
-                    "model": "W_LDS = B_h*ceil(z/2)/8 + 8*sum ceil((z/2)/p_b) per query group (one "
+                    "model": "W_LDS = B_h*ceil(8z/30)/8 + 8*sum ceil((8z/30)/p_b) per query group (one "
                              "popcount pass per stage + one RMW per cross-off); the kernel does less "
                              "(no per-stage pass), so W_LDS over time is not a bandwidth",
                     "peak_GBs": round(LDS_PEAK_GBS, 1), "probe_GBs": round(lds_probe / 1e9, 1),

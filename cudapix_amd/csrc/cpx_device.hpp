@@ -260,11 +260,6 @@ __device__ __forceinline__ uint32_t seg_addr(uint32_t g, uint32_t K, uint32_t T)
   return g + g / K;
 }
 
-__device__ __forceinline__ uint32_t own_addr(uint32_t t, uint32_t j, uint32_t K)
-{
-  return t * (K + 1) + j;
-}
-
 // Bit offset, inside a segment whose bit i is the integer lo + 2i + 1 (lo even),
 // of the first odd multiple of the odd prime p that is >= max(lo + 1, from).
 __device__ __forceinline__ uint64_t first_odd_multiple_bit(uint64_t lo, uint32_t p, uint64_t from)

@@ -3,10 +3,10 @@
 // One context = one device stream + resident tables (compact pi table,
 // prime list, mu*lpf table, wheel patterns) + a batch arena.  A batch of
 // queries is planned on the host (bounds by exact integer roots, tile and
-// block-descriptor lists, tiles ordered longest-first), uploaded with one copy
-// per array, and run as a fixed-shape launch sequence:
-//   zero queue -> setup -> ordinary -> trivial -> easy -> segments(persistent)
-//   -> hard carry -> combine
+// block-descriptor lists, tiles ordered longest-first), uploaded (one copy for a
+// plan up to 256 KB), and run as a fixed-shape launch sequence:
+//   setup (stage tables, ordinary, wheel-stage and trivial leaves)
+//   -> segments (persistent) -> hard carry -> combine
 // which is captured once into a hipGraph and replayed while the arena keeps
 // its capacity.  (The reference instead runs each term as its own host loop
 // of kernel + cudaDeviceSynchronize + thrust reduce, with cudaDeviceReset
@@ -331,7 +331,7 @@ int ensure_tables(cpx_ctx *c, uint64_t R, uint64_t P, uint64_t Y)
   }
   if (Pm >= (1ull << 32)) return ctx_fail(c, CPX_ERANGE, "prime table above 2^32 is not supported");
   free_tables(c);
-  // pi table over [0, 64 * nent), nent a multiple of the 8192-entry segment
+  // pi table over [0, 64 * nent), nent a multiple of 8192 (of a table segment)
   uint64_t nent = (Rm + 1 + 63) / 64;
   nent = (nent + 8191) / 8192 * 8192;
   if ((rc = dbuf_reserve(c, c->pitab, nent, &c->table_bytes))) return rc;

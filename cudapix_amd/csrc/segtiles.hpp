@@ -590,7 +590,6 @@ __device__ __forceinline__ void hard_chunks(const BatchDev &bd, SegShared<T, K> 
                                             uint64_t lo, uint64_t hi)
 {
   constexpr uint32_t NW = T / CPX_WAVE, UPT = K / 32, WU = CPX_WAVE * UPT, WB = WU * 1024;
-  constexpr uint32_t NI = SegShared<T, K>::NI;
   constexpr uint32_t SST = ChunkStages<GS>::SST < T / GS ? ChunkStages<GS>::SST : T / GS;
   const uint32_t t = own_thread();
   const uint32_t lane = t % CPX_WAVE;
@@ -901,7 +900,6 @@ __device__ __forceinline__ void hard_chunks(const BatchDev &bd, SegShared<T, K> 
     const long long a = wave_sum((long long)acc);
     if (lane == 0) sh.acc[wv][0] = a;
   }
-  (void)NI;
 }
 
 // One tile: segment `seg` of a group, replica `rep` of `nrep`.  The wheel
