@@ -47,6 +47,7 @@ struct StreamRec {
   uint64_t n_main;       // main tiles
   uint64_t n_fin;        // carry descriptors
   uint64_t n_comb;       // queries (combine units)
+  uint64_t fin_rows;     // rows of a carry descriptor, on average (sizes the claims)
   uint64_t q_base, tile_base, fin_base;   // its first query, main tile and carry descriptor
   uint64_t nranges;      // its entries in the plan region: bytes [off, off + len) of each
   uint64_t off[12], len[12];   // (multiples of 4; copy units walk their concatenation)

@@ -1829,6 +1829,9 @@ int stream_plan(cpx_ctx *c, std::vector<HostQuery> &hq, BatchSlot &S, const Caps
   ci->q_base = base.q;
   ci->tile_base = base.tiles;
   ci->fin_base = base.fin;
+  ci->fin_rows = 0;
+  for (const BlockDesc &d : pl.fin) ci->fin_rows += d.begin >> 32;
+  if (pl.nfin) ci->fin_rows /= pl.nfin;
   {
     uint64_t *nx = &ci->next.q;
     const uint64_t *b = &base.q, *n = &need.q;

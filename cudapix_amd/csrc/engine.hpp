@@ -162,6 +162,7 @@ struct CohortInfo {
   uint64_t need_bytes = 0;       // plan + out bytes at exactly the capacities the plan needs
   uint64_t hard_segments = 0;
   uint64_t q_base = 0, tile_base = 0, fin_base = 0;   // its first query, tile, carry descriptor
+  uint64_t fin_rows = 0;                              // rows of a carry descriptor, on average
   Caps next{};                   // the arena cursor after its entries
 };
 bool tables_cover(const cpx_ctx *c, uint64_t R, uint64_t P, uint64_t Y);

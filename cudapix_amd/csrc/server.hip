@@ -285,6 +285,7 @@ static int publish(cpx_server *s, uint32_t j, const CohortInfo &ci, std::vector<
   r.seq = seq;
   r.n_main = ci.n_main;
   r.n_fin = ci.n_fin;
+  r.fin_rows = ci.fin_rows;
   r.n_comb = ci.nq;
   r.q_base = ci.q_base;
   r.tile_base = ci.tile_base;

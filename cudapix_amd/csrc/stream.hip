@@ -103,24 +103,26 @@ static __device__ __forceinline__ bool slot_of(const StreamPub *pub, uint32_t ns
 // host may reuse the record, so a head read before a record's reuse no longer
 // matches at the compare-and-swap.  A claim at or past the count (read again
 // after the claim) is no work.
-// A claim takes a run of 16 to 64 units (two shares of the count): a cohort's
-// carry has thousands of units of a few microseconds each, every idle block
-// contends for the one head, and a claim reads pinned memory between its load
-// and its compare-and-swap, so about one succeeds per bus round trip and the
-// claims are the cost of the phase.  (A burst of 100 requests below 1e14, whose
-// carry is about 3000 units: 23 ms with runs of 2, 4 ms with 16.)
-static __device__ __forceinline__ bool claim_phase(uint64_t *head, const uint64_t *count, uint64_t *idx,
-                                                   uint32_t *n)
+// A claim takes a run of units: every idle block contends for the one head, and
+// a claim reads pinned memory between its load and its compare-and-swap, so
+// about one succeeds per bus round trip (2 us).  n units of u microseconds in
+// runs of k cost 2 n / k of claims and k u at the end: k = sqrt(2 n / u), with u
+// about 8 + rows / 100, at most 64.  (Runs of 2 took 23 ms for the 3000 units of
+// 100 requests below 1e14; runs of 16 or more left the 128 long units of one
+// query near 1e17 to 8 blocks, and 200 such requests/s waited 204 ms on average
+// instead of 120.)
+static __device__ __forceinline__ bool claim_phase(uint64_t *head, const uint64_t *count, const uint64_t *rows,
+                                                   uint64_t *idx, uint32_t *n)
 {
   for (;;) {
     const uint64_t v = ld_dev(head);
     const uint32_t i = (uint32_t)v;
     if (i == 0xffffffffu) return false;
     order_acquire();
-    const uint64_t cnt = ld_sys(count);
+    const uint64_t cnt = ld_sys(count), cost = 800 + (rows ? ld_sys(rows) : 0);
     if (i >= cnt) return false;
-    uint64_t k = 2 * cnt / gridDim.x;
-    k = k < 16 ? 16 : (k > 64 ? 64 : k);
+    uint64_t k = (uint64_t)__builtin_sqrtf(200.0f * (float)(cnt - i) / (float)cost);
+    k = k < 1 ? 1 : (k > 64 ? 64 : k);
     if (k > cnt - i) k = cnt - i;
     if (cas_dev(head, v, v + k)) {
       order_acquire();
@@ -153,13 +155,14 @@ static __device__ __forceinline__ bool claim_fifo(uint64_t *head, uint64_t end, 
 // (each claim a compare-and-swap at device scope), so while many tiles are
 // left a claim takes a run of up to 16 consecutive tiles (1 near the end,
 // where the longest-first order leaves the short tiles to balance the grid).
-// Two shares of what is left: the same burst's main phase took 17 ms with a
-// quarter share, 11 with a half, 9 with one; at three the largest cohorts'
-// last long runs show (16 requests to 1e16: 12.5 ms with one share, 14.4 with
-// two, 15-17 with three; 512 requests to 1e13: 22, 16.5 and 16 ms).
+// Half a share of what is left: longer runs serve a burst sooner but hold up the
+// cohorts that join behind a large query's long tiles (a burst of 100 requests
+// below 1e14 takes 13 ms with two shares, 18.6 with a half, 23 with a quarter;
+// 200 requests/s with x < 1e17 wait 276 and 166 ms on average, 100 and 118, and
+// 66 and 112, in two runs each).
 static __device__ __forceinline__ uint64_t main_claim_run(uint64_t left)
 {
-  const uint64_t k = 2 * left / gridDim.x;
+  const uint64_t k = left / (2ull * gridDim.x);
   return k < 1 ? 1 : (k > 16 ? 16 : k);
 }
 
@@ -194,12 +197,12 @@ static __device__ __attribute__((noinline)) void stream_find(const StreamArgs &a
   // are numbered within the cohort; its entries start at the bases)
   uint32_t k;
   for (j = 0; j < a.nslots; j++)
-    if (claim_phase(&ctl->comb_head[j], &pub->rec[j].n_comb, &v, &k)) {
+    if (claim_phase(&ctl->comb_head[j], &pub->rec[j].n_comb, nullptr, &v, &k)) {
       w = {SW_COMB, j, ld_sys(&pub->rec[j].q_base) + v, k};
       return;
     }
   for (j = 0; j < a.nslots; j++)
-    if (claim_phase(&ctl->fin_head[j], &pub->rec[j].n_fin, &v, &k)) {
+    if (claim_phase(&ctl->fin_head[j], &pub->rec[j].n_fin, &pub->rec[j].fin_rows, &v, &k)) {
       w = {SW_FIN, j, ld_sys(&pub->rec[j].fin_base) + v, k};
       return;
     }
