@@ -667,15 +667,44 @@ static void plan_query(const cpx_ctx *c, const HostQuery &h, uint32_t i, uint32_
   }
 }
 
+// Weights of the planning rules: a stage of a segment costs a block about what
+// STAGE_LEAVES leaf candidates do, and a replica (which sieves the segment
+// again) is not made for less than REP_SIEVE times its sieve where the chip is
+// full anyway.
+static const double STAGE_LEAVES = 143.0, REP_SIEVE = 16.0;
+
+// Members of a group at most.  Sharing saves sieving and lengthens the chain of
+// the block that holds the first segments: nearly every stage there has leaves
+// of every member, and a chunk's 96 items are three stages of 32 members but
+// twelve of eight.  A batch of little work waits for that chain, a larger one
+// covers it with other tiles.  Measured (ms, groups of 8 against 32; work = leaf
+// candidates and stages of every query on its own): 512 queries in [1e9, 1e12]
+// 2.49 / 2.76 (4.7e7), 64 in [1e12, 1e13] 1.60 / 2.09 (6.0e7), 512 in [1e9, 1e13]
+// 3.96 / 5.12 (1.7e8); with alpha factor 0.3 and c = 8, 512 in [1e9, 1e13] 3.40 /
+// 3.86 (1.7e8), 512 in [1e11, 1e13] 4.98 / 4.56 (3.2e8), 512 in [1e9, 1e14] 7.17 /
+// 6.98 (7.8e8), 512 in [1e9, 1e15] 21.4 / 16.8 (3.7e9).
+static const double GROUP_WORK = 2.4e8;
+static const uint32_t GROUP_SMALL = 8;
+
+static uint32_t group_members(const std::vector<QPlan> &qps)
+{
+  double work = 0;
+  for (const QPlan &qp : qps) {
+    for (float l : qp.rleaves) work += l;
+    work += STAGE_LEAVES * (double)qp.tm;
+  }
+  return work < GROUP_WORK ? GROUP_SMALL : CPX_GROUP;
+}
+
 // Groups of queries that share the segment sieve: queries with hard rows,
-// in increasing x, with the same wheel, at most CPX_GROUP, and every
+// in increasing x, with the same wheel, at most `most`, and every
 // member's P2 range (from p2_e) above every member's stage primes (segment 0
 // loses its stage primes to the sieve, so they must not be counted as P2
-// primes of another member).  A query with y >= 2^28 stays alone, which
-// keeps a wave's leaf list of a group (at most y/2 candidates per member)
-// below 2^30 entries.
+// primes of another member).  A query with y >= 2^28 stays alone: a member
+// has at most 0.192 y dense candidates (the m coprime to 30030), so a wave's
+// leaf list of 32 members stays below 1.65e9 entries, inside an int32.
 static void make_groups(const cpx_ctx *c, const std::vector<HostQuery> &hq,
-                        const std::vector<QPlan> &qps, std::vector<GroupDev> &groups)
+                        const std::vector<QPlan> &qps, uint32_t most, std::vector<GroupDev> &groups)
 {
   std::vector<uint32_t> hs;
   for (uint32_t i = 0; i < (uint32_t)qps.size(); i++)
@@ -689,7 +718,7 @@ static void make_groups(const cpx_ctx *c, const std::vector<HostQuery> &hq,
     const uint64_t si = d.nstage ? c->h_primes[d.cs + d.nstage - 1] : 0;
     const uint64_t pi = d.p2_nseg ? d.p2_e : ~0ull;
     const bool alone = d.y >= (1ull << 28);
-    if (cur.n && (cur.n == CPX_GROUP || qps[cur.q[0]].d.cs != d.cs || alone || cur_alone ||
+    if (cur.n && (cur.n == most || qps[cur.q[0]].d.cs != d.cs || alone || cur_alone ||
                   std::max(smax, si) > std::min(p2min, pi))) {
       groups.push_back(cur);
       cur = GroupDev{};
@@ -703,12 +732,6 @@ static void make_groups(const cpx_ctx *c, const std::vector<HostQuery> &hq,
   }
   if (cur.n) groups.push_back(cur);
 }
-
-// Weights of the replica rule: a stage of a segment costs a block about what
-// STAGE_LEAVES leaf candidates do, and a replica (which sieves the segment
-// again) is not made for less than REP_SIEVE times its sieve where the chip is
-// full anyway.
-static const double STAGE_LEAVES = 143.0, REP_SIEVE = 16.0;
 
 // pi-table entries that hold a query's P2 primes of the segment [lo, hi), and
 // the leaf candidates that counting the primes of one costs as much as.
@@ -906,7 +929,7 @@ static int build_plan(cpx_ctx *c, const std::vector<HostQuery> &hq, uint32_t mas
   const unsigned nt = plan_threads(nq);
   parallel_for(nq, nt, [&](size_t i) { plan_query(c, hq[i], (uint32_t)(B.q + i), mask, qps[i], nq); });
   pl.groups.clear();
-  make_groups(c, hq, qps, pl.groups);
+  make_groups(c, hq, qps, group_members(qps), pl.groups);
   // leaves of one tile (a segment with more becomes replicas): 16 K at least,
   // 512 K at most, between them four fifths of the work of one of 512 blocks,
   // so that no tile outlasts the others' work and none is sieved more often

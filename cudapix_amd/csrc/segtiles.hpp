@@ -290,8 +290,9 @@ template <int K>
 __device__ __forceinline__ void hard_lane_accumulate(int32_t val, int32_t sg, uint32_t fb, uint32_t my_lo,
                                                      uint32_t my_hi, int64_t &acc, int32_t &wmv)
 {
-  // list offsets are below 2^30: an item has at most y/2 candidates, and
-  // groups of more than one member have y < 2^28
+  // list offsets are below 2^31: an item has at most 0.192 y candidates (m
+  // coprime to 30030), and groups of more than one member have y < 2^28, so
+  // 32 of them at most 1.65e9
   const int32_t lo = min(max((int32_t)my_lo - (int32_t)fb, 0), CPX_WAVE);
   const int32_t hi = min(max((int32_t)my_hi - (int32_t)fb, 0), CPX_WAVE);
   auto range = [&](uint32_t S) {

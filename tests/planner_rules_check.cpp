@@ -1,0 +1,65 @@
+// planner_rules_check.cpp -- host-only checks of the batch planner's rules (CPU
+// test, no GPU): what planner_check.cpp builds, with commands of its own.
+//
+// stdin, one command per line (x decimal, key=value options first: shape=TxK,
+// alpha=<factor>, c=<wheel>; any of them makes the context a tuned one):
+//   groups x x ...   "groups <size> <size> ..." of the plan, by increasing x
+#define main planner_check_main
+#include "planner_check.cpp"
+#undef main
+
+struct Cmd {
+  std::string what;
+  std::vector<HostQuery> hq;
+};
+
+static void plan_into(cpx_ctx *c, Cmd &cmd, Plan &pl)
+{
+  choose_p2tab(c, cmd.hq, TERM_ALL, 0);
+  uint64_t R = 0, P = 0, Y = 0;
+  for (const HostQuery &h : cmd.hq) plan_needs(c, h, TERM_ALL, c->shape.seg_bits(), &R, &P, &Y);
+  fake_tables(c, R, P, Y);
+  CHECK(build_plan(c, cmd.hq, TERM_ALL, pl) == CPX_OK, "build_plan");
+}
+
+int main()
+{
+  std::string line;
+  while (std::getline(std::cin, line)) {
+    if (line.empty()) continue;
+    cpx_ctx ctx;
+    cpx_ctx *c = &ctx;
+    c->opts.c = 6;
+    c->opts.alpha = 0;
+    c->opts.fresh_tables = 0;
+    c->shape = {512, 32};
+    std::istringstream in(line);
+    Cmd cmd;
+    in >> cmd.what;
+    std::string tok;
+    while (in >> tok) {
+      const size_t eq = tok.find('=');
+      if (eq != std::string::npos) {
+        const std::string k = tok.substr(0, eq), v = tok.substr(eq + 1);
+        if (k == "shape") CHECK(std::sscanf(v.c_str(), "%dx%d", &c->shape.threads, &c->shape.kwords) == 2, "shape");
+        if (k == "alpha") c->alpha_scale = std::atof(v.c_str());
+        if (k == "c") c->opts.c = (uint32_t)std::atoi(v.c_str());
+        c->shape_tuned = true;
+        continue;
+      }
+      HostQuery h;
+      CHECK(make_host_query(c, parse_u128(tok), 0, 0, &h) == CPX_OK, "make_host_query");
+      cmd.hq.push_back(h);
+    }
+    if (cmd.what == "groups") {
+      Plan pl;
+      plan_into(c, cmd, pl);
+      std::printf("groups");
+      for (const GroupDev &g : pl.groups) std::printf(" %u", g.n);
+      std::printf("\n");
+    } else {
+      CHECK(false, "unknown command");
+    }
+  }
+  return 0;
+}

@@ -1,0 +1,51 @@
+"""CPU test: the rules the batch planner chooses by (tests/planner_rules_check.cpp,
+the engine's host code with every kernel launcher stubbed, under AddressSanitizer)."""
+import os
+import random
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HIPCC = "/opt/rocm/bin/hipcc"
+
+
+@pytest.fixture(scope="module")
+def checker(tmp_path_factory):
+    if not os.path.exists(HIPCC) or not shutil.which("g++"):
+        pytest.skip("no hipcc")
+    exe = tmp_path_factory.mktemp("planner") / "planner_rules_check"
+    cmd = [HIPCC, "-x", "hip", "--offload-host-only", "-std=c++17", "-O1", "-g",
+           "-Xarch_host", "-fsanitize=address", "-fno-omit-frame-pointer",
+           os.path.join(ROOT, "tests", "planner_rules_check.cpp"), "-o", str(exe), "-lpthread"]
+    subprocess.run(cmd, check=True, capture_output=True)
+    return exe
+
+
+def run(exe, lines):
+    env = dict(os.environ, ASAN_OPTIONS="detect_leaks=0:abort_on_error=0")
+    p = subprocess.run([str(exe)], input="\n".join(lines) + "\n", capture_output=True, text=True,
+                       env=env, timeout=600)
+    assert p.returncode == 0, p.stdout[-2000:] + p.stderr[-4000:]
+    out = [ln.split() for ln in p.stdout.splitlines()]
+    assert len(out) == len(lines), p.stdout
+    return [o[1:] for o in out]
+
+
+def spread(seed, n, lo, hi):
+    r = random.Random(seed)
+    return [int(10 ** r.uniform(lo, hi)) for _ in range(n)]
+
+
+# a batch of little work waits for the chain of the block with its first
+# segments, which grows with the members: groups of eight there, of 32 above
+@pytest.mark.parametrize("n,lo,hi,tuning,most", [
+    (64, 9, 13, "", 8), (128, 9, 13, "", 8), (512, 9, 12, "", 8), (512, 9, 13, "", 8), (64, 12, 13, "", 8),
+    (128, 9, 13, "alpha=0.3 c=8", 8), (512, 9, 12, "alpha=0.3 c=8", 8), (64, 12, 13, "alpha=0.3 c=8", 8),
+    (512, 9, 15, "", 32), (512, 9, 15, "alpha=0.3 c=8", 32), (64, 14, 15, "alpha=0.3 c=8", 32),
+    (256, 14, 15, "", 32)])
+def test_group_members(checker, n, lo, hi, tuning, most):
+    xs = spread(n, n, lo, hi)
+    sizes = list(map(int, run(checker, ["groups %s %s" % (tuning, " ".join(map(str, xs)))])[0]))
+    assert sum(sizes) == n and max(sizes) == most, sizes
