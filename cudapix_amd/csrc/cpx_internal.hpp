@@ -253,6 +253,7 @@ struct SegShape {
   uint64_t seg_bits() const { return 32ull * kwords * threads; }
   uint64_t seg_ints() const { return seg_bits() / 8 * 30; }
 };
+#define CPX_SEG_BITS_MAX (1ull << 20)   // of the largest shape
 
 // ------------------------------------------------------------- launchers
 // tables.hip

@@ -403,6 +403,18 @@ static void plan_needs(const cpx_ctx *c, const HostQuery &h, uint32_t mask, uint
   (void)c;
 }
 
+// Table needs of a batch, the same in every segment shape (the prime list
+// reaches the last P2 segment's end in the largest one: a few hundred primes more at most),
+// so that a call in one shape finds the tables that a call in another built: a
+// lone query below SMALL_SHAPE_X and the same query in a batch or without
+// allocation run in different ones.
+static void batch_needs(const cpx_ctx *c, const std::vector<HostQuery> &hq, uint32_t mask, uint64_t *R,
+                        uint64_t *P, uint64_t *Y)
+{
+  *R = *P = *Y = 0;
+  for (const HostQuery &h : hq) plan_needs(c, h, mask, CPX_SEG_BITS_MAX, R, P, Y);
+}
+
 // One query's share of the plan, with query-local offsets (rows, parts,
 // counters); build_plan places the shares.
 struct QPlan {
@@ -1601,8 +1613,7 @@ static int submit_impl(cpx_ctx *c, const std::vector<HostQuery> &hq_in, uint32_t
   // freed only after the stream has drained (dbuf_reserve), so a batch still
   // in flight in the other slot keeps reading valid tables
   uint64_t R = 0, P = 0, Y = 0;
-  const uint64_t SB = c->shape.seg_bits();
-  for (const HostQuery &h : hq) plan_needs(c, h, mask, SB, &R, &P, &Y);
+  batch_needs(c, hq, mask, &R, &P, &Y);
   const double tt0 = now_ms();
   int rc = ensure_tables(c, R, P, Y);
   if (rc) return rc;
@@ -1717,10 +1728,8 @@ int run_queries_at(cpx_ctx *c, std::vector<HostQuery> &hq, void *d_region, uint6
   choose_p2tab(c, hq, TERM_ALL, 1);
   uint64_t R = 0, P = 0, Y = 0;
   uint32_t cmax = 1;
-  for (const HostQuery &h : hq) {
-    plan_needs(c, h, TERM_ALL, c->shape.seg_bits(), &R, &P, &Y);
-    cmax = std::max(cmax, h.c);
-  }
+  batch_needs(c, hq, TERM_ALL, &R, &P, &Y);
+  for (const HostQuery &h : hq) cmax = std::max(cmax, h.c);
   if (!tables_cover(c, R, P, Y) || !c->wheel.p || cmax > c->wheel_c)
     return ctx_fail(c, CPX_EAGAIN, "the resident tables do not cover this batch (an allocating call at this size "
                                    "builds them)");
@@ -1777,8 +1786,7 @@ void stream_table_needs(const cpx_ctx *c, std::vector<HostQuery> &hq, uint64_t *
   if (p2_lookups)
     for (HostQuery &h : hq)                    // every eligible query, even alone
       h.p2tab = !h.small && h.y < h.sqrtx && h.sqrtx < (1ull << 32) && h.zt < P2TAB_LIMIT;
-  *R = *P = *Y = 0;
-  for (const HostQuery &h : hq) plan_needs(c, h, TERM_ALL, c->shape.seg_bits(), R, P, Y);
+  batch_needs(c, hq, TERM_ALL, R, P, Y);
 }
 
 int stream_plan(cpx_ctx *c, std::vector<HostQuery> &hq, BatchSlot &S, const Caps &cursor, bool grow,

@@ -28,6 +28,9 @@ __global__ __launch_bounds__(T, (SegLds<T, K>::waves())) void k_segments(BatchDe
 #define CPX_SEG_SHAPES(X) \
   X(64, 32) X(64, 64) X(64, 128) X(128, 32) X(128, 64) X(256, 32) X(256, 64) X(256, 128) \
   X(512, 32) X(512, 64)
+#define X(TT, KK) static_assert(32ull * TT * KK <= CPX_SEG_BITS_MAX, "table needs cover every shape");
+CPX_SEG_SHAPES(X)
+#undef X
 
 bool seg_shape_supported(SegShape s)
 {

@@ -4,6 +4,8 @@
 // stdin, one command per line (x decimal, key=value options first: shape=TxK,
 // alpha=<factor>, c=<wheel>; any of them makes the context a tuned one):
 //   groups x x ...   "groups <size> <size> ..." of the plan, by increasing x
+//   needs x x ...    "needs <R> <P> <Y>": the tables the batch asks for, which must
+//                    reach the end of its last P2 segment in the context's shape
 #define main planner_check_main
 #include "planner_check.cpp"
 #undef main
@@ -57,6 +59,16 @@ int main()
       std::printf("groups");
       for (const GroupDev &g : pl.groups) std::printf(" %u", g.n);
       std::printf("\n");
+    } else if (cmd.what == "needs") {
+      choose_p2tab(c, cmd.hq, TERM_ALL, 1);
+      uint64_t R, P, Y;
+      const ShapeScope scope(c, cmd.hq);
+      batch_needs(c, cmd.hq, TERM_ALL, &R, &P, &Y);
+      for (const HostQuery &h : cmd.hq) {
+        const uint64_t SI = c->shape.seg_ints();
+        if (!h.small && h.y < h.sqrtx) CHECK(P >= cpx_isqrt128((u128)(h.zt / SI + 1) * SI), "primes of the last segment");
+      }
+      std::printf("needs %llu %llu %llu\n", (unsigned long long)R, (unsigned long long)P, (unsigned long long)Y);
     } else {
       CHECK(false, "unknown command");
     }

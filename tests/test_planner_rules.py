@@ -49,3 +49,12 @@ def test_group_members(checker, n, lo, hi, tuning, most):
     xs = spread(n, n, lo, hi)
     sizes = list(map(int, run(checker, ["groups %s %s" % (tuning, " ".join(map(str, xs)))])[0]))
     assert sum(sizes) == n and max(sizes) == most, sizes
+
+
+# a query asks for the same tables whatever shape its batch runs in: one that a
+# lone query built serves the same query in a batch or without allocation
+@pytest.mark.parametrize("x", [10 ** 9, 10 ** 10, 10 ** 11, 10 ** 12, 10 ** 15, 10 ** 16, 10 ** 18])
+def test_needs_in_every_shape(checker, x):
+    shapes = ["64x32", "64x128", "128x64", "256x32", "256x128", "512x32", "512x64"]
+    r = run(checker, ["needs %d" % x, "needs %d %d" % (x, x)] + ["needs shape=%s %d" % (s, x) for s in shapes])
+    assert all(v == r[0] for v in r), r
