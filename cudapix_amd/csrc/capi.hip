@@ -1056,7 +1056,28 @@ int cpx_pi_batch_collect(cpx_ctx *c, uint64_t ticket, cpx_u128 *out, cpx_batch_s
 // Times one calibration batch per candidate and keeps the fastest, in three
 // passes: the segment shape, then a factor on the alpha model, then the
 // number of wheel primes c.  Every candidate must return the same pi(x) for
-// every query (bit for bit), or the tuner fails.
+// every query (bit for bit), or the tuner fails.  A tuner that fails leaves the
+// context as it found it.
+struct TuningGuard {
+  cpx_ctx *c;
+  SegShape shape;
+  double alpha_scale;
+  uint32_t wheel_c;
+  bool tuned, keep = false;
+  explicit TuningGuard(cpx_ctx *ctx)
+      : c(ctx), shape(ctx->shape), alpha_scale(ctx->alpha_scale), wheel_c(ctx->opts.c), tuned(ctx->shape_tuned)
+  {
+  }
+  ~TuningGuard()
+  {
+    if (keep) return;
+    c->shape = shape;
+    c->alpha_scale = alpha_scale;
+    c->opts.c = wheel_c;
+    c->shape_tuned = tuned;
+  }
+};
+
 int cpx_autotune(cpx_ctx *c, const cpx_u128 *xs, size_t n, uint32_t *threads, uint32_t *kwords)
 {
   CTX_GUARD(c);
@@ -1091,6 +1112,7 @@ int cpx_autotune(cpx_ctx *c, const cpx_u128 *xs, size_t n, uint32_t *threads, ui
   };
   double best_ms = 1e300, ms = 0;
   SegShape best = c->shape;
+  TuningGuard guard(c);
   c->shape_tuned = true;                 // every trial runs the shape it names
   for (const SegShape &s : cands) {
     if (!seg_shape_supported(s) || seg_blocks_per_cu(s) < 1) continue;
@@ -1122,7 +1144,7 @@ int cpx_autotune(cpx_ctx *c, const cpx_u128 *xs, size_t n, uint32_t *threads, ui
     }
     c->opts.c = best_c;
   }
-  c->shape_tuned = true;
+  guard.keep = true;
   c->generation++;
   if (threads) *threads = (uint32_t)best.threads;
   if (kwords) *kwords = (uint32_t)best.kwords;

@@ -22,3 +22,33 @@ def test_noalloc_after_one_solve(x):
     import cudapix_amd as C
     with C.Context(device=0) as c:
         assert [c.pi(x)] == c.pi_batch_noalloc([x])
+
+
+def _lone_shape(c, x=10 ** 12):
+    st = c.pi_batch([x], stats=True)[1]
+    return st["seg_threads"], st["seg_kwords"]
+
+
+# a tuner that fails (an x it cannot plan, an allocation that fails) leaves the
+# context as it found it: its shape and factors, the lone query's own shape, and
+# a later tune that runs
+@pytest.mark.parametrize("how", ["range", "alloc 2", "alloc 9"])
+def test_failed_tune_leaves_the_context(how):
+    import cudapix_amd as C
+    xs = [10 ** 11, 10 ** 11 + 99, 10 ** 12]
+    with C.Context(device=0) as c:
+        before, lone = c.tuning(), _lone_shape(c)
+        assert lone != (before["seg_threads"], before["seg_kwords"])
+        for call in (c.autotune, lambda v: c.pi_batch(v, tune=True)):
+            try:
+                if how != "range":
+                    C.debug_fail_alloc(int(how.split()[1]))
+                with pytest.raises(C.CpxError):
+                    call(xs + [10 ** 30] if how == "range" else [100 * x for x in xs])
+            finally:
+                C.debug_fail_alloc(0)
+            assert c.tuning() == before and _lone_shape(c) == lone
+        want = [c.pi(x) for x in xs]
+        assert c.pi_batch(xs, tune=True) == want
+        t = c.tuning()
+        assert _lone_shape(c) == (t["seg_threads"], t["seg_kwords"])
