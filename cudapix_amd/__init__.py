@@ -90,7 +90,7 @@ class CpxServerStats(ctypes.Structure):
 # every symbol include/cudapix.h declares (checked by the CPU tests)
 EXPORTS = [
     "cpx_opts_default", "cpx_ctx_create", "cpx_ctx_destroy", "cpx_strerror",
-    "cpx_ctx_last_error", "cpx_choose_y", "cpx_ctx_device_bytes", "cpx_debug_fail_alloc",
+    "cpx_ctx_last_error", "cpx_choose_y", "cpx_ctx_device_bytes", "cpx_debug_fail_alloc", "cpx_debug_graph_captures",
     "cpx_pi_u64", "cpx_pi_u128",
     "cpx_p2_u64", "cpx_p2_u128", "cpx_div_x_by_y",
     "cpx_ordinary_u64", "cpx_ordinary_u128",
@@ -145,6 +145,7 @@ def lib():
         "cpx_choose_y": (ctypes.c_int, [vp, CpxU128, P(U64)]),
         "cpx_ctx_device_bytes": (U64, [vp]),
         "cpx_debug_fail_alloc": (ctypes.c_int, [ctypes.c_int]),
+        "cpx_debug_graph_captures": (U64, [vp]),
         "cpx_pi_u64": (ctypes.c_int, [vp, U64, U64, ctypes.c_uint32, P(U64), P(CpxTerms)]),
         "cpx_pi_u128": (ctypes.c_int, [vp, CpxU128, U64, ctypes.c_uint32, P(CpxU128), P(CpxTerms)]),
         "cpx_p2_u64": (ctypes.c_int, [vp, U64, U64, P(U64)]),
@@ -578,6 +579,10 @@ class Context:
         """Use a tuning (as returned by tuning()) without re-timing it."""
         self._chk(self._L.cpx_set_tuning(self.h, int(seg_threads), int(seg_kwords), float(alpha_scale),
                                          int(c)), "set_tuning")
+
+    def graph_captures(self):
+        """Test hook: how often the context has captured a batch slot's graphs."""
+        return self._L.cpx_debug_graph_captures(self.h)
 
     def request_bytes(self, x):
         return self._L.cpx_request_bytes(self.h, u128(x))

@@ -1178,6 +1178,13 @@ int cpx_get_tuning(cpx_ctx *c, uint32_t *threads, uint32_t *kwords, double *alph
   return CPX_OK;
 }
 
+uint64_t cpx_debug_graph_captures(cpx_ctx *c)
+{
+  if (!c) return 0;
+  std::lock_guard<std::recursive_mutex> g(c->mu);
+  return c->graph_captures;
+}
+
 uint64_t cpx_request_bytes(cpx_ctx *c, cpx_u128 x)
 {
   if (!c) return 0;

@@ -116,6 +116,7 @@ struct cpx_ctx {
   // blocks per CU) measured fastest for single queries to 1e16 on MI355X;
   // cpx_autotune may replace it for a batch
   SegShape shape{512, 32};
+  uint64_t graph_captures = 0;      // batches whose graphs were captured (a test reads it)
   bool shape_tuned = false;
   double alpha_scale = 1.0;                     // factor on the alpha model (autotuned)
 };

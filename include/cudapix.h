@@ -398,6 +398,9 @@ int cpx_probe_peaks(cpx_ctx *ctx, double *lds_bytes_per_s, double *int32_ops_per
  * a test can check the clean CPX_ENOMEM and that nothing leaks; 0 disarms.
  * Process-wide; for tests only. */
 int cpx_debug_fail_alloc(int n);
+/* How often the context has captured the graphs of a batch slot (a batch that
+ * finds its slot's graphs replays them); for tests only. */
+uint64_t cpx_debug_graph_captures(cpx_ctx *ctx);
 
 #ifdef __cplusplus
 }

@@ -52,3 +52,22 @@ def test_failed_tune_leaves_the_context(how):
         assert c.pi_batch(xs, tune=True) == want
         t = c.tuning()
         assert _lone_shape(c) == (t["seg_threads"], t["seg_kwords"])
+
+
+# lone queries between batches, with shapes of their own (below 2e15) and the
+# context's: every result as alone, and no graph captured again on the way
+def test_lone_queries_between_batches():
+    import cudapix_amd as C
+    many = [10 ** 11 + 12345 * k for k in range(20)]
+    lone = [10 ** 9, 10 ** 12 + 1, 3 * 10 ** 15, 10 ** 13 + 7]
+    with C.Context(device=0) as c:
+        want, alone = [c.pi(x) for x in many], [c.pi(x) for x in lone]
+        for x in lone:                           # tables and arena at their largest
+            c.pi_batch([x])
+        c.pi_batch(many)
+        n = c.graph_captures()
+        for _ in range(3):
+            for x, v in zip(lone, alone):
+                assert c.pi_batch([x]) == [v]
+                assert c.pi_batch(many) == want
+        assert c.graph_captures() == n
