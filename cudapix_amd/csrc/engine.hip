@@ -1416,10 +1416,12 @@ static int ensure_graph(cpx_ctx *c, BatchSlot &S, const BatchDev &b)
   return CPX_OK;
 }
 
-uint64_t plan_bytes_estimate(const cpx_ctx *c, const HostQuery &h)
+// Bytes of one query's state (plan and outputs) on its own in segments of
+// `shape`; an estimate that covers what its plan takes.
+static uint64_t state_bytes(const HostQuery &h, SegShape shape)
 {
   if (h.small) return 1024;
-  const double SI = (double)c->shape.seg_ints();
+  const double SI = (double)shape.seg_ints();
   // stages ~ pi(x^(1/4)) <= 1.26 n / ln n
   double q = (double)h.qrtx;
   double B = q < 3 ? 1 : 1.26 * q / std::log(q);
@@ -1446,6 +1448,35 @@ uint64_t plan_bytes_estimate(const cpx_ctx *c, const HostQuery &h)
   const double edesc = 4 + std::min(lookups / EASY_MIN, 2.0 * EASY_TILES) + lookups / EASY_WORK;
   double bytes = pairs * 8 * 1.5 + hseg * 48 + p2seg * 16 + 4096 + B * 80 + (h.y / 2048.0 + 32) * 48 + edesc * 64;
   return (uint64_t)bytes;
+}
+
+uint64_t plan_bytes_estimate(const cpx_ctx *c, const HostQuery &h) { return state_bytes(h, c->shape); }
+
+// A lone query's own segment shape.  One small query does not fill the chip with
+// 512-thread segments: half-size blocks (256 x 32 words) give it twice the tiles
+// and end sooner (1e12: 0.56 against 0.61 ms, 1e15: 1.59 against 1.85; 2e15 even,
+// 4e15: 3.42 against 2.99).  A shape the caller or the tuner chose stays, and the
+// context's stays where a server's budget does not hold the longer rows.
+static const uint64_t SMALL_SHAPE_X = 2000000000000000ull;
+static const SegShape SMALL_SHAPE{256, 32};
+
+static bool lone_shape(const cpx_ctx *c, const HostQuery &h)
+{
+  return !c->shape_tuned && h.x < SMALL_SHAPE_X &&
+         (!c->state_budget || state_bytes(h, SMALL_SHAPE) <= c->state_budget);
+}
+
+// Bytes of a batch of n queries whose plan_bytes_estimates add up to `sum`, the
+// largest x's fourth root qrt: several queries share replicas of their leaf-dense
+// segments, each replica with a row of sum(mu) for every member.  The planner
+// makes a replica of 16 K leaf candidates or of 1 / 640 of the batch's work at
+// least, so about 640 of them, in groups of GROUP_SMALL (in larger groups of more
+// work the single queries' margins cover them).
+uint64_t batch_bytes_estimate(const cpx_ctx *c, uint64_t sum, size_t n, const HostQuery &largest)
+{
+  if (n < 2) return !largest.small && lone_shape(c, largest) ? state_bytes(largest, SMALL_SHAPE) : sum;
+  const double q = (double)largest.qrtx, B = q < 3 ? 1 : 1.26 * q / std::log(q);
+  return sum + (uint64_t)(640.0 * (24 + (double)std::min<size_t>(n, GROUP_SMALL) * (4 * B + 20)));
 }
 
 // P2 by lookups in a resident pi table to x/(y+1) (instead of sieving the
@@ -1580,20 +1611,15 @@ static int launch_passes(cpx_ctx *c, BatchSlot &S, const Plan &pl, const PassPla
   return CPX_OK;
 }
 
-// The segment shape of a solve, for the length of a scope.  One small query on
-// its own does not fill the chip with 512-thread segments: half-size blocks
-// (256 x 32 words) give it twice the tiles and end sooner (1e12: 0.56 against
-// 0.61 ms, 1e15: 1.59 against 1.85; 2e15 even, 4e15: 3.42 against 2.99).  A
-// shape the caller or the tuner chose stays.
-static const uint64_t SMALL_SHAPE_X = 2000000000000000ull;
+// The segment shape of a solve, for the length of a scope.
 struct ShapeScope {
   cpx_ctx *c;
   SegShape keep;
   bool own;                              // not the context's shape
   ShapeScope(cpx_ctx *ctx, const std::vector<HostQuery> &hq)
-      : c(ctx), keep(ctx->shape), own(!ctx->shape_tuned && hq.size() == 1 && hq[0].x < SMALL_SHAPE_X)
+      : c(ctx), keep(ctx->shape), own(hq.size() == 1 && lone_shape(ctx, hq[0]))
   {
-    if (own) c->shape = SegShape{256, 32};
+    if (own) c->shape = SMALL_SHAPE;
   }
   ~ShapeScope() { c->shape = keep; }
 };

@@ -116,6 +116,7 @@ struct cpx_ctx {
   // blocks per CU) measured fastest for single queries to 1e16 on MI355X;
   // cpx_autotune may replace it for a batch
   SegShape shape{512, 32};
+  uint64_t state_budget = 0;        // of a batch-mode server: bytes of one batch's state (0: none)
   uint64_t graph_captures = 0;      // batches whose graphs were captured (a test reads it)
   bool shape_tuned = false;
   double alpha_scale = 1.0;                     // factor on the alpha model (autotuned)
@@ -150,6 +151,7 @@ void free_slots(cpx_ctx *c);
 uint64_t slot_bytes(const cpx_ctx *c);
 uint64_t host_pi(const cpx_ctx *c, uint64_t v);   // v <= prime_limit
 uint64_t plan_bytes_estimate(const cpx_ctx *c, const HostQuery &hq);
+uint64_t batch_bytes_estimate(const cpx_ctx *c, uint64_t sum, size_t n, const HostQuery &largest);
 void free_tables(cpx_ctx *c);
 
 // ---- streaming cohorts (the server's continuous-batching launch)

@@ -472,7 +472,8 @@ static void batch_dispatcher(cpx_server *s)
       continue;
     }
     grp.clear();
-    uint64_t gbytes = 0;
+    uint64_t gsum = 0, gbytes = 0;       // the requests' own estimates, and the batch's
+    HostQuery top{};
     while (!s->pending.empty() && grp.size() < s->opts.max_batch) {
       const Req r = s->pending.front();
       if (r.cancelled) {                 // its result was reported by the cancel
@@ -489,8 +490,12 @@ static void batch_dispatcher(cpx_server *s)
         finish(s, r, {0, 0}, rc, now, now);
         continue;
       }
-      if (!grp.empty() && gbytes + b > s->budget) break;
-      gbytes += b;
+      const HostQuery &most = h.x > top.x ? h : top;
+      const uint64_t all = batch_bytes_estimate(s->lane, gsum + b, grp.size() + 1, most);
+      if (!grp.empty() && all > s->budget) break;
+      gsum += b;
+      gbytes = all;
+      top = most;
       grp.push_back(r);
       s->state[r.ticket] = 1;
       s->pending.pop_front();
@@ -562,6 +567,7 @@ int cpx_server_create(cpx_ctx *c, const cpx_server_opts *o, cpx_server **out)
   }
   cpx_ctx *lc = s->lane;
   if (s->opts.mode == CPX_SERVER_BATCHES) {
+    lc->state_budget = s->budget;
     // tables (with P2 lookups) for the largest x announced
     const u128 mx = ((u128)s->opts.max_x.hi << 64) | s->opts.max_x.lo;
     if (mx >= CPX_SMALL_X) {

@@ -71,3 +71,19 @@ def test_lone_queries_between_batches():
                 assert c.pi_batch([x]) == [v]
                 assert c.pi_batch(many) == want
         assert c.graph_captures() == n
+
+
+# a batch-mode server whose budget holds a lone request's state in the context's shape
+# only, and one that holds a few requests of a burst at a time
+@pytest.mark.parametrize("xs,budget,least", [([10 ** 15], 3600000, 1), ([10 ** 12 + 3 ** k for k in range(24)], 2500000, 2)])
+def test_batch_server_within_its_budget(ctx, xs, budget, least):
+    import cudapix_amd as C
+    with C.Context(device=0) as c:
+        srv = C.Server(c, hbm_budget=budget, mode=C.SERVER_BATCHES)
+        tickets = [srv.submit(x) for x in xs]
+        srv.drain()
+        res = {r["ticket"]: r for r in srv.poll(100)}
+        st = srv.stats()
+        srv.close()
+    assert [(res[t]["status"], res[t]["pi"]) for t in tickets] == [(0, ctx.pi(x)) for x in xs]
+    assert st["max_inflight_bytes"] <= budget and st["batches"] >= least and st["rejected"] == 0

@@ -58,3 +58,29 @@ def test_needs_in_every_shape(checker, x):
     shapes = ["64x32", "64x128", "128x64", "256x32", "256x128", "512x32", "512x64"]
     r = run(checker, ["needs %d" % x, "needs %d %d" % (x, x)] + ["needs shape=%s %d" % (s, x) for s in shapes])
     assert all(v == r[0] for v in r), r
+
+
+# what a batch-mode server admits a batch by covers what the batch's plan takes: lone
+# queries in the shape they run in, batches of every size over the served range
+@pytest.mark.parametrize("tuning", ["", "alpha=0.3 c=8", "shape=256x32", "shape=64x32", "shape=512x64 alpha=0.5"])
+def test_estimate_covers_the_plan(checker, tuning):
+    lists = [[int(10 ** (e / 4))] for e in range(18, 66)] + [[2 * 10 ** 15 - 1], [5], [16384]]
+    for n in (2, 3, 4, 6, 8, 9, 12, 16, 24, 32, 33, 48, 64, 100, 256):
+        for lo, hi in ((5, 9), (9, 10), (9, 11), (11, 12), (12, 13), (9, 13), (13, 14), (9, 14), (14, 15), (9, 15),
+                       (9, 16)):
+            if n * 10 ** hi <= 2 * 10 ** 17:
+                lists.append(spread(n, n, lo, hi))
+    for tables in (0, 1):
+        lines = ["bytes tables=%d %s %s" % (tables, tuning, " ".join(map(str, xs))) for xs in lists
+                 if max(xs) < 10 ** 15 or not tables]
+        for ln, (need, est) in zip(lines, run(checker, lines)):
+            assert int(need) <= int(est), (ln[:80], need, est)
+
+
+# a lone query keeps the context's shape where the budget holds its state in that one only
+def test_lone_shape_within_budget(checker):
+    for x in (10 ** 12, 10 ** 13, 10 ** 14, 10 ** 15):
+        free, one = (list(map(int, r)) for r in run(checker, ["bytes %d" % x, "bytes shape=512x32 %d" % x]))
+        assert one[1] < free[1]
+        tight = list(map(int, run(checker, ["bytes budget=%d %d" % ((free[1] + one[1]) // 2, x)])[0]))
+        assert tight == one, (x, free, one, tight)
