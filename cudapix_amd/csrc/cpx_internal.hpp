@@ -81,12 +81,10 @@ struct QueryDev {
   uint64_t pi_sqrtx;                  // written by setup: pi(sqrt x)
 };
 
-// One stage of the hard-leaf sieve: p_b, floor(x / p_b) and constants that
-// turn the per-stage divisions into multiplications (computed once per query).
+// One stage of the hard-leaf sieve: p_b and the quotients by it, divided once
+// per query.
 struct StageDev {
   uint64_t xp;         // floor(x / p), low 64 bits
-  double inv_p;        // 1 / p rounded to f64
-  uint64_t magic;      // ceil(2^64 / p): a mod p for 32-bit a (Lemire, Kaser, Kurz 2019)
   uint32_t p;
   uint32_t ylo;        // floor(y / p)
   uint32_t xph;        // floor(x / p) >> 64 (nonzero only for the first stages of x above 2^68)
@@ -126,13 +124,6 @@ __host__ __device__ __forceinline__ uint64_t cpx_div_recip_w(uint64_t al, uint32
 __host__ __device__ __forceinline__ bool cpx_quot_below_2_50(uint64_t al, uint32_t ah, uint64_t d)
 {
   return ((((uint64_t)ah) << 14) | (al >> 50)) < d;
-}
-
-// a mod p for 32-bit a with magic = ceil(2^64 / p).
-__host__ __device__ __forceinline__ uint32_t cpx_fastmod32(uint32_t a, uint32_t p, uint64_t magic)
-{
-  uint64_t low = magic * a;
-  return (uint32_t)(((u128)low * p) >> 64);
 }
 
 // Queries of a batch that share one sieve of each segment: a tile sieves its

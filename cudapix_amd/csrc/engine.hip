@@ -1287,8 +1287,6 @@ static void pack_stages(const cpx_ctx *c, const Layout &L, const Plan &pl, char 
       StageDev d;
       d.p = p;
       d.ylo = (uint32_t)(q.y / p);
-      d.inv_p = 1.0 / (double)p;
-      d.magic = ~0ull / p + 1;
       const u128 xq = x / p;
       d.xp = (uint64_t)xq;
       d.xph = (uint32_t)(xq >> 64);

@@ -39,8 +39,6 @@ static __device__ __forceinline__ void setup_query(const BatchDev &bd, uint32_t 
     StageDev d;
     d.p = p;
     d.ylo = (uint32_t)(q.y / p);
-    d.inv_p = 1.0 / (double)p;
-    d.magic = ~0ull / p + 1;
     uint64_t rem;
     const u128 xq = cpx_div128_64(x, p, &rem);
     d.xp = (uint64_t)xq;
