@@ -9,6 +9,9 @@
 //                    reach the end of its last P2 segment in the context's shape
 //   bytes x x ...    "bytes <state> <estimate>": what the batch's plan takes and what
 //                    a batch-mode server admits it by (tables=1: P2 by lookups)
+//   check x x ...    "check <tiles>": check_plan's conditions, and that the wheel-stage
+//                    descriptors cover their odd m, every partial sum has one
+//                    descriptor, and the carry descriptors name their rows
 #define main planner_check_main
 #include "planner_check.cpp"
 #undef main
@@ -25,6 +28,48 @@ static void plan_into(cpx_ctx *c, Cmd &cmd, Plan &pl, uint32_t p2mode = 0)
   for (const HostQuery &h : cmd.hq) plan_needs(c, h, TERM_ALL, c->shape.seg_bits(), &R, &P, &Y);
   fake_tables(c, R, P, Y);
   CHECK(build_plan(c, cmd.hq, TERM_ALL, pl) == CPX_OK, "build_plan");
+}
+
+static void check_descriptors(const cpx_ctx *c, const Plan &pl, const Caps &k)
+{
+  for (size_t i = 0; i < pl.q.size(); i++) {
+    const QueryDev &d = pl.q[i];
+    const QPlan &qp = pl.qps[i];
+    std::vector<int> used(qp.parts, 0);
+    for (const std::vector<BlockDesc> *v : {&qp.ord, &qp.triv, &qp.easy, &qp.fin, &qp.dir, &qp.p2d})
+      for (const BlockDesc &b : *v) {
+        CHECK(b.query == i && b.part < qp.parts, "descriptor's query and part");
+        used[b.part]++;
+      }
+    for (int n : used) CHECK(n == 1, "one descriptor a partial sum");
+    if (d.small) continue;
+    CHECK(d.c <= d.cs && d.cs + d.nstage <= c->nprimes, "stages inside the prime list");
+    const uint32_t h0 = d.n_ord_parts + d.n_triv_parts + d.n_easy_parts, h1 = h0 + d.n_hard_parts;
+    if (d.cs > d.c) {
+      uint64_t at = d.y / c->h_primes[d.cs - 1] / 2;      // odd m = 2i + 1 from here
+      for (const BlockDesc &b : qp.dir) {
+        CHECK(b.part >= h0 && b.part < h1, "wheel stages among the hard parts");
+        CHECK(b.begin == at && b.end > b.begin, "wheel-stage ranges adjoin");
+        at = b.end;
+      }
+      CHECK(at == (d.y + 1) / 2, "wheel stages to y");
+    } else {
+      CHECK(qp.dir.empty(), "no wheel stages");
+    }
+    uint64_t st = 0;
+    for (const BlockDesc &b : qp.fin) {
+      const uint64_t s0 = (uint32_t)b.begin;
+      CHECK(b.part >= h0 && b.part < h1, "carry among the hard parts");
+      CHECK(s0 == st && b.end > s0 && b.end - s0 <= CPX_FIN_STAGES, "carry stages adjoin");
+      st = b.end;
+      uint64_t rows = 0;
+      while (rows < d.hard_nseg && qp.rowinfo[rows].act > s0) rows++;
+      CHECK(b.begin >> 32 == rows, "rows of a carry descriptor");
+    }
+    CHECK(st == d.nstage, "carry of every stage");
+    for (uint64_t s = d.p2_seg0; s < d.p2_seg0 + d.p2_nseg; s++)
+      CHECK(d.mrow_base + qp.rowinfo[s].mrow + qp.rowinfo[s].nrep <= k.mrows, "P2 outputs of every replica");
+  }
 }
 
 int main()
@@ -70,6 +115,19 @@ int main()
       std::printf("groups");
       for (const GroupDev &g : pl.groups) std::printf(" %u", g.n);
       std::printf("\n");
+    } else if (cmd.what == "check") {
+      if (tables) fake_tables(c, cmd.hq[0].zt, cmd.hq[0].sqrtx, cmd.hq[0].y);
+      const ShapeScope scope(c, cmd.hq);
+      Plan pl;
+      plan_into(c, cmd, pl);
+      Caps k{};
+      grown_caps(Caps{}, needed_caps(pl), k);
+      const Layout L = make_layout(k);
+      std::vector<char> image(L.plan_bytes);
+      pack_plan(L, pl, image.data());
+      check_plan(c, pl, L, k, false);
+      check_descriptors(c, pl, k);
+      std::printf("check %zu\n", pl.tiles.size());
     } else if (cmd.what == "bytes") {
       uint64_t sum = 0, top = 0;
       for (size_t i = 0; i < cmd.hq.size(); i++) {

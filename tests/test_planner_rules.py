@@ -84,3 +84,15 @@ def test_lone_shape_within_budget(checker):
         assert one[1] < free[1]
         tight = list(map(int, run(checker, ["bytes budget=%d %d" % ((free[1] + one[1]) // 2, x)])[0]))
         assert tight == one, (x, free, one, tight)
+
+
+# every descriptor list of the plan, at every wheel (x^(1/4) about 11 .. 29) with every c,
+# in the lone query's shape and the context's, in batches and in other shapes
+def test_descriptors(checker):
+    small = [5, 16384, 28560, 28561, 83520, 83521, 130320, 130321, 279840, 279841, 707281]
+    lines = ["check c=%d %d" % (c, x) for c in range(1, 9) for x in small[1:] + [10 ** 9, 10 ** 13]]
+    lines += ["check %d" % int(10 ** (e / 2)) for e in range(9, 35)] + ["check tables=1 %d" % 10 ** 12]
+    for n, lo, hi in ((2, 5, 9), (7, 9, 13), (8, 9, 13), (33, 4, 12), (64, 9, 14), (40, 13, 15)):
+        xs = " ".join(map(str, spread(n, n, lo, hi) + small[:3]))
+        lines += ["check %s %s" % (t, xs) for t in ("", "alpha=0.3 c=8", "c=1", "shape=64x32", "shape=512x64")]
+    run(checker, lines)
