@@ -68,7 +68,7 @@ def primes_upto(n):
     return np.nonzero(s)[0]
 
 
-GROUP = 32  # queries per shared segment sieve (the library's group capacity)
+GROUP = 32  # queries per shared segment sieve (in a batch of much work, as here; 8 in a small one)
 
 # Tuning of the batched runs (segment threads, words per thread, alpha factor,
 # wheel primes): the fastest of the autotuner's choices on the 512-query
@@ -166,8 +166,8 @@ def hbm_model_bytes(terms, primes, seg_bits):
     """W_HBM of one batch launch (a model, labelled as such): 8 B per hard-leaf
     candidate of the sieved stages (the leaf table's entry of each m coprime to
     30030 in (y/p, y]), 4 B when p^2 > y (the prime list's entry), 8 B per
-    easy-leaf pair (one pi-table entry; pairs above sqrt(x/p) are counted from
-    the smaller side with fewer), 8 B per P2 prime (one pi-table entry at x/p),
+    easy-leaf pair p < q <= min(y, x/p^2, sqrt(x/p)) (one pi-table entry; the pairs
+    above sqrt(x/p) are counted from these), 8 B per P2 prime (one pi-table entry at x/p),
     and 4 B per pattern word filled into each segment of each query group
     (seg_bits integers coprime to 30 per segment; replicas of a segment not
     counted).  Tables are resident and
@@ -186,7 +186,7 @@ def hbm_model_bytes(terms, primes, seg_bits):
         for p in ps[ps * ps > y]:
             l_hard += max(0, pi_at(y) - pi_at(max(int(p), y // int(p))))
         for p in primes[pi_at(q4):pi_at(c3)]:
-            hi = min(y, x // (int(p) * int(p)))
+            hi = min(y, x // (int(p) * int(p)), math.isqrt(x // int(p)))
             if hi > p:
                 l_easy += pi_at(hi) - pi_at(int(p))
         n_p2 += max(0, pi_at(sq) - pi_at(y))
