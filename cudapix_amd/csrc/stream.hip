@@ -151,21 +151,6 @@ static __device__ __forceinline__ bool claim_fifo(uint64_t *head, uint64_t end, 
   }
 }
 
-// Main tiles a block claims at once: every block contends for the one head
-// (each claim a compare-and-swap at device scope), so while many tiles are
-// left a claim takes a run of up to 16 consecutive tiles (1 near the end,
-// where the longest-first order leaves the short tiles to balance the grid).
-// Half a share of what is left: longer runs serve a burst sooner but hold up the
-// cohorts that join behind a large query's long tiles (a burst of 100 requests
-// below 1e14 takes 13 ms with two shares, 18.6 with a half, 23 with a quarter;
-// 200 requests/s with x < 1e17 wait 276 and 166 ms on average, 100 and 118, and
-// 66 and 112, in two runs each).
-static __device__ __forceinline__ uint64_t main_claim_run(uint64_t left)
-{
-  const uint64_t k = left / (2ull * gridDim.x);
-  return k < 1 ? 1 : (k > 16 ? 16 : k);
-}
-
 // Thread 0: the block's next unit of work, in priority order.  A claimed run
 // of main tiles [v, v + n) comes back as its first tile, with *run_next and
 // *run_end set to the rest (the caller takes those before looking again).
@@ -208,7 +193,7 @@ static __device__ __attribute__((noinline)) void stream_find(const StreamArgs &a
     }
   uint64_t n = 1;
   const uint64_t h0 = ld_dev(&ctl->main_head);
-  if (claim_fifo(&ctl->main_head, me, &v, main_claim_run(me > h0 ? me - h0 : 0), &n)) {
+  if (claim_fifo(&ctl->main_head, me, &v, cpx_main_claim_run(me > h0 ? me - h0 : 0, gridDim.x), &n)) {
     st_sys(&a.mb->main_claimed, v + n);
     *run_next = v + 1;
     *run_end = v + n;

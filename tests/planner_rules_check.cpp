@@ -9,12 +9,14 @@
 //                    reach the end of its last P2 segment in the context's shape
 //   bytes x x ...    "bytes <state> <estimate>": what the batch's plan takes and what
 //                    a batch-mode server admits it by (tables=1: P2 by lookups)
+//   claim left grid  "claim <tiles>": main tiles a streaming block claims at once
 //   check x x ...    "check <tiles>": check_plan's conditions, and that the wheel-stage
 //                    descriptors cover their odd m, every partial sum has one
 //                    descriptor, and the carry descriptors name their rows
 #define main planner_check_main
 #include "planner_check.cpp"
 #undef main
+#include "../cudapix_amd/csrc/cpx_stream.hpp"
 
 struct Cmd {
   std::string what;
@@ -92,6 +94,14 @@ int main()
     Cmd cmd;
     bool tables = false;
     in >> cmd.what;
+    if (cmd.what == "claim") {
+      uint64_t left;
+      uint32_t grid;
+      in >> left >> grid;
+      std::printf("claim %llu\n", (unsigned long long)cpx_main_claim_run(left, grid));
+      primes.swap(c->h_primes);
+      continue;
+    }
     std::string tok;
     while (in >> tok) {
       const size_t eq = tok.find('=');
