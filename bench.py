@@ -340,7 +340,10 @@ def configs_run(args):
         x = 10 ** 12
         y = 2 * icbrt(x)
         ms, t = timed(cx, x, y, args.reps)
-        print("| C1 | 1e12 | 2 | %d | 2^19 (512 x 32) | %.2f | %d |" % (y, ms, t["pi"]), flush=True)
+        st = cx.pi_batch([x], stats=True)[1]          # the shape a lone query of this size takes
+        shape = (st["seg_threads"], st["seg_kwords"])
+        print("| C1 | 1e12 | 2 | %d | 2^%d (%d x %d) | %.2f | %d |"
+              % (y, round(math.log2(32 * shape[0] * shape[1])), shape[0], shape[1], ms, t["pi"]), flush=True)
     for shape in ((256, 32), (512, 32), (512, 64), (256, 128)):
         bits = 32 * shape[0] * shape[1]
         with C.Context(device=0, seg_threads=shape[0], seg_kwords=shape[1]) as cx:
@@ -362,7 +365,10 @@ def configs_run(args):
 def profile_run(args):
     """One workload only, for profiler runs: `single` = pi(x) on a warm
     context (default shape), `batch` = the 512-query batched step (with
-    --tuning as the timed run's autotune chose it), `copy` = a
+    --tuning as the timed run's autotune chose it), `fresh` = pi(x) with every
+    table rebuilt, a term's name = that term of x at y = 2.5 cbrt(x), `count` =
+    the primes of [x, x + 2^32), `burst` = 100 requests in [1e9, 1e14] to a
+    streaming server, `copy` = a
     device-to-device copy of --copy-mib MiB (the byte-counter calibration),
     `probe` = the LDS and VALU peak microbenchmarks."""
     if args.profile == "copy":
@@ -378,7 +384,39 @@ def profile_run(args):
         print(json.dumps({"profile": "copy", "bytes": n, "reps": args.reps}), flush=True)
         return
     import cudapix_amd as C
-    ctx = C.Context(device=0)
+    ctx = C.Context(device=0, fresh_tables=args.profile == "fresh")
+    if args.profile in ("fresh", "P2", "Ordinary", "S2_trivial", "S3", "V", "count", "burst"):
+        x, what, srv = int(args.x), args.profile, None
+        y = int(2.5 * iroot(x, 3))
+        if what == "burst":
+            import random
+            r = random.Random(1)
+            xs = [int(10 ** r.uniform(9, 14)) for _ in range(100)]
+            srv = C.Server(ctx, max_batch=512, mode=C.SERVER_STREAM, max_x=10 ** 14 + 1)
+
+        def call():
+            if what == "fresh":
+                return ctx.pi(x)
+            if what == "count":
+                return ctx.countPrimes(x, x + (1 << 32))
+            if what == "burst":
+                for v in xs:
+                    srv.submit(v)
+                srv.drain()
+                return len(srv.poll(200))
+            return getattr(ctx, what)(x, y)
+        call()
+        us = []
+        for _ in range(args.reps):
+            t0 = time.time()
+            v = call()
+            us.append((time.time() - t0) * 1e6)
+        print(json.dumps({"profile": what, "x": x, "value": v, "median_us": round(sorted(us)[len(us) // 2], 1)}),
+              flush=True)
+        if srv:
+            srv.close()
+        ctx.close()
+        return
     if args.profile == "probe":
         for _ in range(args.reps):
             lds, valu = ctx.probe_peaks()
@@ -434,7 +472,8 @@ def main():
     ap.add_argument("--serve-xmax", type=float, default=1e16)
     ap.add_argument("--serve-full", action="store_true",
                     help="every stream of the served fixture: lambda 50..2000, 2000 requests, x < 1e17")
-    ap.add_argument("--profile", choices=["single", "batch", "copy", "probe"],
+    ap.add_argument("--profile", choices=["single", "batch", "copy", "probe", "fresh", "P2", "Ordinary", "S2_trivial",
+                                          "S3", "V", "count", "burst"],
                     help="run only one workload --reps times (for rocprofv3) and exit")
     ap.add_argument("--x", type=float, default=1e16, help="x of --profile single")
     ap.add_argument("--reps", type=int, default=3)

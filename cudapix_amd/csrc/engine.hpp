@@ -113,8 +113,8 @@ struct cpx_ctx {
   uint64_t generation = 0;                      // bumps when a table is reallocated
 
   // segment-kernel shape: 512 threads x 32 words (2^19-bit segments, two
-  // blocks per CU) measured fastest for single queries to 1e16 on MI355X;
-  // cpx_autotune may replace it for a batch
+  // blocks per CU) measured fastest for batches and for single queries from
+  // 2e15 (smaller ones take their own, lone_shape); cpx_autotune may replace it
   SegShape shape{512, 32};
   uint64_t state_budget = 0;        // of a batch-mode server: bytes of one batch's state (0: none)
   uint64_t graph_captures = 0;      // batches whose graphs were captured (a test reads it)

@@ -577,7 +577,7 @@ __device__ __forceinline__ void p2_epilogue(const BatchDev &bd, const GroupDev &
 // wave about 50 instructions to find the lanes' first multiples.)
 //
 // Bound by VALU issue: at x = 1e17 the SIMDs have a VALU instruction in flight
-// 87 % of the time (7.5e9 of them in 14.6 ms, 4 cycles each), so what counts is
+// 78 % of the time (6.1e9 of them in 13.4 ms, 4 cycles each), so what counts is
 // instructions per (wave, stage).  Against odd-only bits, own-bits crossing,
 // candidates from every odd m and groups of 8, the layout above took two
 // 512-query batches to 1e15 from 64.2 to 35.5 ms, 1e16 from 7.7 to 5.4 ms, 1e18

@@ -523,8 +523,9 @@ hipError_t launch_count_range(const PiEntry *tab, uint64_t lo, uint64_t hi,
 //   below 2^18     by one lane, class after class;
 //   above          by one lane, multiple after multiple (at most 15 of them,
 //                  of which those coprime to 30 are crossed).
-// Bound by the work per (prime, segment) once the primes outnumber the
-// segment's integers (664,000 of them at 1e14): hence one block of 1024
+// Bound by VALU issue (an instruction in flight in 75 % of the SIMD cycles, LDS
+// bank conflicts in 5.5 %), and by the work per (prime, segment) once a prime has
+// few multiples in a segment (664,000 primes at 1e14): hence one block of 1024
 // threads per CU with all of its LDS, 4.9e6 integers.  2^32 integers at 1e14:
 // 12.1 -> 3.2 ms, against 2^19 odd bits per block and a 64-bit remainder per
 // prime (1e15: 50 -> 8.8 ms for 6e9 integers, 4.5 -> 1.6 ms for 1e6).
