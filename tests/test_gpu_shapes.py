@@ -87,3 +87,15 @@ def test_batch_server_within_its_budget(ctx, xs, budget, least):
         srv.close()
     assert [(res[t]["status"], res[t]["pi"]) for t in tickets] == [(0, ctx.pi(x)) for x in xs]
     assert st["max_inflight_bytes"] <= budget and st["batches"] >= least and st["rejected"] == 0
+
+
+# a wave of the shape with the longest waves crosses off more than 2^16 integers a stage if
+# the caller's wheel leaves it the stages of 3 and 5 (the sieve's own wheel does not)
+@pytest.mark.parametrize("c", [1, 2, 4])
+@pytest.mark.parametrize("x", [10 ** 9 + 7, 10715741739, 26496490190])
+def test_small_wheels_in_the_longest_wave(oracle, x, c):
+    import cudapix_amd as C
+    with C.Context(device=0, seg_threads=64, seg_kwords=128) as k:
+        t = k.pi(x, c=c, terms=True)
+        ref = oracle.pi_dr(x, t["y"], int(t["c"]))
+        assert [t[n] for n in ("hard", "p2", "pi")] == [ref[n] for n in ("hard", "p2", "pi")]
