@@ -695,17 +695,20 @@ static const double STAGE_LEAVES = 143.0, REP_SIEVE = 16.0;
 // 3.96 / 5.12 (1.7e8); with alpha factor 0.3 and c = 8, 512 in [1e9, 1e13] 3.40 /
 // 3.86 (1.7e8), 512 in [1e11, 1e13] 4.98 / 4.56 (3.2e8), 512 in [1e9, 1e14] 7.17 /
 // 6.98 (7.8e8), 512 in [1e9, 1e15] 21.4 / 16.8 (3.7e9).
-static const double GROUP_WORK = 2.4e8;
+// Segments of 2^20 bits, whose blocks have a CU each, gain from larger groups
+// sooner: 64 queries in [1e9, 1e13] 1.33 / 1.59 (1.3e7), 128 of them 2.14 / 2.00
+// (2.7e7) in 512 x 64, 1.67 / 1.93 and 2.63 / 2.50 in 256 x 128.
+static const double GROUP_WORK = 2.4e8, GROUP_WORK_LONG = 2.4e7;
 static const uint32_t GROUP_SMALL = 8;
 
-static uint32_t group_members(const std::vector<QPlan> &qps)
+static uint32_t group_members(const cpx_ctx *c, const std::vector<QPlan> &qps)
 {
   double work = 0;
   for (const QPlan &qp : qps) {
     for (float l : qp.rleaves) work += l;
     work += STAGE_LEAVES * (double)qp.tm;
   }
-  return work < GROUP_WORK ? GROUP_SMALL : CPX_GROUP;
+  return work < (c->shape.seg_bits() > (1u << 19) ? GROUP_WORK_LONG : GROUP_WORK) ? GROUP_SMALL : CPX_GROUP;
 }
 
 // Groups of queries that share the segment sieve: queries with hard rows,
@@ -941,7 +944,7 @@ static int build_plan(cpx_ctx *c, const std::vector<HostQuery> &hq, uint32_t mas
   const unsigned nt = plan_threads(nq);
   parallel_for(nq, nt, [&](size_t i) { plan_query(c, hq[i], (uint32_t)(B.q + i), mask, qps[i], nq); });
   pl.groups.clear();
-  make_groups(c, hq, qps, group_members(qps), pl.groups);
+  make_groups(c, hq, qps, group_members(c, qps), pl.groups);
   // leaves of one tile (a segment with more becomes replicas): 16 K at least,
   // 512 K at most, between them four fifths of the work of one of 512 blocks,
   // so that no tile outlasts the others' work and none is sieved more often

@@ -44,7 +44,8 @@ def spread(seed, n, lo, hi):
     (64, 9, 13, "", 8), (128, 9, 13, "", 8), (512, 9, 12, "", 8), (512, 9, 13, "", 8), (64, 12, 13, "", 8),
     (128, 9, 13, "alpha=0.3 c=8", 8), (512, 9, 12, "alpha=0.3 c=8", 8), (64, 12, 13, "alpha=0.3 c=8", 8),
     (512, 9, 15, "", 32), (512, 9, 15, "alpha=0.3 c=8", 32), (64, 14, 15, "alpha=0.3 c=8", 32),
-    (256, 14, 15, "", 32)])
+    (256, 14, 15, "", 32), (64, 9, 13, "shape=512x64", 8), (128, 9, 13, "shape=512x64", 32),
+    (128, 9, 13, "shape=256x128", 32), (128, 9, 13, "shape=256x64", 8)])
 def test_group_members(checker, n, lo, hi, tuning, most):
     xs = spread(n, n, lo, hi)
     sizes = list(map(int, run(checker, ["groups %s %s" % (tuning, " ".join(map(str, xs)))])[0]))
