@@ -109,19 +109,21 @@ struct StreamArgs {
 };
 
 // Main tiles a block claims at once, of `left` in the FIFO: every block contends
-// for the one head (each claim a compare-and-swap at device scope), so while many
-// tiles are left a claim takes a run of up to 4 consecutive tiles, half a block's
-// share, and 1 near the end, where the longest-first order leaves the short tiles
-// to balance the grid.  A longer run holds up the cohorts that join behind a large
-// query's tiles, which are long themselves (1,966,080 integers, up to 512 K leaves
-// or more); a shorter one makes the claims the cost.  Runs of at most 2, 4, 8 and
-// 16: 200 requests/s with x < 1e17 wait 34, 25, 31 and 71 ms on average (99 %
-// within 103, 91, 111 and 276), 2000 with x < 1e16 97, 30, 50 and 69 ms; at
-// capacity 3038, 6133, 5719 and 5748 requests/s; a burst of 100 below 1e14 takes
-// 18.6, 16.6, 16.5 and 16.0 ms.
+// for the one head (each claim a compare-and-swap at device scope, about one
+// succeeding every 2 us), so while many tiles are left a claim takes a run of up
+// to 4 consecutive tiles, a block's share at most, and 1 near the end, where the
+// longest-first order leaves the short tiles to balance the grid.  A longer run
+// holds up the cohorts that join behind a large query's tiles, which are long
+// themselves (1,966,080 integers, up to 512 K leaves or more); a shorter one makes
+// the claims the cost.  Runs of at most 2, 4, 8 and 16 and half a share: 200
+// requests/s with x < 1e17 wait 34, 25, 31 and 71 ms on average (99 % within 103,
+// 91, 111 and 276), 2000 with x < 1e16 97, 30, 50 and 69 ms; at capacity 3038,
+// 6133, 5719 and 5748 requests/s.  A whole share instead of half, at most 4: 21 (89),
+// 27 ms and 5770/s; a request of 1e14 on its own 5.0 ms instead of 6.4, a burst of
+// 100 below 1e14 12.9 ms instead of 16.6; a quarter: 31 (90), 54 ms, 5668/s, 23 ms.
 __host__ __device__ inline uint64_t cpx_main_claim_run(uint64_t left, uint32_t grid)
 {
-  const uint64_t k = left / (2ull * grid);
+  const uint64_t k = left / grid;
   return k < 1 ? 1 : (k > 4 ? 4 : k);
 }
 

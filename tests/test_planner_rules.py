@@ -99,9 +99,9 @@ def test_descriptors(checker):
     run(checker, lines)
 
 
-# a block of the streaming launch claims half its share of the main tiles, at most four (a
-# cohort that joins waits for the tiles already claimed) and one near the end
+# a block of the streaming launch claims its share of the main tiles, at most four (a cohort
+# that joins waits for the tiles already claimed) and one near the end
 def test_streaming_claims(checker):
-    lefts = [0, 1, 511, 512, 1023, 1024, 2048, 3072, 4096, 5000, 10 ** 5, 10 ** 7]
+    lefts = [0, 1, 511, 512, 1023, 1024, 1536, 2047, 2048, 5000, 10 ** 5, 10 ** 7]
     r = [int(v[0]) for v in run(checker, ["claim %d 512" % n for n in lefts])]
-    assert r == [1, 1, 1, 1, 1, 1, 2, 3, 4, 4, 4, 4]
+    assert r == [1, 1, 1, 1, 1, 2, 3, 3, 4, 4, 4, 4]
